@@ -297,13 +297,15 @@ int hvr_set_empty_skip(hvr_ctx *ctx, int mode);
 int hvr_skip_info(hvr_ctx *ctx, unsigned long long *clear_bricks, unsigned long long *bricks, int *used);
 
 /* Cost-ordered dispatch of single frames (no counterpart in the reference).
- * A frame ends with its longest waves; in row order, long 16x16 ray blocks
+ * A frame ends with its longest waves; in row order, long ray blocks
  * that start after the first round of resident blocks set its end.  With
- * ordering, ray setup files every block under its rays' largest iteration
- * bound and the march starts the longest first.  The image and the sample
- * counts are identical in every mode.  HVR_ORDER_AUTO (the default) orders
- * frames of more blocks than the device keeps resident at once (8 per
- * compute unit) and at least 8 block rows. */
+ * ordering, a pass before the march files every block under an iteration
+ * bound of its rays and the march starts the longest first.  The image and
+ * the sample counts are identical in every mode.  HVR_ORDER_AUTO (the
+ * default) orders frames of more blocks than the device keeps resident at
+ * once (8 per compute unit) and at least 8 block rows, unless the frame is
+ * larger than 2.25 times what is resident or its rays take few steps, where
+ * row order is faster. */
 #define HVR_ORDER_OFF 0
 #define HVR_ORDER_ON 1
 #define HVR_ORDER_AUTO 2

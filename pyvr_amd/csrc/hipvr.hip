@@ -132,11 +132,10 @@ struct hvr_ctx {
     size_t pix_cap;        // pixels d_out and h_pinned hold
     size_t counts_cap;     // pixels d_counts holds
     // cost-ordered dispatch of single frames (k_order_blocks)
-    uint32_t *d_order;     // two sets of 8 x kOrderBuckets counters, then the slots
+    uint32_t *d_order;     // block of each dispatch position, then the slots
     size_t order_words;    // words d_order holds
     int order_mode;        // HVR_ORDER_OFF / _ON / _AUTO
     int order_used;        // whether the last frame was cost-ordered
-    int order_parity;      // counter set of the next ordered frame
     // LUT uploads (hvr_set_lut): pinned staging slots holding the entries and
     // their prefix counts, each reused once the copy that last read it is done
     void *h_lut_stage[4];
@@ -150,10 +149,9 @@ struct hvr_ctx {
 // the bound volume's bricks are transparent for the current LUT.
 static constexpr double kSkipAutoFraction = 0.25;
 
-// HVR_ORDER_AUTO orders a frame's blocks by cost when they are more than the
-// march keeps resident at once (8 blocks of 256 threads per compute unit):
-// only then do blocks start late.
-static constexpr int kOrderAutoBlocksPerCU = 8;
+// The rays the device marches at once with one lane each: 8 blocks of 256
+// threads per compute unit.
+static long long resident_rays(const hvr_ctx *c) { return 2048ll * c->ncu; }
 
 
 // ---------------------------------------------------------------------------
@@ -244,7 +242,7 @@ static void launch_march_generic(const MarchArgs &a)
     const size_t lds = NM == NM_ANY ? 0 : 2 * (size_t)a.lut_n * sizeof(float4);
     hipLaunchKernelGGL((k_march<SF, NM, 3, COUNT, false, false>), dim3(a.nblocks), dim3(256), lds, a.stream, a.fc,
                        a.ts, a.tn, a.lut, a.lut_n, a.out, a.counts, a.skip, a.ntx, a.nblocks,
-                       a.order_cnt, a.order_slots, a.order_cap);
+                       a.order, a.rot);
 }
 
 // The transparent-brick count of the current flags, once its copy to the
@@ -311,21 +309,50 @@ static const uint8_t *brick_flags(hvr_ctx *c, const hvr_volume *v)
     return (double)c->flags_clear >= kSkipAutoFraction * (double)c->flags_total ? c->d_flags : nullptr;
 }
 
-// The march of one frame into `out` (W*H RGBA8 on the device): the fast
-// instances of the scalar volume's format (normals from the same texels, as
-// (rho, 0, 0) of the same volume, or unbound; brick edge 8 or 16), with
-// transparent-brick skipping when the flags say so and buffer loads below
-// 4 GiB, else the generic instance.
-static void launch_march(hvr_ctx *c, const FrameConst &fc, uchar4 *out, bool count, const uint32_t *order_cnt,
-                         const uint32_t *order_slots, int order_cap)
+// Whether a volume is read through buffer loads (32-bit offsets, 24-bit brick
+// indices).
+static bool volume_buf(const hvr_volume *v)
+{
+    return v->bytes <= 0xffffffffull && (uint64_t)v->nbx * v->nby * v->nbz < (1ull << 24);
+}
+
+// How a frame is marched: the fast instances of the scalar volume's format
+// (nm >= 0: normals from the same texels, as (rho, 0, 0) of the same volume,
+// or unbound; brick edge 8 or 16), with transparent-brick skipping when the
+// flags say so and buffer loads below 4 GiB, else the generic instance.
+struct MarchPlan {
+    int nm;
+    const uint8_t *skip;
+    bool buf;
+    int lanes;
+};
+static MarchPlan march_plan(hvr_ctx *c, bool count)
+{
+    MarchPlan m = {-1, nullptr, false, 1};
+    const hvr_volume *S = c->scalar_vol, *N = c->normal_vol;
+    if (c->lut_n > kLutLdsMax || !S || c->scalar_role != HVR_ROLE_SCALAR || !(S->lb == 3 || S->lb == 4)) return m;
+    if (!N) m.nm = NM_ZERO;
+    else if (N == S && c->normal_role == HVR_ROLE_SCALAR) m.nm = NM_ALIAS;
+    else if (N == S && c->normal_role == HVR_ROLE_NORMAL && fmt_has_normal(S->fmt)) m.nm = NM_SAME;
+    if (m.nm < 0) return m;
+    m.skip = brick_flags(c, S);
+    m.buf = volume_buf(S) && !c->force_global;
+    if (m.buf && !count) m.lanes = march_lanes((long long)c->W * c->H, resident_rays(c), m.skip != nullptr);
+    return m;
+}
+
+// The march of one frame into `out` (W*H RGBA8 on the device).
+static void launch_march(hvr_ctx *c, const FrameConst &fc, uchar4 *out, bool count, const MarchPlan &m,
+                         const uint32_t *order)
 {
     MarchArgs a;
     a.fc = fc;
-    a.order_cnt = order_cnt;
-    a.order_slots = order_slots;
-    a.order_cap = order_cap;
-    a.ntx = (c->W + 15) / 16;
-    a.nblocks = a.ntx * ((c->H + 15) / 16);
+    a.lanes = m.lanes;
+    a.order = order;
+    const MarchTile bt = march_tile(m.lanes);
+    a.ntx = (c->W + (1 << bt.lbw) - 1) >> bt.lbw;
+    a.nblocks = a.ntx * ((c->H + (1 << bt.lbh) - 1) >> bt.lbh);
+    a.rot = row_rotation(a.ntx);
     const hvr_volume *S = c->scalar_vol, *N = c->normal_vol;
     a.ts = tex_desc(S, c->scalar_role, fc);
     a.tn = tex_desc(N, c->normal_role, fc);
@@ -333,43 +360,25 @@ static void launch_march(hvr_ctx *c, const FrameConst &fc, uchar4 *out, bool cou
     a.lut_n = c->lut_n;
     a.out = out;
     a.counts = c->d_counts;
-    a.skip = nullptr;
+    a.skip = m.skip;
     a.stream = c->stream;
-    const bool small_lut = c->lut_n <= kLutLdsMax;
     c->skip_used = 0;
-    if (small_lut && !S && !N) {
+    if (c->lut_n <= kLutLdsMax && !S && !N) {
         a.tn = a.ts = tex_desc(nullptr, 0, fc);
         if (count) launch_march_generic<TF_NONE, NM_ZERO, true>(a);
         else launch_march_generic<TF_NONE, NM_ZERO, false>(a);
         return;
     }
-    if (small_lut && S && c->scalar_role == HVR_ROLE_SCALAR && (S->lb == 3 || S->lb == 4)) {
-        int nm = -1;
-        if (!N) nm = NM_ZERO;
-        else if (N == S && c->normal_role == HVR_ROLE_SCALAR) nm = NM_ALIAS;
-        else if (N == S && c->normal_role == HVR_ROLE_NORMAL && fmt_has_scalar(S->fmt)) nm = NM_SAME;
-        if (nm >= 0) {
-            const uint8_t *skip = brick_flags(c, S);
-            const bool buf = a.ts.nbytes32 != 0 && !c->force_global;
-            a.skip = skip;
-            a.tn = tex_desc(nullptr, 0, fc);
-            bool done = false;
-            switch (S->fmt) {
-#define HVR_CASE(F)                                                            \
-    case F:                                                                    \
-        done = launch_march_##F(a, nm, S->lb, count, skip != nullptr, buf);    \
-        break;
-                HVR_FAST_FORMATS(HVR_CASE)
+    if (m.nm >= 0) {
+        a.tn = tex_desc(nullptr, 0, fc);
+        c->skip_used = m.skip != nullptr;
+        switch (S->fmt) {   // every format with a scalar field is a fast one
+#define HVR_CASE(F) \
+    case F: launch_march_##F(a, m.nm, S->lb, count, m.skip != nullptr, m.buf); break;
+            HVR_FAST_FORMATS(HVR_CASE)
 #undef HVR_CASE
-            default: break;
-            }
-            if (done) {
-                c->skip_used = skip != nullptr;
-                return;
-            }
-            a.skip = nullptr;
-            a.tn = tex_desc(N, c->normal_role, fc);
         }
+        return;
     }
     if (count) launch_march_generic<TF_NONE, NM_ANY, true>(a);
     else launch_march_generic<TF_NONE, NM_ANY, false>(a);
@@ -390,17 +399,23 @@ static int enqueue_frame(hvr_ctx *c, bool count, uchar4 *dst, bool count_shaded 
         e1 = (*c->tev)[k + 1];
         e2 = (*c->tev)[k + 2];
     }
+    HIPCHK(hipEventRecord(e0, c->stream));
+    const MarchPlan plan = march_plan(c, count);
+    const MarchTile bt = march_tile(plan.lanes);
+    const int ntx = (c->W + (1 << bt.lbw) - 1) >> bt.lbw, nty = (c->H + (1 << bt.lbh) - 1) >> bt.lbh;
     // cost-ordered dispatch (hvr_set_dispatch_order): the blocks of the
     // first multiple-of-8 block rows are filed by k_order_blocks and marched
     // in decreasing order of their rays' iteration bounds
-    const int ntx = (c->W + 15) / 16, nty = (c->H + 15) / 16, nblocks = ntx * nty;
     const int head_rows = nty >> 3 << 3, cap = (head_rows >> 3) * ntx;
-    const bool ordered = head_rows > 0 && (c->order_mode == HVR_ORDER_ON ||
-                                           (c->order_mode == HVR_ORDER_AUTO &&
-                                            nblocks > kOrderAutoBlocksPerCU * c->ncu));
-    constexpr int kSet = 8 * kOrderBuckets;   // counters per set
+    const double diagonal = std::sqrt((double)fc.ext[0] * fc.ext[0] + (double)fc.ext[1] * fc.ext[1] +
+                                      (double)fc.ext[2] * fc.ext[2]);
+    const bool ordered =
+        head_rows > 0 && (c->order_mode == HVR_ORDER_ON ||
+                          (c->order_mode == HVR_ORDER_AUTO &&
+                           order_auto((long long)ntx * nty, (long long)c->W * c->H, resident_rays(c), plan.lanes,
+                                      std::min((double)fc.max_steps, diagonal / (double)fc.step))));
     if (ordered) {
-        const size_t words = 2 * (size_t)kSet + (size_t)kSet * (size_t)cap;
+        const size_t words = (size_t)head_rows * ntx * (1 + kOrderBuckets);
         if (words > c->order_words) {
             HIPCHK(hipStreamSynchronize(c->stream));
             (void)hipFree(c->d_order);
@@ -408,31 +423,20 @@ static int enqueue_frame(hvr_ctx *c, bool count, uchar4 *dst, bool count_shaded 
             c->order_words = 0;
             HIPCHK(hipMalloc(&c->d_order, words * sizeof(uint32_t)));
             c->order_words = words;
-            // both counter sets start at zero (a kernel: no memset node in
-            // a graph a caller captures)
-            hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, c->stream, c->d_order, 2 * kSet, 0u);
-            HIPCHK(hipGetLastError());
-            c->order_parity = 0;
         }
     }
     c->order_used = ordered;
-    uint32_t *cnt = nullptr, *slots = nullptr;
-    HIPCHK(hipEventRecord(e0, c->stream));
     if (ordered) {
-        // this frame files into one counter set and clears the other
-        const int p = c->order_parity;
-        c->order_parity = p ^ 1;
-        cnt = c->d_order + p * kSet;
-        slots = c->d_order + 2 * kSet;
         // the blocks of the head rows only (the others keep row order)
-        hipLaunchKernelGGL(k_order_blocks, dim3(head_rows * ntx), dim3(256), 0, c->stream, fc, cnt,
-                           c->d_order + (p ^ 1) * kSet, slots, ntx, head_rows, cap);
+        hipLaunchKernelGGL(k_order_blocks, dim3(8), dim3(kOrderThreads), 0, c->stream, fc, c->d_order,
+                           c->d_order + (size_t)head_rows * ntx, ntx, head_rows, cap, bt.lbw, bt.lbh);
         HIPCHK(hipGetLastError());
     }
     // the march sets up its rays itself
     HIPCHK(hipEventRecord(e1, c->stream));
     const bool host = !dst && c->readback_mode == HVR_READBACK_DIRECT;
-    launch_march(c, fc, dst ? dst : host ? (uchar4 *)c->h_pinned_dev : c->d_out, count, cnt, slots, cap);
+    launch_march(c, fc, dst ? dst : host ? (uchar4 *)c->h_pinned_dev : c->d_out, count, plan,
+                 ordered ? c->d_order : nullptr);
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(e2, c->stream));
     c->last_ev[0] = e0;
@@ -1374,11 +1378,6 @@ static BatchLaunchFn batch_fn(int fmt, int nm, int lb, bool count, int ts, bool 
 #undef HVR_CASE
     default: return nullptr;
     }
-}
-
-static bool volume_buf(const hvr_volume *v)
-{
-    return v->bytes <= 0xffffffffull && (uint64_t)v->nbx * v->nby * v->nbz < (1ull << 24);
 }
 
 static size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }

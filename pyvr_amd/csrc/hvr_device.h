@@ -617,35 +617,38 @@ __device__ __forceinline__ RayRec ray_setup(const FrameConst &fc, int px, int py
     return r;
 }
 
-// K1 -- the dispatch order of a cost-ordered frame: one block per 16x16 ray
-// block (row-major, ntx per row) sets up its rays (ray_setup, nothing
-// stored) and files the block for the march (ordered_block) under the
-// largest iteration bound of its rays.
-// `cnt` holds 8 x kOrderBuckets counters (zero on entry), `slots` cap
-// entries per class and bucket; only the blocks of the first `head_rows`
-// block rows (a multiple of 8) are filed.  Block 0 also clears `clear`, the
-// other set of counters, which the previous ordered frame's march read and
-// the next ordered frame fills (counters alternate between frames, so no
-// separate clearing launch is needed).
-static __global__ void __launch_bounds__(256)
-k_order_blocks(const FrameConst fc, uint32_t *__restrict__ cnt, uint32_t *__restrict__ clear,
-               uint32_t *__restrict__ slots, int ntx, int head_rows, int cap)
+// K1 -- the dispatch order of a cost-ordered frame: `order`, the logical block
+// of each dispatch position of the first `head_rows` block rows (a multiple of
+// 8; 2^lbw x 2^lbh pixels each, ntx per row).  One thread block per dispatch
+// class (block row mod 8) files the class's `cap` blocks under the largest
+// iteration bound of three rays of each (two corners and the middle) in
+// kOrderBuckets lists, counted in LDS, and reads them back in order
+// (ordered_block).  Ray setup bounds it; every pixel's ray, and one atomic on
+// global memory per block, took twice as long (4096 blocks 12.6 us, 8192 22).
+static constexpr int kOrderThreads = 1024;
+static __global__ void __launch_bounds__(kOrderThreads)
+k_order_blocks(const FrameConst fc, uint32_t *order, uint32_t *slots, int ntx, int head_rows, int cap, int lbw,
+               int lbh)
 {
-    __shared__ int s_key[4];
-    const int t = blockIdx.x, tx = t % ntx, ty = t / ntx;
-    if (t == 0 && threadIdx.x < 8 * kOrderBuckets) clear[threadIdx.x] = 0u;
-    if (ty >= head_rows) return;   // the whole block
-    const int px = tx * 16 + (threadIdx.x & 15), py = ty * 16 + (threadIdx.x >> 4);
-    int key = 0;
-    if (px < fc.W && py < fc.H) key = ray_setup(fc, px, py).nlim;
-    for (int off = 32; off > 0; off >>= 1) key = max(key, __shfl_xor(key, off, 64));
-    if ((threadIdx.x & 63) == 0) s_key[threadIdx.x >> 6] = key;
+    __shared__ uint32_t s_cnt[8 * kOrderBuckets];   // of this class only
+    const int cls = blockIdx.x;
+    if (threadIdx.x < 8 * kOrderBuckets) s_cnt[threadIdx.x] = 0u;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        const int m = max(max(s_key[0], s_key[1]), max(s_key[2], s_key[3]));
-        const int q = (ty & 7) * kOrderBuckets + order_bucket(m, fc.max_steps);
-        const uint32_t s = atomicAdd(cnt + q, 1u);
-        if (s < (uint32_t)cap) slots[(uint64_t)q * (uint64_t)cap + s] = (uint32_t)t;
+    for (int k = threadIdx.x; k < cap; k += kOrderThreads) {
+        const int tx = k % ntx, ty = (k / ntx) * 8 + cls;
+        int key = 0;
+        for (int c = 0; c < 3; ++c) {
+            const int x = min((tx << lbw) + (((1 << lbw) - 1) * c >> 1), fc.W - 1),
+                      y = min((ty << lbh) + (((1 << lbh) - 1) * c >> 1), fc.H - 1);
+            key = max(key, ray_setup(fc, x, y).nlim);
+        }
+        const int q = cls * kOrderBuckets + order_bucket(key, fc.max_steps);
+        slots[(uint64_t)q * (uint64_t)cap + atomicAdd(&s_cnt[q], 1u)] = (uint32_t)(ty * ntx + tx);
+    }
+    __syncthreads();   // the slots of this class were written by this block
+    for (int k = threadIdx.x; k < cap; k += kOrderThreads) {
+        const int b = k * 8 + cls;
+        order[b] = (uint32_t)ordered_block(b, head_rows * ntx, s_cnt, slots, cap);
     }
 }
 
@@ -757,22 +760,29 @@ __device__ __forceinline__ void composite(const FrameConst &fc, const float4 &q,
     composite_diff(fc, q, NM != NM_ZERO ? lambert(fc, n0, n1, n2) : 0.f, C0, C1, C2, A);
 }
 
-// K2 -- march and composite (volume.frag.glsl:84-121), one thread per ray.
-// A 256-thread block covers 16x16 pixels; each wave64 an 8x8 tile.  Blocks
+// K2 -- march and composite (volume.frag.glsl:84-121), P adjacent lanes per
+// ray (march_lanes; one, in most large frames).  A block of 4 waves covers
+// 16x16, 16x8 or 8x8 pixels; each wave64 an 8x8, 8x4 or 4x4 tile.  Blocks
 // are dispatched round-robin over the 8 XCDs (block b on XCD (b + c) mod 8,
 // c varying from launch to launch), and each XCD runs its blocks in order.
-// The block -> tile mapping deals 16-pixel block rows to the XCDs in turn
+// The block -> tile mapping deals block rows to the XCDs in turn
 // (XCD of b & 7 takes rows b & 7, 8 + (b & 7), ...): the work per row varies
 // strongly over the image (where the rays cross dense matter), so
 // contiguous bands per XCD left some XCDs idle for half the frame, while
 // interleaved rows give every XCD an even share, and its L2 still sees whole
-// rows.  Rows past the last multiple of 8 keep the plain order.  With
-// `order` (a cost-ordered frame, k_order_blocks), each XCD's class of
-// rows is taken in decreasing order of its blocks' iteration bounds
-// instead (ordered_block), so that the long blocks start in the first round
-// of resident blocks rather than after it.  A wave runs
+// rows; within a row the start is rotated (row_rotation) to spread the
+// columns over the XCD's compute units.  Rows past the last multiple of 8
+// keep the plain order.  With `order` (a cost-ordered frame,
+// k_order_blocks), each XCD's class of rows is taken in decreasing order of
+// its blocks' iteration bounds instead, so that the long blocks start in the
+// first round of resident blocks rather than after it.  A wave runs
 // while any of its rays is live; a ray stops at its iteration bound
 // (max_steps at most), when its alpha reaches tau, or when it leaves the box.
+//
+// What bounds it: in frames of more rays than stay resident, VALU issue (about
+// 100 instructions a shaded sample) and, for 16-byte texels, the L1; in smaller
+// ones the chain of one ray's samples (about 1000 cycles each for a wave
+// alone on its SIMD, 500 of them VALU), which lanes shorten.
 //
 // In-box test (:88-92): fl((p - bmin)/ext) lies in [0, 1] exactly when
 // fl(p - bmin) lies in [0, ext] (for ext > 0 the quotient of a larger
@@ -792,13 +802,111 @@ __device__ __forceinline__ bool inbox(const FrameConst &fc, float wx, float wy, 
     return (wz >= 0.f) & (wz <= fc.ext[2]) & (wy >= 0.f) & (wy <= fc.ext[1]) & (wx >= 0.f) & (wx <= fc.ext[0]);
 }
 
+// Exchange inside groups of P adjacent lanes (P = 2 or 4) with quad_perm: the
+// value of the group's lane K, its first lane's, and whether any lane's is not 0.
+template <int P, int K>
+__device__ __forceinline__ int group_lane(int v)
+{
+    constexpr int perm = P == 4 ? K * 0x55 : (K | K << 2 | (K + 2) << 4 | (K + 2) << 6);
+    return __builtin_amdgcn_mov_dpp(v, perm, 0xf, 0xf, true);
+}
+template <int P, int K>
+__device__ __forceinline__ float group_lane(float v)
+{
+    return __int_as_float(group_lane<P, K>(__float_as_int(v)));
+}
+template <int P>
+__device__ __forceinline__ int group_first(int v)
+{
+    return group_lane<P, 0>(v);
+}
+template <int P>
+__device__ __forceinline__ bool group_any(int v)
+{
+    v |= __builtin_amdgcn_mov_dpp(v, 0xb1, 0xf, 0xf, true);             // [1, 0, 3, 2]
+    if constexpr (P == 4) v |= __builtin_amdgcn_mov_dpp(v, 0x4e, 0xf, 0xf, true);   // [2, 3, 0, 1]
+    return v != 0;
+}
+// The group's samples in order, lane 0's first: what composite_diff adds for
+// each, in every lane.  A lane without a sample (`now` false) has a, lam and q
+// zero, which changes nothing while the alphas are finite.  Terms of the
+// fused multiply-adds are read from the other lanes by the add itself.
+template <int P, int K>
+__device__ __forceinline__ void add_color(float tl, float q0, float q1, float q2, float &C0, float &C1, float &C2)
+{
+    // s_nop: a lane's q may have been written by the instruction before
+#define HVR_FMAC3(QP)                                                           \
+    asm volatile("s_nop 1\n\tv_fmac_f32_dpp %0, %3, %6 " QP " row_mask:0xf bank_mask:0xf\n\t" \
+        "v_fmac_f32_dpp %1, %4, %6 " QP " row_mask:0xf bank_mask:0xf\n\t"               \
+        "v_fmac_f32_dpp %2, %5, %6 " QP " row_mask:0xf bank_mask:0xf"                   \
+        : "+v"(C0), "+v"(C1), "+v"(C2)                                              \
+        : "v"(q0), "v"(q1), "v"(q2), "v"(tl))
+    if constexpr (P == 2 && K == 0) HVR_FMAC3("quad_perm:[0,0,2,2]");
+    else if constexpr (P == 2) HVR_FMAC3("quad_perm:[1,1,3,3]");
+    else if constexpr (K == 0) HVR_FMAC3("quad_perm:[0,0,0,0]");
+    else if constexpr (K == 1) HVR_FMAC3("quad_perm:[1,1,1,1]");
+    else if constexpr (K == 2) HVR_FMAC3("quad_perm:[2,2,2,2]");
+    else HVR_FMAC3("quad_perm:[3,3,3,3]");
+#undef HVR_FMAC3
+}
+template <int P, int K>
+__device__ __forceinline__ void group_alpha(float a, float lam, float A, float (&tl)[P], float (&al)[P])
+{
+    const float ta = (1.f - A) * group_lane<P, K>(a);
+    tl[K] = ta * group_lane<P, K>(lam);
+    al[K] = A + ta;
+    if constexpr (K + 1 < P) group_alpha<P, K + 1>(a, lam, al[K], tl, al);
+}
+template <int P, int K>
+__device__ __forceinline__ void group_color(const float (&tl)[P], float q0, float q1, float q2, float &C0, float &C1,
+                                            float &C2)
+{
+    add_color<P, K>(tl[K], q0, q1, q2, C0, C1, C2);
+    if constexpr (K + 1 < P) group_color<P, K + 1>(tl, q0, q1, q2, C0, C1, C2);
+}
+// The same with each sample taken only while alpha is below its lane's tau
+// (-infinity in a lane without a sample).
+template <int P, int K>
+__device__ __forceinline__ void group_select(float tau, float a, float lam, float q0, float q1, float q2, float &C0,
+                                             float &C1, float &C2, float &A)
+{
+    const float ta = (1.f - A) * group_lane<P, K>(a);
+    const float tl = ta * group_lane<P, K>(lam);
+    const float c0 = fmaf(tl, group_lane<P, K>(q0), C0), c1 = fmaf(tl, group_lane<P, K>(q1), C1),
+                c2 = fmaf(tl, group_lane<P, K>(q2), C2), al = A + ta;
+    const bool take = A < group_lane<P, K>(tau);
+    C0 = take ? c0 : C0;
+    C1 = take ? c1 : C1;
+    C2 = take ? c2 : C2;
+    A = take ? al : A;
+    if constexpr (K + 1 < P) group_select<P, K + 1>(tau, a, lam, q0, q1, q2, C0, C1, C2, A);
+}
+template <int P>
+__device__ __forceinline__ void composite_group(float tau, bool now, float a, float lam, float q0, float q1, float q2,
+                                                float &C0, float &C1, float &C2, float &A)
+{
+    float tl[P], al[P];
+    group_alpha<P, 0>(a, lam, A, tl, al);
+    // every ray of the wave still below tau before its last sample, with
+    // finite alphas: no sample is dropped
+    bool plain = true;
+#pragma unroll
+    for (int k = 0; k + 1 < P; ++k) plain &= fabsf(al[k]) < tau;
+    if (__ballot(!plain) == 0) {
+        group_color<P, 0>(tl, q0, q1, q2, C0, C1, C2);
+        A = al[P - 1];
+    } else {
+        group_select<P, 0>(now ? tau : -INFINITY, a, lam, q0, q1, q2, C0, C1, C2, A);
+    }
+}
+
 // The march of one ray (volume.frag.glsl:84-121) from its setup record:
 // accumulated colour (C0, C1, C2), alpha A, and the number of composited
 // samples ns (COUNT).  s_lut: the LUT with its differences in LDS (lut_sample).
 // GATE: interpolate and light the normal only for samples of non-zero
 // alpha (fewer instructions where the march is instruction-bound; the
 // result is identical either way).
-template <int SF, int NM, int LB, bool COUNT, bool SKIP, bool BUF, bool GATE = false>
+template <int SF, int NM, int LB, bool COUNT, bool SKIP, bool BUF, bool GATE = false, int P = 1>
 __device__ __forceinline__ void march_ray(const FrameConst &fc, const TexDesc &ts, const TexDesc &tn,
                                           const float4 *__restrict__ lut_g, int lut_n, const float4 *s_lut,
                                           const RayRec &r, const uint8_t *__restrict__ skip,
@@ -902,7 +1010,78 @@ __device__ __forceinline__ void march_ray(const FrameConst &fc, const TexDesc &t
         const float bqx = -(sx * fc.bmin[0]), bqy = -(sy * fc.bmin[1]), bqz = -(sz * fc.bmin[2]);
         const float lx = sx > 0.f ? fc.ext[0] : 0.f, ly = sy > 0.f ? fc.ext[1] : 0.f,
                     lz = sz > 0.f ? fc.ext[2] : 0.f;
-        if constexpr (!SKIP) {
+        if constexpr (P > 1) {
+            // P adjacent lanes march one ray: lane j holds samples j, P + j, ...
+            // of the in-box run (each position the sum of the same additions
+            // as a single lane's), every lane the ray's colour.  Lanes of a
+            // group leave the loop together.
+            static_assert(!COUNT && !GATE && (P == 2 || P == 4), "");
+            const int j = (int)threadIdx.x & (P - 1);
+            auto advance = [&](int n) {
+#pragma unroll
+                for (int k = 0; k < n; ++k) {
+                    x = __fadd_rn(x, dqx);
+                    y = __fadd_rn(y, dqy);
+                    z = __fadd_rn(z, dqz);
+                }
+            };
+            for (int k = 1; k < P; ++k)
+                if (j >= k) advance(1);
+            i += j;
+            float ax = __fadd_rn(x, bqx), ay = __fadd_rn(y, bqy), az = __fadd_rn(z, bqz);
+            bool in = i < nlim && (az <= lz) & (ay <= ly) & (ax <= lx);
+            Footprint fa = footprint_brick<LB, BUF>(ts, in ? fabsf(az) : 0.f, in ? fabsf(ay) : 0.f,
+                                                    in ? fabsf(ax) : 0.f),
+                      fb;
+            uint32_t flag = SKIP ? ld_global(skip + fa.brick) : 0u;
+            bool live = group_first<P>((int)in) != 0;
+            auto step = [&](const Footprint &f, Footprint &g) {
+                const bool now = SKIP ? in && flag == 0 : in;
+                i += P;
+                advance(P);
+                ax = __fadd_rn(x, bqx);
+                ay = __fadd_rn(y, bqy);
+                az = __fadd_rn(z, bqz);
+                in = i < nlim && (az <= lz) & (ay <= ly) & (ax <= lx);
+                g = footprint_brick<LB, BUF>(ts, fabsf(az), fabsf(ay), fabsf(ax));
+                if (SKIP && in && g.brick != f.brick) flag = ld_global(skip + g.brick);
+                if (group_any<P>((int)now)) {
+                    float a = 0.f, lam = 0.f, q0 = 0.f, q1 = 0.f, q2 = 0.f;
+                    if (now) {
+                        Footprint h = f;
+                        footprint_addr<T, LB, BUF>(ts, h);
+                        float4 q;
+                        float diff = 0.f;
+                        if constexpr (NM == NM_SAME) {
+                            uint32_t raw[4][T / 2];
+                            load_pairs<SF, LB, BUF>(src, h, raw);
+                            float w[8];
+                            fp_weights(h, w);
+                            const float rho = interp_scalar<SF>(raw, w) * u8k;
+                            const float3 n = interp_normal<SF>(raw, w);
+                            q = lut_sample(s_lut, fn1, fn, rho);
+                            diff = lambert(fc, n.x, n.y, n.z);
+                        } else {
+                            const float rho = sample1<SF, LB, BUF>(src, h) * u8k;
+                            q = lut_sample(s_lut, fn1, fn, rho);
+                            if constexpr (NM == NM_ALIAS) diff = lambert(fc, rho, 0.f, 0.f);
+                        }
+                        a = 1.f - __builtin_amdgcn_exp2f(-(q.w * fc.alpha_k));
+                        lam = fmaf(fc.kd, diff, fc.ka);
+                        q0 = q.x;
+                        q1 = q.y;
+                        q2 = q.z;
+                    }
+                    composite_group<P>(fc.tau, now, a, lam, q0, q1, q2, C0, C1, C2, A);
+                }
+                live = group_first<P>((int)in) != 0;
+            };
+            while (live && A < fc.tau) {
+                step(fa, fb);
+                if (!(live && A < fc.tau)) break;
+                step(fb, fa);
+            }
+        } else if constexpr (!SKIP) {
             // the in-box run
             for (; i < nlim; ++i) {
                 if (!(A < fc.tau)) break;
@@ -978,12 +1157,19 @@ __device__ __forceinline__ void load_lut_lds(const float4 *__restrict__ lut_g, i
     }
 }
 
-template <int SF, int NM, int LB, bool COUNT, bool SKIP, bool BUF>
+// Pixels of a block of four waves with P lanes per ray, as log2: a wave covers
+// 8x8, 8x4 or 4x4 pixels, a block 2x2 waves.
+struct MarchTile {
+    int lbw, lbh;
+};
+__host__ __device__ constexpr MarchTile march_tile(int P) { return MarchTile{P == 4 ? 3 : 4, P == 1 ? 4 : 3}; }
+
+template <int SF, int NM, int LB, bool COUNT, bool SKIP, bool BUF, int P = 1>
 __global__ void __launch_bounds__(256)
 k_march(const FrameConst fc, const TexDesc ts, const TexDesc tn, const float4 *__restrict__ lut_g,
         int lut_n, uchar4 *__restrict__ out,
         uint32_t *__restrict__ counts, const uint8_t *__restrict__ skip, int ntx, int nblocks,
-        const uint32_t *__restrict__ order_cnt, const uint32_t *__restrict__ order_slots, int order_cap)
+        const uint32_t *__restrict__ order, int rot)
 {
     extern __shared__ float4 s_lut[];
     if constexpr (NM != NM_ANY) {
@@ -993,26 +1179,26 @@ k_march(const FrameConst fc, const TexDesc ts, const TexDesc tn, const float4 *_
     const int b = blockIdx.x;
     const int head = ((nblocks / ntx) >> 3 << 3) * ntx;   // blocks of the first multiple-of-8 rows
     int logical = b;
-    if (order_cnt) {
-        // cost-ordered (k_order_blocks filed the blocks)
-        logical = ordered_block(b, head, order_cnt, order_slots, order_cap);
-        if (logical < 0 || logical >= nblocks) logical = b;
+    if (order) {
+        if (b < head) logical = (int)order[b];   // cost-ordered (k_order_blocks)
     } else if (b < head) {
         const int j = b >> 3;   // j-th block of its XCD
-        logical = ((j / ntx) * 8 + (b & 7)) * ntx + j % ntx;
+        const int row = j / ntx;
+        logical = (row * 8 + (b & 7)) * ntx + (j + row * rot) % ntx;
     }
     const int tx = logical % ntx, ty = logical / ntx;
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int px = tx * 16 + (wv & 1) * 8 + (lane & 7);
-    const int py = ty * 16 + (wv >> 1) * 8 + (lane >> 3);
+    constexpr MarchTile bt = march_tile(P);
+    const int wv = threadIdx.x >> 6, ray = (threadIdx.x & 63) / P;
+    const int px = (tx << bt.lbw) + ((wv & 1) << (bt.lbw - 1)) + (ray & ((1 << (bt.lbw - 1)) - 1));
+    const int py = (ty << bt.lbh) + ((wv >> 1) << (bt.lbh - 1)) + (ray >> (bt.lbw - 1));
     if (px >= fc.W || py >= fc.H) return;
     const int pix = py * fc.W + px;
     const RayRec r = ray_setup(fc, px, py);
 
     float C0 = 0.f, C1 = 0.f, C2 = 0.f, A = 0.f;
     uint32_t ns = 0;
-    march_ray<SF, NM, LB, COUNT, SKIP, BUF>(fc, ts, tn, lut_g, lut_n, s_lut, r, skip, C0, C1, C2, A, ns);
-    out[pix] = blend_store(fc, C0, C1, C2, A);
+    march_ray<SF, NM, LB, COUNT, SKIP, BUF, false, P>(fc, ts, tn, lut_g, lut_n, s_lut, r, skip, C0, C1, C2, A, ns);
+    if (P == 1 || threadIdx.x % P == 0) out[pix] = blend_store(fc, C0, C1, C2, A);
     if constexpr (COUNT) counts[pix] = ns;
 }
 

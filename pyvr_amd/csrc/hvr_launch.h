@@ -18,10 +18,9 @@ struct MarchArgs {
     uchar4 *out;
     uint32_t *counts;
     const uint8_t *skip;
-    int ntx, nblocks;
-    const uint32_t *order_cnt;     // cost-ordered dispatch (k_order_blocks), or nullptr
-    const uint32_t *order_slots;
-    int order_cap;
+    int lanes;                     // adjacent lanes per ray: 1, 2 or 4
+    int ntx, nblocks, rot;
+    const uint32_t *order;         // cost-ordered dispatch (k_order_blocks), or nullptr
     hipStream_t stream;
 };
 

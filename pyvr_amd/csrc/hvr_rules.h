@@ -130,6 +130,46 @@ constexpr int ordered_block(int b, int head, const U *cnt, const U *slots, int c
     return b;
 }
 
+// Lanes per ray of a single frame's march: with fewer rays than keep the device
+// busy, a frame takes as long as its longest rays, whose samples follow one
+// another; marched by 2 or 4 adjacent lanes, which take successive samples and
+// composite them in order, a ray ends in as many fewer iterations, for more
+// instructions a sample (14-18 % with 2 lanes, about 35 % with 4).  `resident`:
+// the rays the device marches at once with one lane each (524,288 on 256
+// compute units).  Measured (us, 1 / 2 / 4 lanes; cameras averaged): 64^2 of a
+// 256^3 volume 338 / 177 / 100, 362^2 of it 268 / 166 / 116, 512^2 dense
+// 192 / 146 / 154, transparent-skipping 512^2 79 / 63 / 66, 1024^2 504 / 452 /
+// 480 and 366 / 331 / 409, 1280^2 601 / 635 / 720, 2048^2 1237 / 1491 / 1780.
+// Where no brick is stepped over, rays are about equally long and the device
+// stays busy to the end: 724^2 246 / 238 and 257 / 293, 1024^2 394 / 407 and
+// 446 / 487.
+constexpr int march_lanes(long long rays, long long resident, bool skipping)
+{
+    if (8 * rays <= 3 * resident) return 4;
+    return 4 * rays <= (skipping ? 9 : 3) * resident ? 2 : 1;
+}
+
+// Dispatch order of the blocks kept in rows: consecutive blocks of a class
+// (ordered_block) go to its 32 compute units in turn, so with a multiple of 16
+// blocks per row one column of the image, which is dense or empty as a whole
+// more often than not, would stay on one or two units.  Row r of a class is
+// rotated by r times this, which puts a column 13 units further from row to
+// row (512^2, 2 lanes: 232 -> 187 us, 184 -> 149; 256^2, 4 lanes: 106 -> 98).
+// Other widths spread by themselves, and rotating them gained nothing.
+constexpr int row_rotation(int ntx) { return ntx % 16 == 0 ? ((ntx - 13) & 31) % ntx : 0; }
+
+// Whether HVR_ORDER_AUTO orders a frame by cost: with more blocks than the
+// march keeps resident (8 of 256 threads per unit) blocks start late, and up
+// to 2.25 times the resident rays that sets the frame's end; beyond, and where
+// the rays' `steps` are few, the frame loses more to marching all dense blocks
+// at once than it gains (us in row order / ordered: 1024^2, 1 lane, 346 steps
+// 394 / 364, 446 / 422; 2 lanes, 692 steps 529 / 495; 2 lanes, 100 steps
+// 159 / 178; 1536^2 767 / 771; 2048^2, 100 steps 452 / 516).
+constexpr bool order_auto(long long blocks, long long rays, long long resident, int lanes, double steps)
+{
+    return blocks * 256 > resident && 4 * rays <= 9 * resident && steps >= 256.0 * lanes;
+}
+
 // Inverse of a 4x4 matrix (row-major, m[4*r + c]) by Gauss-Jordan
 // elimination with partial pivoting.  Returns false when singular.
 constexpr bool inverse4(const double *m, double *inv)

@@ -18,13 +18,17 @@ namespace {
 constexpr int F = HVR_INST_FMT;
 
 // ---- single-frame march (K2) ----
-template <int NM, int LB, bool COUNT, bool SKIP, bool BUF>
+template <int NM, int LB, bool COUNT, bool SKIP, bool BUF, int P = 1>
 void march(const MarchArgs &a)
 {
+    if constexpr (P == 1 && !COUNT && BUF) {
+        if (a.lanes == 2) return march<NM, LB, COUNT, SKIP, BUF, 2>(a);
+        if (a.lanes == 4) return march<NM, LB, COUNT, SKIP, BUF, 4>(a);
+    }
     const size_t lds = 2 * (size_t)a.lut_n * sizeof(float4);
-    hipLaunchKernelGGL((k_march<F, NM, LB, COUNT, SKIP, BUF>), dim3(a.nblocks), dim3(256), lds, a.stream, a.fc, a.ts,
-                       a.tn, a.lut, a.lut_n, a.out, a.counts, a.skip, a.ntx, a.nblocks,
-                       a.order_cnt, a.order_slots, a.order_cap);
+    hipLaunchKernelGGL((k_march<F, NM, LB, COUNT, SKIP, BUF, P>), dim3(a.nblocks), dim3(256), lds, a.stream, a.fc,
+                       a.ts, a.tn, a.lut, a.lut_n, a.out, a.counts, a.skip, a.ntx, a.nblocks, a.order,
+                       a.rot);
 }
 
 template <int NM, int LB, bool COUNT>
