@@ -117,7 +117,8 @@ struct hvr_ctx {
     int nz_cap;            // entries d_nz holds counts for
     uint32_t lut_gen;
     uint8_t *d_flags;      // per-brick transparent flags of flags_vol
-    uint32_t *d_nclear;    // transparent-brick count written by k_brick_flags
+    uint32_t *d_nclear;    // two transparent-brick counters, which k_brick_flags fills in turn
+    int nclear_slot;       // the counter of the next k_brick_flags
     uint32_t *h_nclear;    // its copy in pinned host memory, valid once flags_ev completed
     hipEvent_t flags_ev;   // recorded after that copy
     bool flags_count_known;   // flags_clear holds the count of the current flags
@@ -279,7 +280,10 @@ static const uint8_t *brick_flags(hvr_ctx *c, const hvr_volume *v)
     };
     if (!(c->flags_vol == v && c->flags_vol_gen == v->gen && c->flags_lut_gen == c->lut_gen)) {
         c->flags_vol = nullptr;
-        if (!c->d_nclear && hipMalloc(&c->d_nclear, sizeof(uint32_t)) != hipSuccess) return none();
+        if (!c->d_nclear) {
+            if (hipMalloc(&c->d_nclear, 2 * sizeof(uint32_t)) != hipSuccess) return none();
+            hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, c->stream, c->d_nclear, 2, 0u);
+        }
         if (nb > c->flags_cap) {
             if (hipStreamSynchronize(c->stream) != hipSuccess) return none();
             (void)hipFree(c->d_flags);
@@ -289,12 +293,13 @@ static const uint8_t *brick_flags(hvr_ctx *c, const hvr_volume *v)
             c->flags_cap = nb;
         }
         // the count comes back asynchronously (no wait in the frame's path)
-        hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, c->stream, c->d_nclear, 1, 0u);
-        hipLaunchKernelGGL(k_brick_flags, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, c->stream,
-                           (const float2 *)v->d_range, (uint32_t)nb, (const int *)c->d_nz, c->lut_n, c->d_flags,
-                           c->d_nclear);
-        if (hipGetLastError() != hipSuccess ||
-            hipMemcpyAsync(c->h_nclear, c->d_nclear, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream) !=
+        uint32_t *count = c->d_nclear + c->nclear_slot;
+        hipLaunchKernelGGL(k_brick_flags, dim3(clearance_tiles(v->nbx, v->nby, v->nbz)), dim3(kClearThreads), 0,
+                           c->stream, (const float2 *)v->d_range, (int)v->nbx, (int)v->nby, (int)v->nbz,
+                           (const int *)c->d_nz, c->lut_n, c->d_flags, count, c->d_nclear + (c->nclear_slot ^ 1));
+        if (hipGetLastError() != hipSuccess) return none();
+        c->nclear_slot ^= 1;
+        if (hipMemcpyAsync(c->h_nclear, count, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream) !=
                 hipSuccess ||
             hipEventRecord(c->flags_ev, c->stream) != hipSuccess)
             return none();
@@ -1330,7 +1335,20 @@ struct BatchReq {
     hvr_params params;
     int W, H;
     std::vector<float> lut;  // n x RGBA
+    uint64_t lut_hash;       // of its bytes
 };
+
+// FNV-1a over the LUT's 32-bit words: requests with other hashes hold other LUTs.
+static uint64_t lut_hash(const std::vector<float> &lut)
+{
+    uint64_t h = 0xcbf29ce484222325ull;
+    for (float f : lut) {
+        uint32_t w;
+        memcpy(&w, &f, 4);
+        h = (h ^ w) * 0x100000001b3ull;
+    }
+    return h;
+}
 
 struct hvr_batch {
     hvr_ctx *ctx;
@@ -1536,6 +1554,7 @@ int hvr_batch_add(hvr_batch *b, hvr_volume *s, int srole, hvr_volume *n, int nro
     r.H = height;
     if (lut_n > 0) r.lut.assign(lut_rgba, lut_rgba + 4 * (size_t)lut_n);
     else r.lut = {0.f, 0.f, 0.f, 1.f};  // unbound LUT texture
+    r.lut_hash = lut_hash(r.lut);
     b->reqs.push_back(std::move(r));
     b->ran = b->counted = false;
     if (index) *index = (int)b->reqs.size() - 1;
@@ -1656,6 +1675,8 @@ int hvr_batch_run_async(hvr_batch *b, int count)
     ReqDesc *descs = (ReqDesc *)(b->h_stage + desc_off);
     size_t lut_at = lut_off, nz_at = nz_off, flag_at = 0;
     int slot = 0;
+    uint32_t flag_tiles = 0;
+    std::vector<std::pair<int, int>> firsts;   // (request, descriptor) of each volume and LUT met first
     for (size_t k = 0; k < cls.size(); ++k) {
         hdr->cls[k].desc_offset = (uint32_t)(desc_off + (size_t)slot * sizeof(ReqDesc));
         hdr->cls[k].nreq = (int)cls[k].members.size();
@@ -1667,17 +1688,34 @@ int hvr_batch_run_async(hvr_batch *b, int count)
             d.fc = frame_const_of(r.params, true, r.W, r.H);
             d.ts = tex_desc(r.vol, HVR_ROLE_SCALAR, d.fc);
             const int n = (int)(r.lut.size() / 4);
-            memcpy(b->h_stage + lut_at, r.lut.data(), r.lut.size() * sizeof(float));
-            lut_prefix_counts(r.lut.data(), n, (int *)(b->h_stage + nz_at));
-            d.lut = (const float4 *)(b->d_stage + lut_at);
-            d.nz = (const int *)(b->d_stage + nz_at);
-            lut_at += r.lut.size() * sizeof(float);
-            nz_at += (size_t)(n + 1) * sizeof(int);
+            // views of one volume through one LUT share its staged copy and flags
+            const ReqDesc *same = nullptr;
+            for (const auto &f : firsts) {
+                const BatchReq &o = b->reqs[f.first];
+                if (o.vol == r.vol && o.lut_hash == r.lut_hash && o.lut.size() == r.lut.size() &&
+                    memcmp(o.lut.data(), r.lut.data(), r.lut.size() * sizeof(float)) == 0)
+                    same = descs + f.second;
+            }
             d.lut_n = n;
             d.range = r.vol->d_range;
-            d.nbricks = r.vol->nbx * r.vol->nby * r.vol->nbz;
-            d.flags = b->d_flags + flag_at;
-            flag_at += align_up(d.nbricks, 256);
+            d.nbz = r.vol->nbz;
+            if (same) {
+                d.lut = same->lut;
+                d.nz = same->nz;
+                d.flags = same->flags;
+            } else {
+                firsts.push_back({i, slot - 1});
+                memcpy(b->h_stage + lut_at, r.lut.data(), r.lut.size() * sizeof(float));
+                lut_prefix_counts(r.lut.data(), n, (int *)(b->h_stage + nz_at));
+                d.lut = (const float4 *)(b->d_stage + lut_at);
+                d.nz = (const int *)(b->d_stage + nz_at);
+                lut_at += r.lut.size() * sizeof(float);
+                nz_at += (size_t)(n + 1) * sizeof(int);
+                d.flags = b->d_flags + flag_at;
+                flag_at += align_up((size_t)r.vol->nbx * r.vol->nby * r.vol->nbz, 256);
+                flag_tiles += clearance_tiles(r.vol->nbx, r.vol->nby, r.vol->nbz);
+            }
+            d.flag_end = flag_tiles;
             d.out = out_pool + b->out_off[i];
             d.counts = count ? b->d_counts + b->out_off[i] : nullptr;
             d.ntx = (r.W + bx - 1) / bx;
@@ -1700,7 +1738,7 @@ int hvr_batch_run_async(hvr_batch *b, int count)
         if (rc == HVR_OK) {
             // counters reset by a kernel (a graph replays kernels reliably)
             hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, b->stream, b->d_counters, kBatchMaxClasses, 0u);
-            hipLaunchKernelGGL(k_batch_flags, dim3(1024), dim3(256), 0, b->stream, (const char *)b->d_stage);
+            hipLaunchKernelGGL(k_batch_flags, dim3(512), dim3(kClearThreads), 0, b->stream, (const char *)b->d_stage);
             if (hipGetLastError() != hipSuccess) rc = HVR_EDEVICE;
         }
         for (size_t k = 0; k < cls.size() && rc == HVR_OK; ++k) {
@@ -1894,7 +1932,8 @@ int hvr_render_async_to_noalloc(hvr_ctx *c, void *dst)
     d.flags = (uint8_t *)(blk + kNoallocFlagsOffset);
     d.out = (uchar4 *)dst;
     d.counts = nullptr;
-    d.nbricks = (uint32_t)nb;
+    d.nbz = S->nbz;
+    d.flag_end = clearance_tiles(S->nbx, S->nby, S->nbz);
     d.lut_n = c->lut_n;
     d.ntx = (c->W + bx - 1) / bx;
     d.tile_end = d.ntx * ((c->H + by - 1) / by);
@@ -1902,7 +1941,7 @@ int hvr_render_async_to_noalloc(hvr_ctx *c, void *dst)
     hipEvent_t e0 = c->ev[0], e1 = c->ev[1], e2 = c->ev[2];
     HIPCHK(hipEventRecord(e0, c->stream));
     hipLaunchKernelGGL(k_stage_request, dim3(1), dim3(64), 0, c->stream, blk, off, hdr, d);
-    hipLaunchKernelGGL(k_batch_flags, dim3(1024), dim3(256), 0, c->stream, (const char *)blk);
+    hipLaunchKernelGGL(k_batch_flags, dim3(512), dim3(kClearThreads), 0, c->stream, (const char *)blk);
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(e1, c->stream));
     if (const int rc = fn(blk, 0, (uint32_t *)(blk + off.counter), (int)align_up((size_t)c->lut_n, 256), c->ncu,

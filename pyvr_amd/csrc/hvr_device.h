@@ -791,15 +791,33 @@ __device__ __forceinline__ void composite(const FrameConst &fc, const float4 &q,
 // monotonically), so the loop skips the leading outside samples (the entry
 // point may round outside) and ends at the first outside sample after them.
 //
-// Transparent bricks (SKIP instances): `skip[brick]` is set when every LUT
+// Transparent bricks (SKIP instances): `skip[brick]`, the brick's clearance
+// (hvr_rules.h), is not 0 when every LUT
 // entry that a density of the brick can weight is transparent (alpha 0 and
 // a finite colour).  Such a sample contributes exactly nothing
 // (C += (1-A)*lambda*rgb*0, A += (1-A)*0; lambda is finite because the
 // Lambert term is 0 or max(dot, 0) with fmaxf dropping a NaN), so it is
-// counted and stepped over without loading texels.
+// counted and stepped over without loading texels.  Where every ray of the
+// wave is in a brick of clearance 2 and more, the wave walks on as far as the
+// least of them allows without looking at flags or the box (the positions are
+// the same additions; a sample past the box ends the ray as before): 5
+// instructions a step instead of 26.  Letting each ray leap by itself spread
+// the rays of a wave over different depths, and the texels they then no
+// longer shared cost more than the leaps gained (512^3 batch 7.77 -> 8.2 ms;
+// the whole wave 7.77 -> 7.44).
 __device__ __forceinline__ bool inbox(const FrameConst &fc, float wx, float wy, float wz)
 {
     return (wz >= 0.f) & (wz <= fc.ext[2]) & (wy >= 0.f) & (wy <= fc.ext[1]) & (wx >= 0.f) & (wx <= fc.ext[0]);
+}
+
+// 1 / the texels a ray may move per step along any axis (leap_rate), rays
+// walking texture x, y, z along world z, y, x.
+__device__ __forceinline__ float leap_inverse(const FrameConst &fc, const TexDesc &t, const RayRec &r)
+{
+    const float x = leap_rate(r.dsx, t.k2, fmaxf(fabsf(fc.bmin[0]), fabsf(fc.bmax[0]))),
+                y = leap_rate(r.dsy, t.k1, fmaxf(fabsf(fc.bmin[1]), fabsf(fc.bmax[1]))),
+                z = leap_rate(r.dsz, t.k0, fmaxf(fabsf(fc.bmin[2]), fabsf(fc.bmax[2])));
+    return 1.f / fmaxf(fmaxf(x, y), z);
 }
 
 // Exchange inside groups of P adjacent lanes (P = 2 or 4) with quad_perm: the
@@ -1035,7 +1053,18 @@ __device__ __forceinline__ void march_ray(const FrameConst &fc, const TexDesc &t
                       fb;
             uint32_t flag = SKIP ? ld_global(skip + fa.brick) : 0u;
             bool live = group_first<P>((int)in) != 0;
+            const float inv = SKIP ? leap_inverse(fc, ts, r) : 0.f;
             auto step = [&](const Footprint &f, Footprint &g) {
+                if constexpr (SKIP) {
+                    if (__ballot(in && flag < 2) == 0) {
+                        int n = in ? leap_steps((int)flag, LB, inv) : 1 << 20;   // the group's first lane is in
+                        while (__ballot(n < 4) == 0) {
+                            advance(4);
+                            i += 4;
+                            n -= 4;
+                        }
+                    }
+                }
                 const bool now = SKIP ? in && flag == 0 : in;
                 i += P;
                 advance(P);
@@ -1115,8 +1144,24 @@ __device__ __forceinline__ void march_ray(const FrameConst &fc, const TexDesc &t
                       fb;
             uint32_t flag = ld_global(skip + fa.brick);
             bool clear = in && flag != 0;
+            const float inv = leap_inverse(fc, ts, r);
             // one sample: f the current sample's footprint, g receives the next one's
             auto step = [&](const Footprint &f, Footprint &g) {
+                if constexpr (!COUNT) {
+                    if (__ballot(!(clear && flag > 1)) == 0) {
+                        int n = leap_steps((int)flag, LB, inv);
+                        while (__ballot(n < 4) == 0) {
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) {
+                                x = __fadd_rn(x, dqx);
+                                y = __fadd_rn(y, dqy);
+                                z = __fadd_rn(z, dqz);
+                            }
+                            i += 4;
+                            n -= 4;
+                        }
+                    }
+                }
                 ++i;
                 x = __fadd_rn(x, dqx);
                 y = __fadd_rn(y, dqy);
@@ -1239,25 +1284,94 @@ k_brick_range(const char *__restrict__ texels, uint32_t brick_bytes, uint32_t nb
 // over densities in [lo, hi] are floor(u(lo)) .. ceil(u(hi)); the range is
 // widened by a margin for the rounding of the interpolated density.  `nz`
 // is the prefix count (N + 1 values) of entries that are not exactly
-// transparent (alpha != 0, or a non-finite colour).  `n_clear` counts the
-// transparent bricks (one atomic per wave).
+// transparent (alpha != 0, or a non-finite colour).
 __device__ __forceinline__ bool brick_clear(float2 r, const int *__restrict__ nz, int n)
 {
     return brick_clear_range(r.x, r.y, nz, n);
 }
 
-static __global__ void __launch_bounds__(256)
-k_brick_flags(const float2 *__restrict__ range, uint32_t nbricks, const int *__restrict__ nz, int n,
-              uint8_t *__restrict__ flags, uint32_t *__restrict__ n_clear)
+// The clearance (hvr_rules.h) of a tile of 8x8x8 bricks, by one block of 1024
+// threads.  Whether each brick of the tile and of the kMaxClearance - 1 = 4
+// bricks around it is transparent (brick_clear) makes 16x16 rows of 16 bits;
+// then one thread per row: the bricks whose every neighbour within r is in
+// the set are e & e << 1 & e >> 1 of those for r - 1, and the same with the
+// neighbour rows in y and z through LDS.  Bits past the ends of the rows read
+// as not transparent, which reaches no brick of the tile in four steps.  The
+// reads of the ranges and of the LUT's prefix counts bound it (each brick's
+// range is read for 8 tiles, from L2), so a block has 16 waves to keep them in
+// flight: 7.6 us for the 35937 bricks of a 256^3 volume, where one thread per
+// brick, without clearances, took 9.3.  s: 512 words of LDS.  Returns the transparent bricks of the tile this
+// thread's row holds.
+static constexpr int kClearTile = 8, kClearThreads = 1024;
+__device__ __forceinline__ int clearance_tile(const float2 *__restrict__ range, const int *__restrict__ nz, int n,
+                                              int nbx, int nby, int nbz, int tile, uint8_t *__restrict__ flags,
+                                              uint32_t *s)
 {
-    const uint32_t brick = blockIdx.x * 256 + threadIdx.x;
-    bool clear = false;
-    if (brick < nbricks) {
-        clear = brick_clear(range[brick], nz, n);
-        flags[brick] = clear ? 1 : 0;
+    constexpr int H = kMaxClearance - 1, N = kClearTile + 2 * H;
+    static_assert(N == 16, "16 rows of 16 bits per plane");
+    const int ntx = (nbx + kClearTile - 1) / kClearTile, nty = (nby + kClearTile - 1) / kClearTile;
+    const int x0 = tile % ntx * kClearTile - H, y0 = tile / ntx % nty * kClearTile - H,
+              z0 = tile / ntx / nty * kClearTile - H;
+    const int t = threadIdx.x, lane = t & 63;
+#pragma unroll
+    for (int row = t >> 4; row < N * N; row += kClearThreads / 16) {
+        const int x = x0 + (t & 15), y = y0 + (row & 15), z = z0 + (row >> 4);
+        bool clear = true;   // past the volume
+        if (x >= 0 && x < nbx && y >= 0 && y < nby && z >= 0 && z < nbz)
+            clear = brick_clear(ld_global(range + ((uint64_t)z * nby + y) * nbx + x), nz, n);
+        const uint64_t m = __ballot(clear);
+        if ((lane & 15) == 0) s[row] = (uint32_t)(m >> lane) & 0xffffu;
     }
-    const uint64_t m = __ballot(clear);
-    if ((threadIdx.x & 63) == 0 && m) atomicAdd(n_clear, (uint32_t)__popcll(m));
+    __syncthreads();
+    const bool own = t < N * N;
+    const int ry = t & 15, rz = t >> 4;
+    uint32_t e = own ? s[t] : 0u, cnt = 0u;   // cnt: a nibble for each brick of the tile in this row
+    const uint32_t first = e >> H & 0xffu;
+    for (int r = 0;; ++r) {
+        uint32_t b = e >> H & 0xffu;   // its bits to the low bits of the nibbles
+        b = (b | b << 12) & 0x000f000fu;
+        b = (b | b << 6) & 0x03030303u;
+        b = (b | b << 3) & 0x11111111u;
+        cnt += b;
+        if (r == H) break;
+        e = e & e << 1 & e >> 1;
+        if (own) s[256 + t] = e;
+        __syncthreads();
+        if (own) {
+            e &= (ry > 0 ? s[256 + t - 1] : 0u) & (ry < 15 ? s[256 + t + 1] : 0u);
+            s[t] = e;
+        }
+        __syncthreads();
+        if (own) e &= (rz > 0 ? s[t - 16] : 0u) & (rz < 15 ? s[t + 16] : 0u);
+    }
+    int clear = 0;
+    const int y = y0 + ry, z = z0 + rz;
+    if (own && ry >= H && ry < H + kClearTile && rz >= H && rz < H + kClearTile && y < nby && z < nbz) {
+        uint8_t *f = flags + ((uint64_t)z * nby + y) * nbx + (x0 + H);
+        const int w = min(kClearTile, nbx - (x0 + H));
+        for (int k = 0; k < w; ++k) st_global(f + k, (uint8_t)(cnt >> 4 * k & 15u));
+        clear = __popc(first & ((1u << w) - 1u));
+    }
+    __syncthreads();   // s may be filled again
+    return clear;
+}
+__host__ __device__ constexpr uint32_t clearance_tiles(uint32_t nbx, uint32_t nby, uint32_t nbz)
+{
+    return ((nbx + kClearTile - 1) / kClearTile) * ((nby + kClearTile - 1) / kClearTile) *
+           ((nbz + kClearTile - 1) / kClearTile);
+}
+
+// `n_clear` counts the transparent bricks; block 0 clears `next`, the counter
+// of the next launch.
+static __global__ void __launch_bounds__(kClearThreads)
+k_brick_flags(const float2 *__restrict__ range, int nbx, int nby, int nbz, const int *__restrict__ nz, int n,
+              uint8_t *__restrict__ flags, uint32_t *__restrict__ n_clear, uint32_t *__restrict__ next)
+{
+    __shared__ uint32_t s[512];
+    if (blockIdx.x == 0 && threadIdx.x == 0) *next = 0u;
+    int c = clearance_tile(range, nz, n, nbx, nby, nbz, blockIdx.x, flags, s);
+    for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, 64);
+    if ((threadIdx.x & 63) == 0 && c) atomicAdd(n_clear, (uint32_t)c);
 }
 
 // K3 -- upload: convert a slab of host float32 data (numpy C order = GL
@@ -1475,7 +1589,8 @@ struct ReqDesc {
     uint8_t *flags;                // per-brick transparent flags for this LUT
     uchar4 *out;                   // W*H RGBA8, bottom row first
     uint32_t *counts;              // W*H composited-sample counts (counting runs)
-    uint32_t nbricks;
+    uint32_t nbz;                  // bricks along z
+    uint32_t flag_end;             // one past this request's last tile of k_batch_flags
     int lut_n;
     int ntx;                       // tiles along x
     int tile_end;                  // one past this request's last tile in its class
@@ -1588,16 +1703,26 @@ k_batch(const char *__restrict__ block, int cls, uint32_t *__restrict__ counter)
     }
 }
 
-// Transparent-brick flags of every request of a batch for its own LUT.
-static __global__ void __launch_bounds__(256) k_batch_flags(const char *__restrict__ block)
+// Clearances of every request of a batch for its own LUT: tiles are
+// numbered through the requests (requests that share volume and LUT share
+// one set of flags, and all but the first have no tiles).
+static __global__ void __launch_bounds__(kClearThreads) k_batch_flags(const char *__restrict__ block)
 {
+    __shared__ uint32_t s[512];
     const BatchHeader *hdr = (const BatchHeader *)block;
     const ReqDesc *__restrict__ reqs = (const ReqDesc *)(block + hdr->all_offset);
-    const uint32_t stride = gridDim.x * 256u;
-    for (int q = 0; q < hdr->nreq; ++q) {
-        const ReqDesc &R = reqs[q];
-        for (uint32_t b = blockIdx.x * 256u + threadIdx.x; b < R.nbricks; b += stride)
-            st_global(R.flags + b, (uint8_t)(brick_clear(ld_global(R.range + b), R.nz, R.lut_n) ? 1 : 0));
+    const int nreq = hdr->nreq;
+    const uint32_t total = reqs[nreq - 1].flag_end;
+    for (uint32_t t = blockIdx.x; t < total; t += gridDim.x) {
+        int lo = 0, hi = nreq - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if (reqs[mid].flag_end > t) hi = mid;
+            else lo = mid + 1;
+        }
+        const ReqDesc &R = reqs[lo];
+        clearance_tile(R.range, R.nz, R.lut_n, (int)R.ts.nbx, (int)R.ts.nby, (int)R.nbz,
+                       (int)(t - (lo ? reqs[lo - 1].flag_end : 0u)), R.flags, s);
     }
 }
 

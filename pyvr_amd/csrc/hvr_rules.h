@@ -70,6 +70,27 @@ constexpr bool brick_clear_range(float lo, float hi, const int *nz, int n)
     return nz[i1 + 1] - nz[i0] == 0;
 }
 
+// Clearance of a brick: 0 when it is not transparent for the LUT, else
+// r + 1 for the largest r <= kMaxClearance - 1 such that every brick within r
+// bricks of it along every axis is transparent (bricks outside the volume
+// count as transparent: a ray that gets there has left the box).
+//
+// From a sample in a brick of clearance d, a ray stays among transparent
+// bricks for as many further steps as it needs to move (d - 1) bricks of B
+// texels along any axis.  `leap_rate` bounds its motion per step along one
+// axis, in texels: the step ds times the texels per unit k, plus the rounding
+// of the position (at most half an ulp of the larger bound in magnitude, `m`,
+// taken doubled).  With `inv` = 1 / the largest rate of the three axes,
+// leap_steps is floor(((d - 1) B - 1) inv), the 1 covering the rounding of the
+// texel coordinates at both ends (below 2^-21 of at most 2^20 texels).
+constexpr int kMaxClearance = 5;
+constexpr float leap_rate(float ds, float k, float m) { return ((ds < 0.f ? -ds : ds) + m * 0x1p-23f) * k * 1.000001f; }
+constexpr int leap_steps(int d, int lb, float inv)
+{
+    const float n = (float)(((d - 1) << lb) - 1) * inv;
+    return n > 0.f ? (n < 65536.f ? (int)n : 65536) : 0;   // 0 for a NaN
+}
+
 // Prefix counts (n + 1 values) of LUT entries that are not exactly
 // transparent.  The march reads entry i as v[i] + a*(v[i+1] - v[i]) with a
 // in [0, 1), so entry i yields alpha 0 and a finite colour for every a (the
