@@ -80,7 +80,7 @@ struct hvr_volume {
     uint32_t brick_bytes;  // (2^lb + 1)^3 texels
     uint64_t bytes;
     void *d_texels;
-    bool scalar_loaded, normals_loaded;
+    bool scalar_loaded, normals_loaded, cleared;
     float2 *d_range;       // per-brick scalar range (after a scalar upload)
     uint32_t gen;          // bumped on every upload
 };
@@ -458,43 +458,108 @@ static void noalloc_setup(int device);
 
 // ---------------------------------------------------------------------------
 // C ABI
-template <int F, int LB>
-static void launch_range(hvr_volume *v, uint32_t nb)
+// Build brick layers [bz0, bz1) of volume v (k_build) from the source in `a`.
+template <int F>
+static void launch_build(const hvr_volume *v, const BuildArgs &a, unsigned blocks)
 {
-    hipLaunchKernelGGL((k_brick_range<F, LB>), dim3((nb + 3) / 4), dim3(256), 0, v->ctx->stream,
-                       (const char *)v->d_texels, v->brick_bytes, nb, v->d_range);
+    const hipStream_t st = v->ctx->stream;
+    // voxel offsets of 32 bits where the field's floats fit 4 GiB
+    const auto go = [&](auto index) {
+        using I = decltype(index);
+        if (v->lb == 2) hipLaunchKernelGGL((k_build<F, 2, I>), dim3(blocks), dim3(256), 0, st, a);
+        else if (v->lb == 3) hipLaunchKernelGGL((k_build<F, 3, I>), dim3(blocks), dim3(256), 0, st, a);
+        else hipLaunchKernelGGL((k_build<F, 4, I>), dim3(blocks), dim3(256), 0, st, a);
+    };
+    if ((uint64_t)v->s0 * v->s1 * v->s2 < (1ull << 30)) go(uint32_t(0));
+    else go(uint64_t(0));
 }
-
-// Per-brick scalar range of a volume (for transparent-brick skipping).
-static int compute_range(hvr_volume *v)
+static int build_layers(const hvr_volume *v, BuildArgs a, uint32_t bz0, uint32_t bz1)
 {
-    hvr_ctx *c = v->ctx;
-    const uint64_t nb = (uint64_t)v->nbx * v->nby * v->nbz;
-    if (!v->d_range) HIPCHK(hipMalloc(&v->d_range, nb * sizeof(float2)));
-#define HVR_RG(F)                                                 \
-    case F:                                                       \
-        if (v->lb == 2) launch_range<F, 2>(v, (uint32_t)nb);      \
-        else if (v->lb == 3) launch_range<F, 3>(v, (uint32_t)nb); \
-        else launch_range<F, 4>(v, (uint32_t)nb);                 \
-        break;
+    a.dst = (char *)v->d_texels;
+    a.s0 = v->s0;
+    a.s1 = v->s1;
+    a.s2 = v->s2;
+    a.nbx = v->nbx;
+    a.nby = v->nby;
+    a.inv_n12 = 1.0 / ((double)v->s1 * v->s2);
+    a.inv_s2 = 1.0 / v->s2;
+    a.bz0 = bz0;
+    a.runs = (uint64_t)((v->nbx + build_bricks(v->lb) - 1) / build_bricks(v->lb)) * v->nby * (bz1 - bz0);
+    const unsigned blocks = (unsigned)std::min<uint64_t>(a.runs, (1u << 24) - 1);   // below 2^32 threads
     switch (v->fmt) {
-        HVR_RG(TF_S_F32)
-        HVR_RG(TF_S_F16)
-        HVR_RG(TF_S_U8)
-        HVR_RG(TF_C_F32_F32)
-        HVR_RG(TF_C_F16_F32)
-        HVR_RG(TF_C_U8_F32)
-        HVR_RG(TF_C_F32_SN8)
-        HVR_RG(TF_C_F16_SN8)
-        HVR_RG(TF_C_U8_SN8)
-        HVR_RG(TF_C_F16_F16)
-    default: return HVR_OK;
+#define HVR_BUILD(F) \
+    case F: launch_build<F>(v, a, blocks); break;
+        HVR_BUILD(TF_S_F32)
+        HVR_BUILD(TF_S_F16)
+        HVR_BUILD(TF_S_U8)
+        HVR_BUILD(TF_N_F32)
+        HVR_BUILD(TF_N_SN8)
+        HVR_BUILD(TF_C_F32_F32)
+        HVR_BUILD(TF_C_F16_F32)
+        HVR_BUILD(TF_C_U8_F32)
+        HVR_BUILD(TF_C_F32_SN8)
+        HVR_BUILD(TF_C_F16_SN8)
+        HVR_BUILD(TF_C_U8_SN8)
+        HVR_BUILD(TF_C_F16_F16)
+        HVR_BUILD(TF_N_F16)
+#undef HVR_BUILD
+    default: return fail(HVR_EINVAL, "bad texel format");
     }
-#undef HVR_RG
     HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(c->stream));
     return HVR_OK;
 }
+
+// The density ranges' buffer, before the scalar is written.
+static int need_range(hvr_volume *v)
+{
+    if (!v->d_range) HIPCHK(hipMalloc(&v->d_range, (size_t)v->nbx * v->nby * v->nbz * sizeof(float2)));
+    return HVR_OK;
+}
+
+static size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
+
+// The context's staging buffer, of at least `need` bytes.
+static int need_stage(hvr_ctx *c, size_t need)
+{
+    if (c->stage_bytes >= need) return HVR_OK;
+    HIPCHK(hipStreamSynchronize(c->stream));
+    (void)hipFree(c->d_stage);
+    c->d_stage = nullptr;
+    c->stage_bytes = 0;
+    HIPCHK(hipMalloc(&c->d_stage, need));
+    c->stage_bytes = need;
+    return HVR_OK;
+}
+static constexpr size_t kMaxStage = (size_t)256 << 20;   // what stays allocated, but for larger single planes
+
+// Device memory for a whole field while a volume is built from it: the staging
+// buffer up to kMaxStage, else an allocation given back (after the stream's
+// work) at the end of the scope.
+struct FieldBuffer {
+    hvr_ctx *c;
+    char *p = nullptr;
+    bool own = false;
+    explicit FieldBuffer(hvr_ctx *ctx) : c(ctx) {}
+    FieldBuffer(const FieldBuffer &) = delete;
+    int get(size_t bytes)
+    {
+        if (bytes <= kMaxStage) {
+            if (const int rc = need_stage(c, bytes)) return rc;
+            p = (char *)c->d_stage;
+            return HVR_OK;
+        }
+        HIPCHK(hipMalloc(&p, bytes));
+        own = true;
+        return HVR_OK;
+    }
+    ~FieldBuffer()
+    {
+        // also after a failure: nothing queued may still read the buffer
+        // (or, in the caller's frame, the host memory copied from)
+        (void)hipStreamSynchronize(c->stream);
+        if (own) (void)hipFree(p);
+    }
+};
 
 extern "C" {
 
@@ -762,10 +827,7 @@ int hvr_volume_create(hvr_ctx *c, int s0, int s1, int s2, int sf, int nf, hvr_vo
     const size_t bytes = (size_t)v->bytes;
     hipError_t e = hipSetDevice(c->device);
     if (e == hipSuccess) e = hipMalloc(&v->d_texels, bytes);
-    if (e == hipSuccess) e = hipMemsetAsync(v->d_texels, 0, bytes, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) {
-        (void)hipFree(v->d_texels);
         delete v;
         return fail_hip(e, "hvr_volume_create");
     }
@@ -773,58 +835,37 @@ int hvr_volume_create(hvr_ctx *c, int s0, int s1, int s2, int sf, int nf, hvr_vo
     return HVR_OK;
 }
 
+// The scalar (part 1) or normal (part 2) field of volume v from host data, in
+// groups of brick layers whose source planes (with the one plane of the
+// neighbours on both sides) fit the staging buffer of up to 256 MiB.
 static int upload_part(hvr_volume *v, const float *data, int part)
 {
     hvr_ctx *c = v->ctx;
     HIPCHK(hipSetDevice(c->device));
     const int comps = part == 1 ? 1 : 3;
+    const int B = 1 << v->lb;
     const uint64_t plane = (uint64_t)v->s0 * v->s1;
-    // stage whole z-planes, up to 256 MiB per chunk
-    const size_t max_stage = (size_t)256 << 20;
-    uint64_t zper = max_stage / (plane * comps * sizeof(float));
-    if (zper < 1) zper = 1;
-    if (zper > (uint64_t)v->s2) zper = v->s2;
-    const size_t need = (size_t)(zper * plane * comps * sizeof(float));
-    if (c->stage_bytes < need) {
-        HIPCHK(hipStreamSynchronize(c->stream));
-        (void)hipFree(c->d_stage);
-        c->d_stage = nullptr;
-        c->stage_bytes = 0;
-        HIPCHK(hipMalloc(&c->d_stage, need));
-        c->stage_bytes = need;
-    }
-    for (uint64_t z0 = 0; z0 < (uint64_t)v->s2; z0 += zper) {
-        const uint64_t nz = (z0 + zper <= (uint64_t)v->s2) ? zper : v->s2 - z0;
-        const uint64_t nvox = nz * plane;
-        HIPCHK(hipMemcpyAsync(c->d_stage, data + z0 * plane * comps, nvox * comps * sizeof(float),
-                              hipMemcpyHostToDevice, c->stream));
-        const unsigned nblk = (unsigned)((nvox + 255) / 256);
-#define HVR_UP(F)                                                                                      \
-    case F:                                                                                            \
-        hipLaunchKernelGGL(k_upload<F>, dim3(nblk), dim3(256), 0, c->stream, (char *)v->d_texels, v->s0, \
-                           v->s1, v->s2, v->lb, v->nbx, v->nby, v->nbz, v->brick_bytes,                     \
-                           (const float *)c->d_stage,                                                   \
-                           part, (int)z0, nvox);                                                        \
-        break;
-        switch (v->fmt) {
-            HVR_UP(TF_S_F32)
-            HVR_UP(TF_S_F16)
-            HVR_UP(TF_S_U8)
-            HVR_UP(TF_N_F32)
-            HVR_UP(TF_N_SN8)
-            HVR_UP(TF_C_F32_F32)
-            HVR_UP(TF_C_F16_F32)
-            HVR_UP(TF_C_U8_F32)
-            HVR_UP(TF_C_F32_SN8)
-            HVR_UP(TF_C_F16_SN8)
-            HVR_UP(TF_C_U8_SN8)
-            HVR_UP(TF_C_F16_F16)
-            HVR_UP(TF_N_F16)
-        default: return fail(HVR_EINVAL, "bad texel format");
-        }
-#undef HVR_UP
-        HIPCHK(hipGetLastError());
-        // the staging buffer is reused by the next chunk
+    const size_t row = (size_t)(plane * comps * sizeof(float));
+    const uint64_t fit = kMaxStage / row;   // planes
+    const uint32_t group = fit > (uint64_t)B + 2 ? (uint32_t)((fit - 2) / B) : 1;   // layers
+    if (const int rc = need_stage(c, (size_t)std::min<uint64_t>((uint64_t)group * B + 2, (uint64_t)v->s2) * row)) return rc;
+    if (part == 1)
+        if (const int rc = need_range(v)) return rc;
+    BuildArgs a;
+    memset(&a, 0, sizeof(a));
+    (part == 1 ? a.scalar : a.normal) = c->d_stage;
+    a.keep = part == 1 ? v->normals_loaded : v->scalar_loaded;
+    a.range = part == 1 ? v->d_range : nullptr;
+    for (uint32_t bz = 0; bz < v->nbz; bz += group) {
+        // voxel planes of layers [bz, end): texel Z holds voxel Z - 1
+        const uint32_t end = std::min(v->nbz, bz + group);
+        const int64_t z0 = std::min<int64_t>(std::max<int64_t>((int64_t)bz * B - 1, 0), v->s2 - 1),
+                      z1 = std::min<int64_t>((int64_t)end * B, v->s2);   // one past the last
+        a.first = (uint64_t)z0 * plane;
+        HIPCHK(hipMemcpyAsync(c->d_stage, data + a.first * comps, (size_t)(z1 - z0) * row, hipMemcpyHostToDevice,
+                              c->stream));
+        if (const int rc = build_layers(v, a, bz, end)) return rc;
+        // the staging buffer is reused by the next group
         HIPCHK(hipStreamSynchronize(c->stream));
     }
     return HVR_OK;
@@ -835,38 +876,20 @@ static int upload_part(hvr_volume *v, const float *data, int part)
 static int volume_from_field(hvr_volume *v, const float *d_field, bool normals)
 {
     hvr_ctx *c = v->ctx;
-    const uint64_t nvox = (uint64_t)v->s0 * v->s1 * v->s2;
-    const unsigned nblk = (unsigned)((nvox + 255) / 256);
-#define HVR_UPF(F)                                                                                           \
-    case F:                                                                                                  \
-        if (fmt_has_scalar(F))                                                                               \
-            hipLaunchKernelGGL(k_upload<F>, dim3(nblk), dim3(256), 0, c->stream, (char *)v->d_texels, v->s0,   \
-                               v->s1, v->s2, v->lb, v->nbx, v->nby, v->nbz, v->brick_bytes, d_field, 1, 0, nvox); \
-        if (normals && fmt_has_normal(F))                                                                    \
-            hipLaunchKernelGGL(k_normals_from_field<F>, dim3(nblk), dim3(256), 0, c->stream,                 \
-                               (char *)v->d_texels, v->s0, v->s1, v->s2, v->lb, v->nbx, v->nby, v->nbz,      \
-                               v->brick_bytes, d_field, nvox);                                               \
-        break;
-    switch (v->fmt) {
-        HVR_UPF(TF_S_F32)
-        HVR_UPF(TF_S_F16)
-        HVR_UPF(TF_S_U8)
-        HVR_UPF(TF_C_F32_F32)
-        HVR_UPF(TF_C_F16_F32)
-        HVR_UPF(TF_C_U8_F32)
-        HVR_UPF(TF_C_F32_SN8)
-        HVR_UPF(TF_C_F16_SN8)
-        HVR_UPF(TF_C_U8_SN8)
-        HVR_UPF(TF_C_F16_F16)
-    default: return fail(HVR_EINVAL, "the volume has no scalar field");
-    }
-#undef HVR_UPF
-    HIPCHK(hipGetLastError());
+    if (!fmt_has_scalar(v->fmt)) return fail(HVR_EINVAL, "the volume has no scalar field");
+    if (const int rc = need_range(v)) return rc;
+    BuildArgs a;
+    memset(&a, 0, sizeof(a));
+    normals = normals && fmt_has_normal(v->fmt);
+    (normals ? a.field : a.scalar) = d_field;
+    a.keep = !normals && v->normals_loaded;
+    a.range = v->d_range;
+    if (const int rc = build_layers(v, a, 0, v->nbz)) return rc;
     HIPCHK(hipStreamSynchronize(c->stream));
     v->scalar_loaded = true;
-    if (normals && fmt_has_normal(v->fmt)) v->normals_loaded = true;
+    if (normals) v->normals_loaded = true;
     ++v->gen;
-    return compute_range(v);
+    return HVR_OK;
 }
 
 int hvr_volume_upload_scalar_normals(hvr_volume *v, const float *data)
@@ -880,15 +903,11 @@ int hvr_volume_upload_scalar_normals(hvr_volume *v, const float *data)
     hvr_ctx *c = v->ctx;
     HIPCHK(hipSetDevice(c->device));
     const size_t bytes = (size_t)v->s0 * v->s1 * v->s2 * sizeof(float);
-    float *d_field = nullptr;
-    HIPCHK(hipMalloc(&d_field, bytes));
-    int rc = HVR_OK;
-    if (hipMemcpy(d_field, data, bytes, hipMemcpyHostToDevice) != hipSuccess)
-        rc = fail(HVR_EDEVICE, "copying the scalar field to the device failed");
-    if (rc == HVR_OK) rc = volume_from_field(v, d_field, true);
-    (void)hipStreamSynchronize(c->stream);   // also after a failure: nothing queued may still read the field
-    (void)hipFree(d_field);
-    return rc;
+    FieldBuffer f(c);
+    if (const int rc = f.get(bytes)) return rc;
+    if (hipMemcpyAsync(f.p, data, bytes, hipMemcpyHostToDevice, c->stream) != hipSuccess)
+        return fail(HVR_EDEVICE, "copying the scalar field to the device failed");
+    return volume_from_field(v, (const float *)f.p, true);
 }
 
 int hvr_volume_generate_blobs(hvr_volume *v, int n_blobs, const double *centers, const double *sigmas,
@@ -913,24 +932,24 @@ int hvr_volume_generate_blobs(hvr_volume *v, int n_blobs, const double *centers,
     }
     spec.noise = noise;
     spec.seed = seed;
-    const uint64_t nvox = (uint64_t)v->s0 * v->s1 * v->s2;
-    float *d_field = nullptr;
-    BlobSpec *d_spec = nullptr;
-    HIPCHK(hipMalloc(&d_field, nvox * sizeof(float)));
-    int rc = HVR_OK;
-    if (hipMalloc(&d_spec, sizeof(spec)) != hipSuccess ||
-        hipMemcpy(d_spec, &spec, sizeof(spec), hipMemcpyHostToDevice) != hipSuccess)
-        rc = fail(HVR_EDEVICE, "staging the blob parameters failed");
-    if (rc == HVR_OK) {
-        hipLaunchKernelGGL(k_blob_field, dim3((unsigned)((nvox + 255) / 256)), dim3(256), 0, c->stream, d_field,
-                           v->s0, v->s1, v->s2, (const BlobSpec *)d_spec, nvox);
-        if (hipGetLastError() != hipSuccess) rc = fail(HVR_EDEVICE, "blob field kernel launch failed");
-    }
-    if (rc == HVR_OK) rc = volume_from_field(v, d_field, normals);
-    (void)hipStreamSynchronize(c->stream);
-    (void)hipFree(d_spec);
-    (void)hipFree(d_field);
-    return rc;
+    const uint64_t nvox = (uint64_t)v->s0 * v->s1 * v->s2, len = (uint64_t)v->s0 + v->s1 + v->s2;
+    // the parameters, the factors, then the field
+    const size_t fac_at = align_up(sizeof(spec), 256), field_at = fac_at + align_up(len * n_blobs * sizeof(double), 256);
+    FieldBuffer f(c);
+    if (const int rc = f.get(field_at + nvox * sizeof(float))) return rc;
+    const BlobSpec *d_spec = (const BlobSpec *)f.p;
+    double *fac = (double *)(f.p + fac_at);
+    float *field = (float *)(f.p + field_at);
+    if (hipMemcpyAsync(f.p, &spec, sizeof(spec), hipMemcpyHostToDevice, c->stream) != hipSuccess)
+        return fail(HVR_EDEVICE, "staging the blob parameters failed");
+    if (n_blobs)
+        hipLaunchKernelGGL(k_blob_factors, dim3((unsigned)std::min<uint64_t>((len * n_blobs + 255) / 256, 1u << 20)),
+                           dim3(256), 0, c->stream, fac, v->s0, v->s1, v->s2, d_spec);
+    const uint64_t waves = (((uint64_t)v->s2 + 63) / 64) * (((uint64_t)v->s1 + kBlobRows - 1) / kBlobRows) * v->s0;
+    hipLaunchKernelGGL(k_blob_field, dim3((unsigned)std::min<uint64_t>((waves + 3) / 4, (1u << 24) - 1)), dim3(256), 0,
+                       c->stream, field, v->s0, v->s1, v->s2, d_spec, (const double *)fac);
+    if (hipGetLastError() != hipSuccess) return fail(HVR_EDEVICE, "blob field kernel launch failed");
+    return volume_from_field(v, field, normals);
 }
 
 int hvr_volume_upload_scalar(hvr_volume *v, const float *data)
@@ -942,7 +961,7 @@ int hvr_volume_upload_scalar(hvr_volume *v, const float *data)
     if (rc != HVR_OK) return rc;
     v->scalar_loaded = true;
     ++v->gen;
-    return compute_range(v);
+    return HVR_OK;
 }
 
 int hvr_volume_upload_normals(hvr_volume *v, const float *data)
@@ -1074,6 +1093,14 @@ int hvr_bind(hvr_ctx *c, hvr_volume *s, int srole, hvr_volume *n, int nrole)
         if (role == HVR_ROLE_SCALAR && !fmt_has_scalar(v->fmt)) return fail(HVR_EINVAL, "volume has no scalar field");
         if (role == HVR_ROLE_NORMAL && !fmt_has_normal(v->fmt)) return fail(HVR_EINVAL, "volume has no normal field");
     }
+    // a volume that was never loaded reads as zeros (a load writes every texel)
+    for (hvr_volume *v : {s, n})
+        if (v && !v->scalar_loaded && !v->normals_loaded && !v->cleared) {
+            HIPCHK(hipSetDevice(c->device));
+            HIPCHK(hipMemsetAsync(v->d_texels, 0, (size_t)v->bytes, c->stream));
+            HIPCHK(hipStreamSynchronize(c->stream));
+            v->cleared = true;
+        }
     c->scalar_vol = s;
     c->normal_vol = n;
     c->scalar_role = srole;
@@ -1397,8 +1424,6 @@ static BatchLaunchFn batch_fn(int fmt, int nm, int lb, bool count, int ts, bool 
     default: return nullptr;
     }
 }
-
-static size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 // Grow a device (and optionally pinned host) buffer to at least `need`
 // bytes.  Returns true when it was reallocated.

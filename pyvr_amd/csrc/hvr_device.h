@@ -1247,37 +1247,6 @@ k_march(const FrameConst fc, const TexDesc ts, const TexDesc tn, const float4 *_
     if constexpr (COUNT) counts[pix] = ns;
 }
 
-// K4 -- per-brick density range of a volume's scalar field: one wave per
-// brick reduces the decoded scalar of its E^3 texels (apron included, so
-// the range covers every footprint the brick serves).  A NaN widens the
-// range to everything.  UNORM8 ranges are in decoded units (raw / 255).
-template <int F, int LB>
-__global__ void __launch_bounds__(256)
-k_brick_range(const char *__restrict__ texels, uint32_t brick_bytes, uint32_t nbricks,
-              float2 *__restrict__ range)
-{
-    const uint32_t brick = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    if (brick >= nbricks) return;
-    constexpr int E = (1 << LB) + 1, N = E * E * E, T = texel_bytes(F);
-    const char *base = texels + (uint64_t)brick * brick_bytes;
-    float lo = INFINITY, hi = -INFINITY;
-    bool nan = false;
-    for (int k = lane; k < N; k += 64) {
-        float v = fetch1<F>(base + (uint64_t)k * T);
-        if constexpr (fmt_u8_scalar(F)) v *= 1.0f / 255.0f;
-        nan |= v != v;
-        lo = fminf(lo, v);
-        hi = fmaxf(hi, v);
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-        lo = fminf(lo, __shfl_xor(lo, off, 64));
-        hi = fmaxf(hi, __shfl_xor(hi, off, 64));
-        nan |= __shfl_xor((int)nan, off, 64) != 0;
-    }
-    if (lane == 0) range[brick] = nan ? make_float2(-INFINITY, INFINITY) : make_float2(lo, hi);
-}
-
 // K5 -- transparent-brick flags for one LUT.  A sample of density rho reads
 // u = clamp(rho*N - 1/2, 0, N-1) and weights entry floor(u) by 1 - frac(u)
 // and entry floor(u) + 1 by frac(u), so the entries with non-zero weight
@@ -1374,12 +1343,9 @@ k_brick_flags(const float2 *__restrict__ range, int nbx, int nby, int nbz, const
     if ((threadIdx.x & 63) == 0 && c) atomicAdd(n_clear, (uint32_t)c);
 }
 
-// K3 -- upload: convert a slab of host float32 data (numpy C order = GL
-// texel order, x fastest) into the volume's texel format and scatter each
-// texel to every slot of the brick layout that holds it (its own slot, the
-// apron copy in the previous brick, and the edge replicas at X = 0 and
-// X = s+1).  part: 1 = scalar field, 2 = normal field (3 floats per voxel).
-// The other part of an interleaved texel is preserved.
+// K3 -- build: a volume's bricks from float32 data in numpy C order (= GL texel
+// order, x fastest).  Sources: the scalar field, the normal field (3 floats
+// per voxel), or a scalar field that also gives the normals by its gradient.
 __device__ __forceinline__ uint32_t enc_sn8(float v)
 {
     v = fminf(fmaxf(v, -1.f), 1.f);  // NaN -> -1 .. kept finite
@@ -1391,89 +1357,47 @@ __device__ __forceinline__ uint32_t enc_u8(float v)
     v = fminf(fmaxf(v, 0.f), 1.f);
     return (uint32_t)rintf(v * 255.f);
 }
+__device__ __forceinline__ uint32_t enc_h(float v) { return (uint32_t)__half_as_ushort(__float2half_rn(v)); }
 
+// A texel as words (the low bytes of one word below 4 bytes): the scalar or
+// the normal put in place, the rest kept.
 template <int F>
-__device__ __forceinline__ void store_part(char *p, int part, const float *val)
+__device__ __forceinline__ void put_scalar(uint32_t *w, float v)
 {
-    if (part == 1) {
-        const float v = val[0];
-        if constexpr (F == TF_S_F32) *(float *)p = v;
-        else if constexpr (F == TF_S_F16) *(__half *)p = __float2half_rn(v);
-        else if constexpr (F == TF_S_U8) *(uint8_t *)p = (uint8_t)enc_u8(v);
-        else if constexpr (F == TF_C_F32_F32) ((float *)p)[3] = v;
-        else if constexpr (F == TF_C_F16_F32) ((uint32_t *)p)[3] = (uint32_t)__half_as_ushort(__float2half_rn(v));
-        else if constexpr (F == TF_C_U8_F32) ((uint32_t *)p)[3] = enc_u8(v);
-        else if constexpr (F == TF_C_F32_SN8) ((float *)p)[0] = v;
-        else if constexpr (F == TF_C_U8_SN8) ((uint8_t *)p)[3] = (uint8_t)enc_u8(v);
-        else if constexpr (F == TF_C_F16_F16 || F == TF_C_F16_SN8) *(__half *)p = __float2half_rn(v);
-    } else {
-        const float nx = val[0], ny = val[1], nz = val[2];
+    if constexpr (F == TF_S_F32 || F == TF_C_F32_SN8) w[0] = __float_as_uint(v);
+    else if constexpr (F == TF_S_F16) w[0] = enc_h(v);
+    else if constexpr (F == TF_S_U8) w[0] = enc_u8(v);
+    else if constexpr (F == TF_C_F32_F32) w[3] = __float_as_uint(v);
+    else if constexpr (F == TF_C_F16_F32) w[3] = enc_h(v);
+    else if constexpr (F == TF_C_U8_F32) w[3] = enc_u8(v);
+    else if constexpr (F == TF_C_U8_SN8) w[0] = (w[0] & 0xffffffu) | enc_u8(v) << 24;
+    else if constexpr (F == TF_C_F16_F16 || F == TF_C_F16_SN8) w[0] = (w[0] & 0xffff0000u) | enc_h(v);
+}
+template <int F>
+__device__ __forceinline__ void put_normal(uint32_t *w, float nx, float ny, float nz)
+{
+    if constexpr (F == TF_N_F32 || F == TF_C_F32_F32 || F == TF_C_F16_F32 || F == TF_C_U8_F32) {
+        w[0] = __float_as_uint(nx);
+        w[1] = __float_as_uint(ny);
+        w[2] = __float_as_uint(nz);
+    } else if constexpr (F == TF_N_SN8 || F == TF_C_F32_SN8 || F == TF_C_U8_SN8) {
         const uint32_t packed = enc_sn8(nx) | (enc_sn8(ny) << 8) | (enc_sn8(nz) << 16);
-        if constexpr (F == TF_N_F32 || F == TF_C_F32_F32 || F == TF_C_F16_F32 || F == TF_C_U8_F32) {
-            float *q = (float *)p;
-            q[0] = nx; q[1] = ny; q[2] = nz;
-            if constexpr (F == TF_N_F32) q[3] = 0.f;
-        } else if constexpr (F == TF_N_SN8) {
-            *(uint32_t *)p = packed;
-        } else if constexpr (F == TF_C_F32_SN8) {
-            ((uint32_t *)p)[1] = packed;
-        } else if constexpr (F == TF_C_F16_SN8) {
-            // the SNORM8 integers as halves (exact), which the march feeds
-            // to v_fma_mix without a conversion per channel and tap
-            __half *q = (__half *)p;   // halves 1..3; half 0 is the scalar
-            q[1] = __int2half_rn((int)(int8_t)(packed & 0xffu));
-            q[2] = __int2half_rn((int)(int8_t)((packed >> 8) & 0xffu));
-            q[3] = __int2half_rn((int)(int8_t)((packed >> 16) & 0xffu));
-        } else if constexpr (F == TF_C_U8_SN8) {
-            uint8_t *q = (uint8_t *)p;
-            q[0] = (uint8_t)(packed & 0xffu); q[1] = (uint8_t)((packed >> 8) & 0xffu);
-            q[2] = (uint8_t)((packed >> 16) & 0xffu);
-        } else if constexpr (F == TF_C_F16_F16) {
-            __half *q = (__half *)p;   // halves 1..3; half 0 is the scalar
-            q[1] = __float2half_rn(nx); q[2] = __float2half_rn(ny); q[3] = __float2half_rn(nz);
-        } else if constexpr (F == TF_N_F16) {
-            __half *q = (__half *)p;
-            q[0] = __float2half_rn(nx); q[1] = __float2half_rn(ny); q[2] = __float2half_rn(nz);
-            q[3] = __float2half_rn(0.f);
-        }
+        if constexpr (F == TF_N_SN8) w[0] = packed;
+        else if constexpr (F == TF_C_F32_SN8) w[1] = packed;
+        else w[0] = (w[0] & 0xff000000u) | packed;
+    } else if constexpr (F == TF_C_F16_SN8) {
+        // the SNORM8 integers as halves (exact), which the march feeds
+        // to v_fma_mix without a conversion per channel and tap
+        const auto h = [](float v) { return (uint32_t)__half_as_ushort(__int2half_rn((int)(int8_t)enc_sn8(v))); };
+        w[0] = (w[0] & 0xffffu) | h(nx) << 16;
+        w[1] = h(ny) | h(nz) << 16;
+    } else if constexpr (F == TF_C_F16_F16) {
+        w[0] = (w[0] & 0xffffu) | enc_h(nx) << 16;
+        w[1] = enc_h(ny) | enc_h(nz) << 16;
+    } else if constexpr (F == TF_N_F16) {
+        w[0] = enc_h(nx) | enc_h(ny) << 16;
+        w[1] = enc_h(nz);
     }
-}
-
-// Write one voxel's part (val: 1 or 3 floats) to every slot holding its
-// texel; (x, y, z) are GL texel coordinates.
-template <int F>
-__device__ __forceinline__ void scatter_texel(char *__restrict__ dst, int x, int y, int z, int s0, int s1, int s2,
-                                              int lb, uint32_t nbx, uint32_t nby, uint32_t nbz,
-                                              uint32_t brick_bytes, int part, const float *val)
-{
-    uint32_t bx[4], lx[4], by[4], ly[4], bz[4], lz[4];
-    const int nx = axis_slots(x, s0, lb, nbx, bx, lx);
-    const int ny = axis_slots(y, s1, lb, nby, by, ly);
-    const int nz = axis_slots(z, s2, lb, nbz, bz, lz);
-    const uint32_t E = (1u << lb) + 1u;
-    constexpr uint32_t T = (uint32_t)texel_bytes(F);
-    for (int k = 0; k < nz; ++k)
-        for (int j = 0; j < ny; ++j)
-            for (int i = 0; i < nx; ++i) {
-                const uint32_t brick = (bz[k] * nby + by[j]) * nbx + bx[i];
-                const uint32_t local = (lz[k] * E + ly[j]) * E + lx[i];
-                store_part<F>(dst + (uint64_t)brick * brick_bytes + (uint64_t)local * T, part, val);
-            }
-}
-
-template <int F>
-__global__ void __launch_bounds__(256)
-k_upload(char *__restrict__ dst, int s0, int s1, int s2, int lb, uint32_t nbx, uint32_t nby, uint32_t nbz,
-         uint32_t brick_bytes, const float *__restrict__ src, int part, int z0, uint64_t nvox)
-{
-    const uint64_t l = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (l >= nvox) return;
-    const uint64_t plane = (uint64_t)s0 * (uint64_t)s1;
-    const int z = (int)(l / plane) + z0;
-    const uint64_t rem = l % plane;
-    const int y = (int)(rem / (uint64_t)s0), x = (int)(rem % (uint64_t)s0);
-    scatter_texel<F>(dst, x, y, z, s0, s1, s2, lb, nbx, nby, nbz, brick_bytes, part,
-                     src + (part == 1 ? l : 3 * l));
 }
 
 // Normals of a device float32 field (numpy C order, shape (s0, s1, s2)),
@@ -1483,37 +1407,156 @@ k_upload(char *__restrict__ dst, int s0, int s1, int s2, int lb, uint32_t nbx, u
 // spacing), the norm sqrt((gx^2 + gy^2) + gz^2) summed left to right as
 // numpy does, plus float32(1e-8), and each component divided by it -- all
 // correctly rounded float32 operations.  Every axis has at least 2 voxels.
-__device__ __forceinline__ float np_gradient(const float *__restrict__ f, uint64_t l, int i, int n, uint64_t st)
+template <typename I>
+__device__ __forceinline__ float np_gradient(const float *__restrict__ f, I l, int i, int n, I st)
 {
-    if (i == 0) return __fsub_rn(f[l + st], f[l]);
-    if (i == n - 1) return __fsub_rn(f[l], f[l - st]);
-    return __fmul_rn(__fsub_rn(f[l + st], f[l - st]), 0.5f);  // /2, exact
+    // the voxel itself stands in for the neighbour past a face
+    const float hi = f[i == n - 1 ? l : l + st], lo = f[i == 0 ? l : l - st], d = __fsub_rn(hi, lo);
+    return i == 0 || i == n - 1 ? d : __fmul_rn(d, 0.5f);  // /2, exact
 }
 
-template <int F>
-__global__ void __launch_bounds__(256)
-k_normals_from_field(char *__restrict__ dst, int s0, int s1, int s2, int lb, uint32_t nbx, uint32_t nby,
-                     uint32_t nbz, uint32_t brick_bytes, const float *__restrict__ field, uint64_t nvox)
+// l / d for l below 2^32: the quotient by double multiplication is off by one at most.
+__device__ __forceinline__ uint32_t div_u32(uint32_t l, uint32_t d, double inv)
 {
-    const uint64_t l = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (l >= nvox) return;
-    // numpy coordinates of flat index l
-    const uint64_t n12 = (uint64_t)s1 * (uint64_t)s2;
-    const int i0 = (int)(l / n12);
-    const uint64_t r12 = l % n12;
-    const int i1 = (int)(r12 / (uint64_t)s2), i2 = (int)(r12 % (uint64_t)s2);
-    const float gx = np_gradient(field, l, i0, s0, n12);
-    const float gy = np_gradient(field, l, i1, s1, (uint64_t)s2);
-    const float gz = np_gradient(field, l, i2, s2, 1);
-    const float nn = __fadd_rn(__fsqrt_rn(__fadd_rn(__fadd_rn(__fmul_rn(gx, gx), __fmul_rn(gy, gy)), __fmul_rn(gz, gz))),
-                               1e-8f);
-    const float val[3] = {__fdiv_rn(gx, nn), __fdiv_rn(gy, nn), __fdiv_rn(gz, nn)};
-    // GL texel coordinates of the same flat index
-    const uint64_t plane = (uint64_t)s0 * (uint64_t)s1;
-    const int z = (int)(l / plane);
-    const uint64_t rem = l % plane;
-    const int y = (int)(rem / (uint64_t)s0), x = (int)(rem % (uint64_t)s0);
-    scatter_texel<F>(dst, x, y, z, s0, s1, s2, lb, nbx, nby, nbz, brick_bytes, 2, val);
+    uint32_t q = (uint32_t)((double)l * inv);
+    if (q * d > l) --q;                  // q * d is below 2^32 + d
+    else if (l - q * d >= d) ++q;
+    return q;
+}
+
+struct BuildArgs {
+    char *dst;
+    int s0, s1, s2;            // GL size
+    uint32_t nbx, nby, bz0;    // bricks; the launch's first brick layer
+    uint64_t runs;             // groups of build_bricks bricks along x in the launch
+    const float *scalar;       // the source, of one kind
+    const float *normal;
+    const float *field;
+    uint64_t first;            // flat index of the source's first voxel
+    double inv_n12, inv_s2;    // 1 / (s1 s2), 1 / s2
+    int keep;                  // the texels hold the other part, which stays
+    float2 *range;             // per-brick density range, where the scalar is written
+};
+constexpr int build_bricks(int lb) { return lb == 4 ? 4 : 8; }   // bricks along x per block
+
+// One wave per brick (all 4 of a block for 16^3 bricks, which are as many
+// times fewer), build_bricks bricks along x per block.  Every slot of a brick
+// is written once, in order, from its voxel: texel X = c + 1 of an axis holds
+// voxel c, X = 0 and X = s + 1 the edge voxels, and slots past those are 0.
+// Per-brick density range (for the transparent-brick flags): over all slots as
+// stored, the apron included, so that it covers every footprint the brick
+// serves; a NaN widens it to everything.  UNORM8 ranges are in decoded units
+// (raw / 255).
+// Writing the bricks bounds a scalar or normal part (FP32+FP32x3 192^3: 70 us
+// for the scalar and 126 for the normals, which read the texels too; 2.6 and
+// 3.5 TB/s), the
+// instructions of the gradient, its norm and its divisions a field.  Writing
+// whole texels in order, the range formed on the way, replaces a thread per
+// voxel that scattered it to its up to eight slots, a clearing pass and a pass
+// for the ranges: FP16+FP16x3 255x193x160 from a field 174 -> 91 us, 320^3 in
+// 16^3 bricks 709 -> 270; FP32+FP32x3 192^3 in its two parts 236 -> 196.
+template <int F, int LB, typename I>
+__global__ void __launch_bounds__(256)
+k_build(const BuildArgs a)
+{
+    constexpr uint32_t B = 1u << LB, E = B + 1u, N = E * E * E, T = (uint32_t)texel_bytes(F), W = (T + 3) / 4;
+    constexpr uint32_t G = (uint32_t)build_bricks(LB), V = LB == 4 ? 4 : 1;   // V: waves per brick
+    __shared__ float s_range[3][4];
+    const uint32_t ngx = (a.nbx + G - 1) / G, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const I plane = (I)a.s0 * (I)a.s1, n12 = (I)a.s1 * (I)a.s2, first = (I)a.first;
+    for (uint64_t run = blockIdx.x; run < a.runs; run += gridDim.x)
+    for (uint32_t j = wave / V; j < G; j += 4 / V) {
+        const uint32_t bx = (uint32_t)(run % ngx) * G + j, by = (uint32_t)(run / ngx % a.nby),
+                       bz = a.bz0 + (uint32_t)(run / ngx / a.nby);
+        if (bx >= a.nbx) break;
+        const uint64_t brick = ((uint64_t)bz * a.nby + by) * a.nbx + bx;
+        char *out = a.dst + brick * ((uint64_t)N * T);
+        float lo = INFINITY, hi = -INFINITY;
+        bool nan = false;
+        for (uint32_t k = wave % V * 64 + lane; k < N; k += 64 * V) {
+            const uint32_t X = bx * B + k % E, Y = by * B + k / E % E, Z = bz * B + k / (E * E);
+            uint32_t w[W] = {};
+            if (X <= (uint32_t)a.s0 + 1u && Y <= (uint32_t)a.s1 + 1u && Z <= (uint32_t)a.s2 + 1u) {
+                const int x = slot_voxel(X, a.s0), y = slot_voxel(Y, a.s1), z = slot_voxel(Z, a.s2);
+                const I l = (I)z * plane + (I)y * (I)a.s0 + (I)x;
+                if (T >= 4 && a.keep) {
+#pragma unroll
+                    for (uint32_t q = 0; q < W; ++q) w[q] = ((const uint32_t *)(out + k * T))[q];
+                }
+                if (a.normal) {
+                    const float *n = a.normal + 3 * (uint64_t)(l - first);
+                    put_normal<F>(w, n[0], n[1], n[2]);
+                } else if (a.scalar) {
+                    put_scalar<F>(w, a.scalar[l - first]);
+                } else {
+                    put_scalar<F>(w, a.field[l]);
+                    if constexpr (fmt_has_normal(F)) {
+                        // numpy coordinates of flat index l
+                        int i0 = z, i1 = y, i2 = x;
+                        if (a.s0 != a.s2) {
+                            if constexpr (sizeof(I) == 4) {
+                                i0 = (int)div_u32(l, n12, a.inv_n12);
+                                const uint32_t r = l - (uint32_t)i0 * n12;
+                                i1 = (int)div_u32(r, (uint32_t)a.s2, a.inv_s2);
+                                i2 = (int)(r - (uint32_t)i1 * (uint32_t)a.s2);
+                            } else {
+                                i0 = (int)(l / n12);
+                                const I r = l - (I)i0 * n12;
+                                i1 = (int)(r / (I)a.s2);
+                                i2 = (int)(r - (I)i1 * (I)a.s2);
+                            }
+                        }
+                        const float gx = np_gradient(a.field, l, i0, a.s0, n12);
+                        const float gy = np_gradient(a.field, l, i1, a.s1, (I)a.s2);
+                        const float gz = np_gradient(a.field, l, i2, a.s2, (I)1);
+                        const float nn = __fadd_rn(
+                            __fsqrt_rn(__fadd_rn(__fadd_rn(__fmul_rn(gx, gx), __fmul_rn(gy, gy)), __fmul_rn(gz, gz))),
+                            1e-8f);
+                        put_normal<F>(w, __fdiv_rn(gx, nn), __fdiv_rn(gy, nn), __fdiv_rn(gz, nn));
+                    }
+                }
+            }
+            char *p = out + k * T;
+            if constexpr (T == 1) *(uint8_t *)p = (uint8_t)w[0];
+            else if constexpr (T == 2) *(uint16_t *)p = (uint16_t)w[0];
+            else {
+#pragma unroll
+                for (uint32_t q = 0; q < W; ++q) ((uint32_t *)p)[q] = w[q];
+            }
+            if constexpr (fmt_has_scalar(F)) {
+                float v;
+                if constexpr (F == TF_S_F16) v = h16f(w[0]);
+                else if constexpr (F == TF_S_U8) v = (float)w[0];
+                else if constexpr (F == TF_S_F32) v = __uint_as_float(w[0]);
+                else v = decode_scalar<F>(w);
+                if constexpr (fmt_u8_scalar(F)) v *= 1.0f / 255.0f;
+                nan |= v != v;
+                lo = fminf(lo, v);
+                hi = fmaxf(hi, v);
+            }
+        }
+        if (fmt_has_scalar(F) && a.range) {
+            for (int off = 32; off > 0; off >>= 1) {
+                lo = fminf(lo, __shfl_xor(lo, off, 64));
+                hi = fmaxf(hi, __shfl_xor(hi, off, 64));
+            }
+            nan = __ballot(nan) != 0;
+            if constexpr (V > 1) {   // every wave of the block is at this brick
+                if (lane == 0) {
+                    s_range[0][wave] = lo;
+                    s_range[1][wave] = hi;
+                    s_range[2][wave] = nan ? 1.f : 0.f;
+                }
+                __syncthreads();
+                lo = fminf(fminf(s_range[0][0], s_range[0][1]), fminf(s_range[0][2], s_range[0][3]));
+                hi = fmaxf(fmaxf(s_range[1][0], s_range[1][1]), fmaxf(s_range[1][2], s_range[1][3]));
+                nan = s_range[2][0] + s_range[2][1] + s_range[2][2] + s_range[2][3] != 0.f;
+                __syncthreads();
+            }
+            if (lane == 0 && wave % V == 0) a.range[brick] = nan ? make_float2(-INFINITY, INFINITY) : make_float2(lo, hi);
+        }
+    }
 }
 
 // Seeded Gaussian-blob field generated on the device (numpy C order): the
@@ -1545,29 +1588,61 @@ __device__ __forceinline__ double np_linspace(int i, int n)
     return (double)i * (2.0 / (double)(n - 1)) + -1.0;
 }
 
+// The blobs' factors exp(-(axis - centre)^2 / (2 sigma^2)) along each axis:
+// for blob b, s0 of them at fac + b * (s0 + s1 + s2), then s1, then s2.
 static __global__ void __launch_bounds__(256)
-k_blob_field(float *__restrict__ out, int s0, int s1, int s2, const BlobSpec *__restrict__ spec, uint64_t nvox)
+k_blob_factors(double *__restrict__ fac, int s0, int s1, int s2, const BlobSpec *__restrict__ spec)
 {
-    const uint64_t l = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (l >= nvox) return;
-    const uint64_t n12 = (uint64_t)s1 * (uint64_t)s2;
-    const int i0 = (int)(l / n12);
-    const uint64_t r12 = l % n12;
-    const int i1 = (int)(r12 / (uint64_t)s2), i2 = (int)(r12 % (uint64_t)s2);
-    const double x = np_linspace(i0, s0), y = np_linspace(i1, s1), z = np_linspace(i2, s2);
-    double acc = 0.0;
-    for (int b = 0; b < spec->n; ++b) {
+    const int len = s0 + s1 + s2;
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < (int64_t)len * spec->n;
+         t += (int64_t)gridDim.x * 256) {
+        const int b = (int)(t / len), j = (int)(t % len);
+        const int axis = j < s0 ? 0 : j < s0 + s1 ? 1 : 2;
+        const int i = axis == 0 ? j : axis == 1 ? j - s0 : j - s0 - s1;
         const double k = 2.0 * spec->s[b] * spec->s[b];
-        const double dx = x - spec->c[3 * b], dy = y - spec->c[3 * b + 1], dz = z - spec->c[3 * b + 2];
-        const double fx = exp(-(dx * dx) / k), fy = exp(-(dy * dy) / k), fz = exp(-(dz * dz) / k);
-        acc += spec->a[b] * (fx * (fy * fz));
+        const double d = np_linspace(i, axis == 0 ? s0 : axis == 1 ? s1 : s2) - spec->c[3 * b + axis];
+        fac[t] = exp(-(d * d) / k);
     }
-    if (spec->noise > 0.0) {
-        const uint64_t h = splitmix64(spec->seed ^ splitmix64(l));
-        const double u = (double)(h >> 11) * 0x1p-53;  // [0, 1)
-        acc += (2.0 * u - 1.0) * spec->noise;
+}
+
+// A wave takes 64 voxels along the last axis and kBlobRows rows of the middle
+// one: the last axis' factor is a load per blob, the others' are scalar.
+// With every factor computed at every voxel (three exponentials in double per
+// blob) the kernel took 1058 us for 8 blobs at 320^3; these two take 106.
+static constexpr int kBlobRows = 8;
+static __global__ void __launch_bounds__(256)
+k_blob_field(float *__restrict__ out, int s0, int s1, int s2, const BlobSpec *__restrict__ spec,
+             const double *__restrict__ fac)
+{
+    const uint64_t nz = ((uint64_t)s2 + 63) / 64, ny = ((uint64_t)s1 + kBlobRows - 1) / kBlobRows, total = nz * ny * s0;
+    const int len = s0 + s1 + s2, n = spec->n;
+    const double noise = spec->noise;
+    for (uint64_t t = (uint64_t)blockIdx.x * 4 + (uint64_t)(__builtin_amdgcn_readfirstlane((int)threadIdx.x) >> 6);
+         t < total; t += (uint64_t)gridDim.x * 4) {
+        const int i2 = (int)(t % nz) * 64 + (int)(threadIdx.x & 63), j1 = (int)(t / nz % ny) * kBlobRows,
+                  i0 = (int)(t / nz / ny);
+        const int c2 = min(i2, s2 - 1);
+        double acc[kBlobRows] = {};
+        for (int b = 0; b < n; ++b) {
+            const double *f = fac + (int64_t)b * len;
+            const double amp = spec->a[b], fx = f[i0], fz = f[s0 + s1 + c2];
+#pragma unroll
+            for (int r = 0; r < kBlobRows; ++r) acc[r] += amp * (fx * (f[s0 + min(j1 + r, s1 - 1)] * fz));
+        }
+        if (i2 >= s2) continue;
+#pragma unroll
+        for (int r = 0; r < kBlobRows; ++r) {
+            if (j1 + r >= s1) break;
+            const uint64_t l = ((uint64_t)i0 * s1 + (uint64_t)(j1 + r)) * s2 + (uint64_t)i2;
+            double v = acc[r];
+            if (noise > 0.0) {
+                const uint64_t h = splitmix64(spec->seed ^ splitmix64(l));
+                const double u = (double)(h >> 11) * 0x1p-53;  // [0, 1)
+                v += (2.0 * u - 1.0) * noise;
+            }
+            out[l] = (float)fmin(fmax(v, 0.0), 1.0);
+        }
     }
-    out[l] = (float)fmin(fmax(acc, 0.0), 1.0);
 }
 
 // ---------------------------------------------------------------------------

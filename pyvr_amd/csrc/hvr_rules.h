@@ -45,6 +45,14 @@ constexpr int axis_slots(int c, int s, int lb, uint32_t nb, uint32_t br[4], uint
     return n;
 }
 
+// The voxel that texel X of an axis (extended coordinates) holds, X <= s + 1:
+// the inverse of axis_slots, which names the slots of a voxel.
+constexpr int slot_voxel(uint32_t X, int s)
+{
+    const int c = (int)X - 1;
+    return c < 0 ? 0 : c < s ? c : s - 1;
+}
+
 // Whether a brick whose density range is [lo, hi] can only ever sample LUT
 // entries that are exactly transparent.  A sample of density rho reads
 // u = clamp(rho*N - 1/2, 0, N-1) and weights entry floor(u) by 1 - frac(u)
