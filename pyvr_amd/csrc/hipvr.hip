@@ -80,8 +80,9 @@ struct hvr_volume {
     uint32_t brick_bytes;  // (2^lb + 1)^3 texels
     uint64_t bytes;
     void *d_texels;
+    size_t block_bytes;    // of the allocation: the texels, then the ranges
     bool scalar_loaded, normals_loaded, cleared;
-    float2 *d_range;       // per-brick scalar range (after a scalar upload)
+    float2 *d_range;       // per-brick scalar range (formats with a scalar field)
     uint32_t gen;          // bumped on every upload
 };
 
@@ -100,6 +101,8 @@ struct hvr_ctx {
     bool last_host;       // the last frame was written to h_pinned
     float *d_stage;  // upload staging
     size_t stage_bytes;
+    char *h_up;           // pinned ring the uploads go through (upload_host), or nullptr
+    hipEvent_t up_ev[3];  // after the last copy out of each of its parts
     hipEvent_t ev[4];
     hipEvent_t rev[4];   // readback chunks (hvr_read)
     hipEvent_t last_ev[3];  // the last frame's events (ev[] or a timing region's)
@@ -154,6 +157,87 @@ static constexpr double kSkipAutoFraction = 0.25;
 // threads per compute unit.
 static long long resident_rays(const hvr_ctx *c) { return 2048ll * c->ncu; }
 
+
+// ---------------------------------------------------------------------------
+// Device memory of volumes.  A program that shows a sequence of volumes frees
+// one block and allocates another of the same size for each; above 64 MB hipMalloc
+// and hipFree take 60 and 265 us, and blocks of hundreds of MB that come and
+// go at that rate have stalled hipMalloc for 11 ms at a time.  The last block
+// freed on a device is therefore kept for the next volume on it, from any
+// context: at most one, of at most kSpareMax bytes.  It is given back when
+// the next volume cannot use it (too small, or more than a quarter too large),
+// when an allocation fails for want of memory, and with the device's last
+// context.  A block is put aside only once the device is idle, as hipFree
+// would wait for, so no stream still reads it.
+static constexpr size_t kSpareMax = (size_t)512 << 20;
+static constexpr int kMaxDevices = 64;
+struct SpareBlock {
+    void *p;
+    size_t bytes;
+    int contexts;   // live contexts of the device
+};
+static std::mutex g_spare_mu;
+static SpareBlock g_spare[kMaxDevices];
+
+// Take the device's spare block out (nullptr if there is none).
+static void *spare_take(int device, size_t *bytes)
+{
+    if (device < 0 || device >= kMaxDevices) return nullptr;
+    std::lock_guard<std::mutex> lock(g_spare_mu);
+    void *p = g_spare[device].p;
+    *bytes = g_spare[device].bytes;
+    g_spare[device].p = nullptr;
+    return p;
+}
+// hipMalloc that gives the spare block back before it fails; the device is current.
+static hipError_t dev_malloc(int device, void **p, size_t n)
+{
+    hipError_t e = hipMalloc(p, n);
+    if (e == hipErrorOutOfMemory) {
+        size_t b;
+        if (void *spare = spare_take(device, &b)) {
+            (void)hipGetLastError();
+            (void)hipFree(spare);
+            e = hipMalloc(p, n);
+        }
+    }
+    return e;
+}
+static hipError_t block_alloc(int device, void **p, size_t n, size_t *got)
+{
+    size_t b = 0;
+    if (void *spare = spare_take(device, &b)) {
+        if (b >= n && b - n <= n / 4) {
+            *p = spare;
+            *got = b;
+            return hipSuccess;
+        }
+        (void)hipFree(spare);
+    }
+    *got = n;
+    return dev_malloc(device, p, n);
+}
+static void block_free(int device, void *p, size_t n)
+{
+    if (!p) return;
+    if (n <= kSpareMax && device >= 0 && device < kMaxDevices && hipDeviceSynchronize() == hipSuccess) {
+        std::lock_guard<std::mutex> lock(g_spare_mu);
+        std::swap(g_spare[device].p, p);
+        g_spare[device].bytes = n;
+    }
+    (void)hipFree(p);   // the block before, or this one
+}
+static void context_count(int device, int by)
+{
+    if (device < 0 || device >= kMaxDevices) return;
+    bool last;
+    {
+        std::lock_guard<std::mutex> lock(g_spare_mu);
+        last = (g_spare[device].contexts += by) == 0;
+    }
+    size_t b;
+    if (last) (void)hipFree(spare_take(device, &b));
+}
 
 // ---------------------------------------------------------------------------
 // FP64 uniform preparation
@@ -270,7 +354,7 @@ static bool flags_count(hvr_ctx *c, bool wait)
 // image, so the choice only affects speed); nullptr otherwise.
 static const uint8_t *brick_flags(hvr_ctx *c, const hvr_volume *v)
 {
-    if (c->skip_mode == HVR_SKIP_OFF || !v || !v->d_range || !c->d_nz) return nullptr;
+    if (c->skip_mode == HVR_SKIP_OFF || !v || !v->scalar_loaded || !c->d_nz) return nullptr;
     const uint64_t nb = (uint64_t)v->nbx * v->nby * v->nbz;
     // without flags the frame takes the non-skipping kernel: a failure here
     // is handled, not reported
@@ -289,7 +373,7 @@ static const uint8_t *brick_flags(hvr_ctx *c, const hvr_volume *v)
             (void)hipFree(c->d_flags);
             c->d_flags = nullptr;
             c->flags_cap = 0;
-            if (hipMalloc(&c->d_flags, nb) != hipSuccess) return none();
+            if (dev_malloc(c->device, (void **)&c->d_flags, nb) != hipSuccess) return none();
             c->flags_cap = nb;
         }
         // the count comes back asynchronously (no wait in the frame's path)
@@ -426,7 +510,7 @@ static int enqueue_frame(hvr_ctx *c, bool count, uchar4 *dst, bool count_shaded 
             (void)hipFree(c->d_order);
             c->d_order = nullptr;
             c->order_words = 0;
-            HIPCHK(hipMalloc(&c->d_order, words * sizeof(uint32_t)));
+            HIPCHK(dev_malloc(c->device, (void **)&c->d_order, words * sizeof(uint32_t)));
             c->order_words = words;
         }
     }
@@ -509,13 +593,6 @@ static int build_layers(const hvr_volume *v, BuildArgs a, uint32_t bz0, uint32_t
     return HVR_OK;
 }
 
-// The density ranges' buffer, before the scalar is written.
-static int need_range(hvr_volume *v)
-{
-    if (!v->d_range) HIPCHK(hipMalloc(&v->d_range, (size_t)v->nbx * v->nby * v->nbz * sizeof(float2)));
-    return HVR_OK;
-}
-
 static size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 // The context's staging buffer, of at least `need` bytes.
@@ -526,11 +603,45 @@ static int need_stage(hvr_ctx *c, size_t need)
     (void)hipFree(c->d_stage);
     c->d_stage = nullptr;
     c->stage_bytes = 0;
-    HIPCHK(hipMalloc(&c->d_stage, need));
+    HIPCHK(dev_malloc(c->device, (void **)&c->d_stage, need));
     c->stage_bytes = need;
     return HVR_OK;
 }
 static constexpr size_t kMaxStage = (size_t)256 << 20;   // what stays allocated, but for larger single planes
+
+// Host data to the device, in stream order.  From pageable memory one thread of
+// the runtime copies into pinned memory, at 30 GB/s; here four threads do
+// (CopyPool), piece by piece through a ring of three pinned parts, while the
+// pieces before cross the link at its 57 GB/s.  The caller's data is read when
+// this returns.  Less than a piece, and where the ring cannot be had, goes
+// the runtime's way.
+static constexpr size_t kUploadPiece = (size_t)4 << 20;
+static int upload_host(hvr_ctx *c, void *dst, const void *src, size_t bytes)
+{
+    if (bytes >= kUploadPiece && !c->h_up) {
+        bool ok = hipHostMalloc((void **)&c->h_up, 3 * kUploadPiece, hipHostMallocDefault) == hipSuccess;
+        for (hipEvent_t &e : c->up_ev)
+            if (ok && !e) ok = hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+        if (!ok) {
+            (void)hipGetLastError();
+            if (c->h_up) (void)hipHostFree(c->h_up);
+            c->h_up = nullptr;
+        }
+    }
+    if (bytes < kUploadPiece || !c->h_up) {
+        HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
+        return HVR_OK;
+    }
+    for (size_t at = 0, k = 0; at < bytes; at += kUploadPiece, ++k) {
+        const size_t n = std::min(kUploadPiece, bytes - at);
+        char *part = c->h_up + k % 3 * kUploadPiece;
+        HIPCHK(hipEventSynchronize(c->up_ev[k % 3]));   // at once when never recorded
+        hvr::CopyPool::get().copy((uint8_t *)part, (const uint8_t *)src + at, n);
+        HIPCHK(hipMemcpyAsync((char *)dst + at, part, n, hipMemcpyHostToDevice, c->stream));
+        HIPCHK(hipEventRecord(c->up_ev[k % 3], c->stream));
+    }
+    return HVR_OK;
+}
 
 // Device memory for a whole field while a volume is built from it: the staging
 // buffer up to kMaxStage, else an allocation given back (after the stream's
@@ -548,7 +659,7 @@ struct FieldBuffer {
             p = (char *)c->d_stage;
             return HVR_OK;
         }
-        HIPCHK(hipMalloc(&p, bytes));
+        HIPCHK(dev_malloc(c->device, (void **)&p, bytes));
         own = true;
         return HVR_OK;
     }
@@ -612,6 +723,7 @@ int hvr_create(int device, int width, int height, hvr_ctx **out)
     hvr_ctx *c = new hvr_ctx();
     memset(c, 0, sizeof(*c));
     c->device = device;
+    context_count(device, 1);
     c->W = width;
     c->H = height;
     c->brick_log2 = 3;
@@ -624,7 +736,7 @@ int hvr_create(int device, int width, int height, hvr_ctx **out)
     noalloc_setup(device);
     hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&c->ncu, hipDeviceAttributeMultiprocessorCount, device);
-    if (e == hipSuccess) e = hipMalloc(&c->d_out, npix * sizeof(uchar4));
+    if (e == hipSuccess) e = dev_malloc(device, (void **)&c->d_out, npix * sizeof(uchar4));
     if (e == hipSuccess) e = hipHostMalloc(&c->h_pinned, npix * 4, hipHostMallocDefault);
     if (e == hipSuccess) e = hipHostGetDevicePointer(&c->h_pinned_dev, c->h_pinned, 0);
     if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_nclear, sizeof(uint32_t), hipHostMallocDefault);
@@ -636,7 +748,7 @@ int hvr_create(int device, int width, int height, hvr_ctx **out)
         // unbound LUT: a 1-texel (0, 0, 0, 1) texture (GL incomplete texture)
         c->lut_cap = 1;
         c->lut_n = 1;
-        e = hipMalloc(&c->d_lut, sizeof(float4));
+        e = dev_malloc(device, (void **)&c->d_lut, sizeof(float4));
         const float4 unbound = make_float4(0.f, 0.f, 0.f, 1.f);
         if (e == hipSuccess) e = hipMemcpy(c->d_lut, &unbound, sizeof(float4), hipMemcpyHostToDevice);
     }
@@ -669,7 +781,7 @@ int hvr_resize(hvr_ctx *c, int width, int height)
         c->h_pinned_dev = nullptr;
         c->last_host = false;
         c->pix_cap = 0;
-        HIPCHK(hipMalloc(&c->d_out, npix * sizeof(uchar4)));
+        HIPCHK(dev_malloc(c->device, (void **)&c->d_out, npix * sizeof(uchar4)));
         HIPCHK(hipHostMalloc(&c->h_pinned, npix * 4, hipHostMallocDefault));
         HIPCHK(hipHostGetDevicePointer(&c->h_pinned_dev, c->h_pinned, 0));
         HIPCHK(hipMemset(c->d_out, 0, npix * sizeof(uchar4)));
@@ -695,6 +807,9 @@ int hvr_destroy(hvr_ctx *c)
     (void)hipFree(c->d_order);
     if (c->h_pinned) (void)hipHostFree(c->h_pinned);
     if (c->h_nclear) (void)hipHostFree(c->h_nclear);
+    if (c->h_up) (void)hipHostFree(c->h_up);
+    for (hipEvent_t e : c->up_ev)
+        if (e) (void)hipEventDestroy(e);
     if (c->flags_ev) (void)hipEventDestroy(c->flags_ev);
     for (int i = 0; i < 4; ++i) {
         if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
@@ -707,6 +822,7 @@ int hvr_destroy(hvr_ctx *c)
         delete c->tev;
     }
     if (c->stream) (void)hipStreamDestroy(c->stream);
+    context_count(c->device, -1);
     delete c;
     return HVR_OK;
 }
@@ -824,13 +940,15 @@ int hvr_volume_create(hvr_ctx *c, int s0, int s1, int s2, int sf, int nf, hvr_vo
         return fail(HVR_EINVAL, "volume too large (brick index exceeds 32 bits)");
     }
     v->bytes = nbricks * v->brick_bytes;
-    const size_t bytes = (size_t)v->bytes;
+    const size_t range_at = align_up((size_t)v->bytes, 256),
+                 bytes = fmt_has_scalar(fmt) ? range_at + (size_t)nbricks * sizeof(float2) : (size_t)v->bytes;
     hipError_t e = hipSetDevice(c->device);
-    if (e == hipSuccess) e = hipMalloc(&v->d_texels, bytes);
+    if (e == hipSuccess) e = block_alloc(c->device, &v->d_texels, bytes, &v->block_bytes);
     if (e != hipSuccess) {
         delete v;
         return fail_hip(e, "hvr_volume_create");
     }
+    if (fmt_has_scalar(fmt)) v->d_range = (float2 *)((char *)v->d_texels + range_at);
     *out = v;
     return HVR_OK;
 }
@@ -849,8 +967,6 @@ static int upload_part(hvr_volume *v, const float *data, int part)
     const uint64_t fit = kMaxStage / row;   // planes
     const uint32_t group = fit > (uint64_t)B + 2 ? (uint32_t)((fit - 2) / B) : 1;   // layers
     if (const int rc = need_stage(c, (size_t)std::min<uint64_t>((uint64_t)group * B + 2, (uint64_t)v->s2) * row)) return rc;
-    if (part == 1)
-        if (const int rc = need_range(v)) return rc;
     BuildArgs a;
     memset(&a, 0, sizeof(a));
     (part == 1 ? a.scalar : a.normal) = c->d_stage;
@@ -862,8 +978,7 @@ static int upload_part(hvr_volume *v, const float *data, int part)
         const int64_t z0 = std::min<int64_t>(std::max<int64_t>((int64_t)bz * B - 1, 0), v->s2 - 1),
                       z1 = std::min<int64_t>((int64_t)end * B, v->s2);   // one past the last
         a.first = (uint64_t)z0 * plane;
-        HIPCHK(hipMemcpyAsync(c->d_stage, data + a.first * comps, (size_t)(z1 - z0) * row, hipMemcpyHostToDevice,
-                              c->stream));
+        if (const int rc = upload_host(c, c->d_stage, data + a.first * comps, (size_t)(z1 - z0) * row)) return rc;
         if (const int rc = build_layers(v, a, bz, end)) return rc;
         // the staging buffer is reused by the next group
         HIPCHK(hipStreamSynchronize(c->stream));
@@ -877,7 +992,6 @@ static int volume_from_field(hvr_volume *v, const float *d_field, bool normals)
 {
     hvr_ctx *c = v->ctx;
     if (!fmt_has_scalar(v->fmt)) return fail(HVR_EINVAL, "the volume has no scalar field");
-    if (const int rc = need_range(v)) return rc;
     BuildArgs a;
     memset(&a, 0, sizeof(a));
     normals = normals && fmt_has_normal(v->fmt);
@@ -905,8 +1019,7 @@ int hvr_volume_upload_scalar_normals(hvr_volume *v, const float *data)
     const size_t bytes = (size_t)v->s0 * v->s1 * v->s2 * sizeof(float);
     FieldBuffer f(c);
     if (const int rc = f.get(bytes)) return rc;
-    if (hipMemcpyAsync(f.p, data, bytes, hipMemcpyHostToDevice, c->stream) != hipSuccess)
-        return fail(HVR_EDEVICE, "copying the scalar field to the device failed");
+    if (const int rc = upload_host(c, f.p, data, bytes)) return rc;
     return volume_from_field(v, (const float *)f.p, true);
 }
 
@@ -993,8 +1106,7 @@ int hvr_volume_destroy(hvr_volume *v)
     if (c->scalar_vol == v) c->scalar_vol = nullptr;
     if (c->normal_vol == v) c->normal_vol = nullptr;
     if (c->flags_vol == v) c->flags_vol = nullptr;
-    (void)hipFree(v->d_texels);
-    (void)hipFree(v->d_range);
+    block_free(c->device, v->d_texels, v->block_bytes);
     delete v;
     return HVR_OK;
 }
@@ -1018,14 +1130,14 @@ int hvr_set_lut(hvr_ctx *c, const float *rgba, int n)
         (void)hipFree(c->d_lut);
         c->d_lut = nullptr;
         c->lut_cap = 0;
-        HIPCHK(hipMalloc(&c->d_lut, lut_bytes));
+        HIPCHK(dev_malloc(c->device, (void **)&c->d_lut, lut_bytes));
         c->lut_cap = cnt;
     }
     if (cnt > c->nz_cap) {
         (void)hipFree(c->d_nz);
         c->d_nz = nullptr;
         c->nz_cap = 0;
-        HIPCHK(hipMalloc(&c->d_nz, nz_bytes));
+        HIPCHK(dev_malloc(c->device, (void **)&c->d_nz, nz_bytes));
         c->nz_cap = cnt;
     }
     if (lut_bytes + nz_bytes > c->lut_stage_bytes) {
@@ -1129,7 +1241,7 @@ int hvr_device_alloc(hvr_ctx *c, uint64_t bytes, void **ptr)
     if (!c || !ptr) return fail(HVR_EINVAL, "null argument");
     *ptr = nullptr;
     HIPCHK(hipSetDevice(c->device));
-    HIPCHK(hipMalloc(ptr, bytes ? bytes : 1));
+    HIPCHK(dev_malloc(c->device, ptr, bytes ? bytes : 1));
     return HVR_OK;
 }
 
@@ -1277,7 +1389,7 @@ static int sample_counts(hvr_ctx *c, uint32_t *counts, bool shaded)
         (void)hipFree(c->d_counts);
         c->d_counts = nullptr;
         c->counts_cap = 0;
-        HIPCHK(hipMalloc(&c->d_counts, npix * sizeof(uint32_t)));
+        HIPCHK(dev_malloc(c->device, (void **)&c->d_counts, npix * sizeof(uint32_t)));
         c->counts_cap = npix;
     }
     int rc = enqueue_frame(c, true, nullptr, shaded);
@@ -1312,12 +1424,12 @@ int hvr_touched_bricks(hvr_ctx *c, unsigned long long *touched, unsigned long lo
         (void)hipFree(c->d_counts);
         c->d_counts = nullptr;
         c->counts_cap = 0;
-        HIPCHK(hipMalloc(&c->d_counts, npix * sizeof(uint32_t)));
+        HIPCHK(dev_malloc(c->device, (void **)&c->d_counts, npix * sizeof(uint32_t)));
         c->counts_cap = npix;
     }
     const uint64_t nb = (uint64_t)S->nbx * S->nby * S->nbz;
     uint8_t *d_marks = nullptr;
-    HIPCHK(hipMalloc(&d_marks, nb));
+    HIPCHK(dev_malloc(c->device, (void **)&d_marks, nb));
     std::vector<uint8_t> marks(nb);
     int rc = hipMemsetAsync(d_marks, 0, nb, c->stream) == hipSuccess ? HVR_OK : fail(HVR_EDEVICE, "memset");
     if (rc == HVR_OK) rc = enqueue_frame(c, true, nullptr, false, d_marks);
@@ -1427,7 +1539,7 @@ static BatchLaunchFn batch_fn(int fmt, int nm, int lb, bool count, int ts, bool 
 
 // Grow a device (and optionally pinned host) buffer to at least `need`
 // bytes.  Returns true when it was reallocated.
-static int grow(void **d, void **h, size_t *cap, size_t need, bool *moved)
+static int grow(int device, void **d, void **h, size_t *cap, size_t need, bool *moved)
 {
     if (need <= *cap) return HVR_OK;
     size_t n = *cap ? *cap : 4096;
@@ -1439,7 +1551,7 @@ static int grow(void **d, void **h, size_t *cap, size_t need, bool *moved)
         *h = nullptr;
     }
     *cap = 0;
-    HIPCHK(hipMalloc(d, n));
+    HIPCHK(dev_malloc(device, d, n));
     if (h) HIPCHK(hipHostMalloc(h, n, hipHostMallocDefault));
     *cap = n;
     *moved = true;
@@ -1557,7 +1669,7 @@ int hvr_batch_add(hvr_batch *b, hvr_volume *s, int srole, hvr_volume *n, int nro
     if (!b || !p) return fail(HVR_EINVAL, "null argument");
     if (!s || s->ctx != b->ctx || (n && n->ctx != b->ctx))
         return fail(HVR_EINVAL, "a batch request needs a scalar volume of the batch's context");
-    if (srole != HVR_ROLE_SCALAR || !fmt_has_scalar(s->fmt) || !s->scalar_loaded || !s->d_range)
+    if (srole != HVR_ROLE_SCALAR || !fmt_has_scalar(s->fmt) || !s->scalar_loaded)
         return fail(HVR_EINVAL, "the scalar sampler must read an uploaded scalar field");
     int nm;
     if (!n) nm = NM_ZERO;
@@ -1602,9 +1714,9 @@ int hvr_batch_reserve(hvr_batch *b, int max_requests, unsigned long long max_pix
     const size_t pixels = (size_t)max_pixels + 64 * nreq;   // each request padded to 64 pixels
     const size_t flags = nreq * align_up((size_t)max_bricks, 256);
     bool moved = false, moved_out = false;
-    if (const int rc = grow((void **)&b->d_stage, (void **)&b->h_stage, &b->stage_cap, stage, &moved)) return rc;
-    if (const int rc = grow((void **)&b->d_out, (void **)&b->h_out, &b->out_cap, pixels * 4, &moved_out)) return rc;
-    if (const int rc = grow((void **)&b->d_flags, nullptr, &b->flags_cap, flags, &moved_out)) return rc;
+    if (const int rc = grow(b->ctx->device, (void **)&b->d_stage, (void **)&b->h_stage, &b->stage_cap, stage, &moved)) return rc;
+    if (const int rc = grow(b->ctx->device, (void **)&b->d_out, (void **)&b->h_out, &b->out_cap, pixels * 4, &moved_out)) return rc;
+    if (const int rc = grow(b->ctx->device, (void **)&b->d_flags, nullptr, &b->flags_cap, flags, &moved_out)) return rc;
     if (moved_out) b->h_out_dev_of = nullptr;   // a new pinned pool may reuse the old address
     if (moved) batch_drop_graph(b);
     return HVR_OK;
@@ -1671,13 +1783,13 @@ int hvr_batch_run_async(hvr_batch *b, int count)
     const size_t nz_off = align_up(lut_off + lut_bytes, 256);
     const size_t stage_need = align_up(nz_off + nz_bytes, 256);
     bool moved = false;
-    if (const int rc = grow((void **)&b->d_stage, (void **)&b->h_stage, &b->stage_cap, stage_need, &moved)) return rc;
+    if (const int rc = grow(b->ctx->device, (void **)&b->d_stage, (void **)&b->h_stage, &b->stage_cap, stage_need, &moved)) return rc;
     bool moved_out = false;
-    if (const int rc = grow((void **)&b->d_out, (void **)&b->h_out, &b->out_cap, pixels * 4, &moved_out)) return rc;
-    if (const int rc = grow((void **)&b->d_flags, nullptr, &b->flags_cap, flag_bytes, &moved_out)) return rc;
+    if (const int rc = grow(b->ctx->device, (void **)&b->d_out, (void **)&b->h_out, &b->out_cap, pixels * 4, &moved_out)) return rc;
+    if (const int rc = grow(b->ctx->device, (void **)&b->d_flags, nullptr, &b->flags_cap, flag_bytes, &moved_out)) return rc;
     if (count) {
         size_t cb = b->counts_cap * 4;
-        if (const int rc = grow((void **)&b->d_counts, (void **)&b->h_counts, &cb, pixels * 4, &moved_out)) return rc;
+        if (const int rc = grow(b->ctx->device, (void **)&b->d_counts, (void **)&b->h_counts, &cb, pixels * 4, &moved_out)) return rc;
         b->counts_cap = cb / 4;
     }
     if (moved_out) b->h_out_dev_of = nullptr;   // a new pinned pool may reuse the old address
@@ -1877,7 +1989,6 @@ static_assert(256 + sizeof(ReqDesc) <= kNoallocFlagsOffset, "descriptor fits bef
 
 static __device__ __align__(256) unsigned char scratch[HVR_NOALLOC_SCRATCH_BYTES];
 
-static constexpr int kMaxDevices = 64;
 static std::mutex g_scratch_mu;
 static void *g_scratch_ptr[kMaxDevices];         // device address of `scratch` per device
 static hipError_t g_scratch_err[kMaxDevices];    // the lookup's result per device
@@ -1919,7 +2030,7 @@ int hvr_render_async_to_noalloc(hvr_ctx *c, void *dst)
     if (!c || !dst) return fail(HVR_EINVAL, "null argument");
     HIPCHK(hipSetDevice(c->device));
     const hvr_volume *S = c->scalar_vol, *N = c->normal_vol;
-    if (!S || c->scalar_role != HVR_ROLE_SCALAR || !fmt_has_scalar(S->fmt) || !S->scalar_loaded || !S->d_range)
+    if (!S || c->scalar_role != HVR_ROLE_SCALAR || !fmt_has_scalar(S->fmt) || !S->scalar_loaded)
         return fail(HVR_ESTATE, "hvr_render_async_to_noalloc: the scalar sampler must read an uploaded scalar field");
     int nm;
     if (!N) nm = NM_ZERO;
@@ -1996,8 +2107,8 @@ int hvr_volume_download(hvr_volume *v, float *scalar, float *normals)
     zper = std::max<uint64_t>(1, std::min<uint64_t>(zper, (uint64_t)v->s2));
     float *d_s = nullptr, *d_n = nullptr;
     int rc = HVR_OK;
-    if (scalar && hipMalloc(&d_s, zper * plane * 4) != hipSuccess) rc = fail(HVR_ENOMEM, "download staging");
-    if (rc == HVR_OK && normals && hipMalloc(&d_n, zper * plane * 12) != hipSuccess)
+    if (scalar && dev_malloc(c->device, (void **)&d_s, zper * plane * 4) != hipSuccess) rc = fail(HVR_ENOMEM, "download staging");
+    if (rc == HVR_OK && normals && dev_malloc(c->device, (void **)&d_n, zper * plane * 12) != hipSuccess)
         rc = fail(HVR_ENOMEM, "download staging");
     for (uint64_t z0 = 0; rc == HVR_OK && z0 < (uint64_t)v->s2; z0 += zper) {
         const uint64_t nz = std::min<uint64_t>(zper, (uint64_t)v->s2 - z0);

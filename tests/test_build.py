@@ -125,3 +125,71 @@ def test_a_volume_never_loaded_reads_as_zeros(hip):
         empty.destroy()
     finally:
         r.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(1024, 1023, 1), (1024, 1024, 1), (1024, 1025, 1), (1024, 1024, 3), (512, 1031, 9)])
+def test_uploads_around_the_piece_size(hip, shape):
+    """Pieces of 4 MiB go through three pinned parts in turn."""
+    rng = np.random.default_rng(shape[1])
+    c = _Context(hip, 3)
+    try:
+        v = c.volume(shape, "f32", "f32x3")
+        for _ in range(2):
+            a, n = rng.random(shape, dtype=np.float32), rng.random(shape + (3,), dtype=np.float32)
+            v.upload_scalar(a)
+            v.upload_normals(n)
+            s, m = v.download(True, True)
+            assert np.array_equal(s, a) and np.array_equal(m, n)
+        v.destroy()
+    finally:
+        c.close()
+
+
+@pytest.mark.gpu
+def test_a_block_kept_from_one_volume_serves_the_next(hip):
+    """Volumes of equal, slightly smaller and larger sizes after one another, in
+    two contexts, and one loaded in the block of a volume released while a
+    batch that reads it is in flight."""
+    from pyvr_amd.hip_renderer.batch import BatchRenderer, DeviceBlobVolume
+
+    rng = np.random.default_rng(5)
+    one, two = _Context(hip, 3), _Context(hip, 4)
+    try:
+        for edge in (64, 64, 62, 40, 90, 64):
+            for c in (one, two):
+                shape = (edge, edge + 1, edge - 3)
+                a, n = rng.random(shape, dtype=np.float32), rng.random(shape + (3,), dtype=np.float32)
+                v = c.volume(shape, "f16", "f16x3")
+                v.upload_normals(n)
+                v.upload_scalar(a)
+                s, m = v.download(True, True)
+                assert np.array_equal(s, scenes.dequant_scalar(a, "f16"))
+                assert np.array_equal(m, scenes.dequant_normals(n, "f16x3"))
+                v.destroy()
+    finally:
+        one.close()
+        two.close()
+    b = BatchRenderer(scalar_format="f16", normal_format="f16x3")
+    try:
+        vols = [DeviceBlobVolume(shape=(96, 96, 96), seed=k) for k in range(3)]
+        ctf, otf = scenes.c0(size=8, image=8).ctf, scenes.seeded_otf(5, seed=3)
+        want = []
+        for overlap in (False, True):
+            for k, vol in enumerate(vols):
+                for _ in range(4):
+                    b.add(vol, scenes.standard_camera(0.3 * k, 0.2, 3.0), ctf, otf, 640, 640)
+                slot = b.submit()
+                if not overlap:
+                    b.wait(slot)
+                b.release(vol)
+                b.upload(vols[(k + 1) % 3])
+                b.wait(slot)
+                img = [b.result(i, slot) for i in range(4)]
+                if overlap:
+                    assert img == want[k], k
+                else:
+                    want.append(img)
+        assert want[0] != want[1] != want[2]
+    finally:
+        b.close()
