@@ -114,6 +114,7 @@ struct hvr_ctx {
     int brick_log2;
     // per-launch timing region (hvr_timing_begin/end)
     std::vector<hipEvent_t> *tev;
+    std::vector<char> *tev_ordered;   // whether the frame had a pass before its march
     int timing_max, timing_n;
     // transparent-brick skipping
     int *d_nz;             // prefix counts of non-transparent LUT entries (lut_n + 1)
@@ -481,14 +482,16 @@ static int enqueue_frame(hvr_ctx *c, bool count, uchar4 *dst, bool count_shaded 
     fc.touched = touched;
     // events of this frame: the context's own, or the next slots of an
     // open timing region; hvr_last_kernel_ms reads the frame's events
+    // (each event is a packet of its own on the stream, for up to 5 us of the
+    // frame: a frame with nothing before its march has no first event)
     hipEvent_t e0 = c->ev[0], e1 = c->ev[1], e2 = c->ev[2];
-    if (c->tev && c->timing_n < c->timing_max) {
-        const size_t k = 3 * (size_t)c->timing_n++;
+    const int timed = c->tev && c->timing_n < c->timing_max ? c->timing_n++ : -1;
+    if (timed >= 0) {
+        const size_t k = 3 * (size_t)timed;
         e0 = (*c->tev)[k];
         e1 = (*c->tev)[k + 1];
         e2 = (*c->tev)[k + 2];
     }
-    HIPCHK(hipEventRecord(e0, c->stream));
     const MarchPlan plan = march_plan(c, count);
     const MarchTile bt = march_tile(plan.lanes);
     const int ntx = (c->W + (1 << bt.lbw) - 1) >> bt.lbw, nty = (c->H + (1 << bt.lbh) - 1) >> bt.lbh;
@@ -517,10 +520,12 @@ static int enqueue_frame(hvr_ctx *c, bool count, uchar4 *dst, bool count_shaded 
     c->order_used = ordered;
     if (ordered) {
         // the blocks of the head rows only (the others keep row order)
+        HIPCHK(hipEventRecord(e0, c->stream));
         hipLaunchKernelGGL(k_order_blocks, dim3(8), dim3(kOrderThreads), 0, c->stream, fc, c->d_order,
                            c->d_order + (size_t)head_rows * ntx, ntx, head_rows, cap, bt.lbw, bt.lbh);
         HIPCHK(hipGetLastError());
     }
+    if (timed >= 0) (*c->tev_ordered)[(size_t)timed] = ordered;
     // the march sets up its rays itself
     HIPCHK(hipEventRecord(e1, c->stream));
     const bool host = !dst && c->readback_mode == HVR_READBACK_DIRECT;
@@ -528,7 +533,7 @@ static int enqueue_frame(hvr_ctx *c, bool count, uchar4 *dst, bool count_shaded 
                  ordered ? c->d_order : nullptr);
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(e2, c->stream));
-    c->last_ev[0] = e0;
+    c->last_ev[0] = ordered ? e0 : e1;
     c->last_ev[1] = e1;
     c->last_ev[2] = e2;
     c->events_recorded = true;
@@ -820,6 +825,7 @@ int hvr_destroy(hvr_ctx *c)
     if (c->tev) {
         for (hipEvent_t e : *c->tev) (void)hipEventDestroy(e);
         delete c->tev;
+        delete c->tev_ordered;
     }
     if (c->stream) (void)hipStreamDestroy(c->stream);
     context_count(c->device, -1);
@@ -1277,7 +1283,11 @@ int hvr_timing_begin(hvr_ctx *c, int max_frames)
     if (!c) return fail(HVR_EINVAL, "ctx is null");
     if (max_frames <= 0 || max_frames > (1 << 16)) return fail(HVR_EINVAL, "max_frames out of range");
     HIPCHK(hipSetDevice(c->device));
-    if (!c->tev) c->tev = new std::vector<hipEvent_t>();
+    if (!c->tev) {
+        c->tev = new std::vector<hipEvent_t>();
+        c->tev_ordered = new std::vector<char>();
+    }
+    c->tev_ordered->assign((size_t)max_frames, 0);
     while (c->tev->size() < 3 * (size_t)max_frames) {
         hipEvent_t e;
         HIPCHK(hipEventCreate(&e));
@@ -1296,7 +1306,7 @@ int hvr_timing_end(hvr_ctx *c, double *march_ms, double *setup_ms, int *frames)
     double m = 0.0, s = 0.0;
     for (int i = 0; i < c->timing_n; ++i) {
         float a = 0.f, b = 0.f;
-        HIPCHK(hipEventElapsedTime(&a, (*c->tev)[3 * i], (*c->tev)[3 * i + 1]));
+        if ((*c->tev_ordered)[i]) HIPCHK(hipEventElapsedTime(&a, (*c->tev)[3 * i], (*c->tev)[3 * i + 1]));
         HIPCHK(hipEventElapsedTime(&b, (*c->tev)[3 * i + 1], (*c->tev)[3 * i + 2]));
         s += a;
         m += b;
@@ -1454,7 +1464,7 @@ int hvr_last_kernel_ms(hvr_ctx *c, float *march_ms, float *setup_ms)
     HIPCHK(hipSetDevice(c->device));
     HIPCHK(hipEventSynchronize(c->last_ev[2]));
     float a = 0.f, b = 0.f;
-    HIPCHK(hipEventElapsedTime(&a, c->last_ev[0], c->last_ev[1]));
+    if (c->last_ev[0] != c->last_ev[1]) HIPCHK(hipEventElapsedTime(&a, c->last_ev[0], c->last_ev[1]));
     HIPCHK(hipEventElapsedTime(&b, c->last_ev[1], c->last_ev[2]));
     if (setup_ms) *setup_ms = a;
     if (march_ms) *march_ms = b;
