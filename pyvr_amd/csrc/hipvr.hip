@@ -1748,6 +1748,7 @@ int hvr_batch_run_async(hvr_batch *b, int count)
         int fmt, nm, lb;
         bool buf;
         std::vector<int> members;
+        int variant, bx, by;   // kernel variant and the pixels of its block tile
     };
     std::vector<Cls> cls;
     int lut_cap = 1;
@@ -1760,7 +1761,7 @@ int hvr_batch_run_async(hvr_batch *b, int count)
             ++k;
         if (k == (int)cls.size()) {
             if (k == kBatchMaxClasses) return fail(HVR_EINVAL, "a batch mixes more than 8 volume layouts");
-            cls.push_back({r.vol->fmt, r.nm, r.vol->lb, buf, {}});
+            cls.push_back({r.vol->fmt, r.nm, r.vol->lb, buf, {}, 0, 0, 0});
         }
         cls[k].members.push_back(i);
         lut_cap = std::max(lut_cap, (int)(r.lut.size() / 4));
@@ -1775,9 +1776,21 @@ int hvr_batch_run_async(hvr_batch *b, int count)
     // sizes
     // the block tile of k_batch: 2 waves across, W / 2 down (counting runs
     // use the default variant)
-    const int variant = count ? (int)BV_DEFAULT : b->variant;
-    const int bx = b->tile_shape == HVR_TILE_16X4 ? 32 : 16;
-    const int by = (b->tile_shape == HVR_TILE_16X4 ? 4 : 8) * (batch_variant_waves(variant) / 2);
+    for (Cls &k : cls) {
+        k.variant = count ? (int)BV_DEFAULT : b->variant;
+        k.bx = b->tile_shape == HVR_TILE_16X4 ? 32 : 16;
+        k.by = (b->tile_shape == HVR_TILE_16X4 ? 4 : 8) * (batch_variant_waves(k.variant) / 2);
+        // few rays: several lanes each, as in a single frame of as many
+        long long rays = 0;
+        for (int i : k.members) rays += (long long)b->reqs[i].W * b->reqs[i].H;
+        const int lanes = march_lanes(rays, 2048ll * b->ncu, true);
+        if (lanes > 1 && !count && k.buf && k.variant == BV_DEFAULT && b->tile_shape == HVR_TILE_8X8) {
+            const MarchTile bt = march_tile(lanes);
+            k.variant = lanes == 4 ? BV_LANES4 : BV_LANES2;
+            k.bx = 1 << bt.lbw;
+            k.by = 1 << bt.lbh;
+        }
+    }
     size_t desc_off = align_up(sizeof(BatchHeader), 256);
     size_t lut_off = align_up(desc_off + (size_t)nreq * sizeof(ReqDesc), 256);
     size_t lut_bytes = 0, nz_bytes = 0, pixels = 0, flag_bytes = 0;
@@ -1865,17 +1878,17 @@ int hvr_batch_run_async(hvr_batch *b, int count)
             d.flag_end = flag_tiles;
             d.out = out_pool + b->out_off[i];
             d.counts = count ? b->d_counts + b->out_off[i] : nullptr;
-            d.ntx = (r.W + bx - 1) / bx;
-            tiles += d.ntx * ((r.H + by - 1) / by);
+            d.ntx = (r.W + cls[k].bx - 1) / cls[k].bx;
+            tiles += d.ntx * ((r.H + cls[k].by - 1) / cls[k].by);
             d.tile_end = tiles;
         }
     }
     // the graph for this shape
     std::string key = std::to_string(b->stage_cap) + "/" + std::to_string(lut_cap) + "/" +
-                      std::to_string(count) + "/" + std::to_string(b->tile_shape) + "/" + std::to_string(variant);
+                      std::to_string(count) + "/" + std::to_string(b->tile_shape);
     for (const Cls &k : cls)
         key += "/" + std::to_string(k.fmt) + "." + std::to_string(k.nm) + "." + std::to_string(k.lb) + "." +
-               std::to_string(k.buf);
+               std::to_string(k.buf) + "." + std::to_string(k.variant);
     if (key != b->key || !b->exec) {
         batch_drop_graph(b);
         HIPCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
@@ -1890,7 +1903,7 @@ int hvr_batch_run_async(hvr_batch *b, int count)
         }
         for (size_t k = 0; k < cls.size() && rc == HVR_OK; ++k) {
             const BatchLaunchFn fn =
-                batch_fn(cls[k].fmt, cls[k].nm, cls[k].lb, count != 0, b->tile_shape, cls[k].buf, variant);
+                batch_fn(cls[k].fmt, cls[k].nm, cls[k].lb, count != 0, b->tile_shape, cls[k].buf, cls[k].variant);
             rc = fn ? fn(b->d_stage, (int)k, b->d_counters + k, lut_cap, b->ncu, b->stream) : HVR_EINVAL;
         }
         hipGraph_t g = nullptr;
@@ -2048,7 +2061,9 @@ int hvr_render_async_to_noalloc(hvr_ctx *c, void *dst)
     else if (N == S && c->normal_role == HVR_ROLE_NORMAL && fmt_has_normal(S->fmt)) nm = NM_SAME;
     else return fail(HVR_ESTATE, "hvr_render_async_to_noalloc: normals must come from the scalar volume, or none");
     const bool buf = volume_buf(S) && !c->force_global;
-    const BatchLaunchFn fn = batch_fn(S->fmt, nm, S->lb, false, HVR_TILE_8X8, buf);
+    const int lanes = buf ? march_lanes((long long)c->W * c->H, resident_rays(c), true) : 1;
+    const BatchLaunchFn fn = batch_fn(S->fmt, nm, S->lb, false, HVR_TILE_8X8, buf,
+                                      lanes == 4 ? BV_LANES4 : lanes == 2 ? BV_LANES2 : BV_DEFAULT);
     if (!fn) return fail(HVR_EINVAL, "hvr_render_async_to_noalloc: brick edge must be 8 or 16 (log2 3 or 4)");
     if (c->lut_n > kLutLdsMax) return fail(HVR_EINVAL, "hvr_render_async_to_noalloc: LUT above 2048 entries");
     const uint64_t nb = (uint64_t)S->nbx * S->nby * S->nbz;
@@ -2066,8 +2081,8 @@ int hvr_render_async_to_noalloc(hvr_ctx *c, void *dst)
     hdr.all_offset = off.desc;
     hdr.cls[0].desc_offset = off.desc;
     hdr.cls[0].nreq = 1;
-    // the block tile of k_batch with 8x8 ray tiles and the default variant
-    const int bx = 16, by = 8 * (kBatchWaves / 2);
+    const MarchTile bt = march_tile(lanes);   // the block tile of k_batch
+    const int bx = 1 << bt.lbw, by = 1 << bt.lbh;
     ReqDesc d;
     memset(&d, 0, sizeof(d));
     d.fc = frame_const(c);

@@ -1714,14 +1714,17 @@ struct TileShape<1> {
 // compiler then keeps a few per-ray values in scratch outside the march
 // loop rather than run 7 waves.  16-byte texels would spill inside the
 // loop, so their kernels keep the registers they need.
+// P lanes per ray (march_lanes, by a class's rays; no gating): a wave covers
+// 8x4 or 4x4 pixels then.
 template <int SF, int NM, int LB, bool COUNT, int TS, bool BUF, int W = kBatchWaves, bool SKIP = true,
-          bool GATE = true>
+          bool GATE = true, int P = 1>
 __global__ void __launch_bounds__(64 * W, texel_bytes(SF) > 8 ? 1 : 8)
 k_batch(const char *__restrict__ block, int cls, uint32_t *__restrict__ counter)
 {
     extern __shared__ float4 s_lut[];
     __shared__ int s_item[2];
-    constexpr int WX = TileShape<TS>::WX, WY = TileShape<TS>::WY, BX = 2 * WX, BY = W / 2 * WY;
+    static_assert(P == 1 || TS == 0, "several lanes march square tiles");
+    constexpr int WX = P == 4 ? 4 : TileShape<TS>::WX, WY = P == 1 ? TileShape<TS>::WY : 4, BX = 2 * WX, BY = W / 2 * WY;
     const BatchHeader *hdr = (const BatchHeader *)block;
     const int nreq = hdr->cls[cls].nreq;
     if (nreq <= 0) return;
@@ -1760,17 +1763,18 @@ k_batch(const char *__restrict__ block, int cls, uint32_t *__restrict__ counter)
         }
         const int lt = t - (q ? reqs[q - 1].tile_end : 0);
         const int tx = lt % R.ntx, ty = lt / R.ntx;
-        const int px = tx * BX + (wv & 1) * WX + lane % WX;
-        const int py = ty * BY + (wv >> 1) * WY + lane / WX;
+        const int px = tx * BX + (wv & 1) * WX + lane / P % WX;
+        const int py = ty * BY + (wv >> 1) * WY + lane / P / WX;
         if (px < R.fc.W && py < R.fc.H) {
             const RayRec r = ray_setup(R.fc, px, py);
             float C0 = 0.f, C1 = 0.f, C2 = 0.f, A = 0.f;
             uint32_t ns = 0;
-            march_ray<SF, NM, LB, COUNT, SKIP, BUF, GATE>(R.fc, R.ts, R.ts, R.lut, R.lut_n, s_lut, r,
+            march_ray<SF, NM, LB, COUNT, SKIP, BUF, GATE && P == 1, P>(R.fc, R.ts, R.ts, R.lut, R.lut_n, s_lut, r,
                                                            R.flags, C0, C1, C2, A, ns);
             const int ln = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));   // = lane
-            const int pix = (ty * BY + (wv >> 1) * WY + ln / WX) * R.fc.W + tx * BX + (wv & 1) * WX + ln % WX;
-            st_global(R.out + pix, blend_store(R.fc, C0, C1, C2, A));
+            const int pix =
+                (ty * BY + (wv >> 1) * WY + ln / P / WX) * R.fc.W + tx * BX + (wv & 1) * WX + ln / P % WX;
+            if (P == 1 || ln % P == 0) st_global(R.out + pix, blend_store(R.fc, C0, C1, C2, A));
             if constexpr (COUNT) st_global(R.counts + pix, ns);
         }
         // every thread is done with this tile's LDS before the next fetch

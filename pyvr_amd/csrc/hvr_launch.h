@@ -33,7 +33,9 @@ enum BatchVariant : int {
     BV_WAVES8 = 2,    // 8 waves per block
     BV_NOGATE = 3,    // normals for every shaded sample
     BV_NOSKIP = 4,    // no transparent-brick skipping
-    BV_COUNT = 5
+    BV_LANES2 = 5,    // 2 or 4 lanes per ray, in BV_DEFAULT's place (batch_lanes)
+    BV_LANES4 = 6,
+    BV_COUNT = 7
 };
 constexpr int batch_variant_waves(int v) { return v == BV_WAVES2 ? 2 : v == BV_WAVES8 ? 8 : kBatchWaves; }
 

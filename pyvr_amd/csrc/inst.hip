@@ -53,16 +53,16 @@ void march_nm(const MarchArgs &a, int lb, bool count, bool skip, bool buf)
 }
 
 // ---- batched march ----
-template <int NM, int LB, bool COUNT, int TS, bool BUF, int W, bool SKIP, bool GATE>
+template <int NM, int LB, bool COUNT, int TS, bool BUF, int W, bool SKIP, bool GATE, int P = 1>
 int batch_launch(const char *blk, int cls, uint32_t *ctr, int lut_cap, int ncu, hipStream_t st)
 {
     const size_t lds = 2 * (size_t)lut_cap * sizeof(float4);
     int per = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_batch<F, NM, LB, COUNT, TS, BUF, W, SKIP, GATE>, 64 * W,
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_batch<F, NM, LB, COUNT, TS, BUF, W, SKIP, GATE, P>, 64 * W,
                                                      lds) != hipSuccess ||
         per < 1)
         per = 1;
-    hipLaunchKernelGGL((k_batch<F, NM, LB, COUNT, TS, BUF, W, SKIP, GATE>), dim3(per * ncu), dim3(64 * W), lds, st,
+    hipLaunchKernelGGL((k_batch<F, NM, LB, COUNT, TS, BUF, W, SKIP, GATE, P>), dim3(per * ncu), dim3(64 * W), lds, st,
                        blk, cls, ctr);
     return hipGetLastError() == hipSuccess ? HVR_OK : HVR_EDEVICE;
 }
@@ -79,8 +79,13 @@ BatchLaunchFn batch_variant(int v)
         case BV_WAVES8: return batch_launch<NM, LB, false, TS, BUF, 8, true, true>;
         case BV_NOGATE: return batch_launch<NM, LB, false, TS, BUF, kBatchWaves, true, false>;
         case BV_NOSKIP: return batch_launch<NM, LB, false, TS, BUF, kBatchWaves, false, true>;
-        default: return nullptr;
+        default: break;
         }
+        if constexpr (TS == 0 && BUF) {
+            if (v == BV_LANES2) return batch_launch<NM, LB, false, TS, BUF, kBatchWaves, true, true, 2>;
+            if (v == BV_LANES4) return batch_launch<NM, LB, false, TS, BUF, kBatchWaves, true, true, 4>;
+        }
+        return nullptr;
     }
 }
 

@@ -53,3 +53,27 @@ def test_lanes_give_the_same_bytes(hip, wh, sf, nf, normals, ymax, tau):
                     assert counts.max() > 30 and img.max() > 0
     finally:
         r.close()
+
+
+@pytest.mark.parametrize("lb", [3, 4])
+@pytest.mark.parametrize("sizes", [[(5, 3)], [(17, 9), (130, 67)], [(443, 443)], [(445, 443)], [(512, 512), (64, 65)],
+                                   [(1086, 1086)], [(1087, 1087)], [(300, 200)] * 20])
+def test_batches_of_few_rays_give_the_same_bytes(hip, sizes, lb):
+    """Batches are marched by lanes by the rays of a class; a counting run by one."""
+    from pyvr_amd.hip_renderer.batch import BatchRenderer, DeviceBlobVolume
+
+    b = BatchRenderer(scalar_format="f16", normal_format="f16x3", brick_log2=lb)
+    try:
+        vols = [DeviceBlobVolume(shape=s, n_blobs=6, seed=k, with_normals=k < 2)
+                for k, s in enumerate(((33, 20, 47), (64, 64, 64), (40, 50, 30)))]   # the last: a class of its own
+        ctf = scenes.c0(size=8, image=8).ctf
+        for k, (w, h) in enumerate(sizes):
+            b.add(vols[k % 3], scenes.standard_camera(0.7 + k, 0.4, 2.6), ctf, scenes.seeded_otf(5, seed=w, y_max=0.9), w, h,
+                  opacity_threshold=(0.5, 0.99, 1.5)[k % 3])
+        b.run()
+        got = [b.result(i) for i in range(len(sizes))]
+        b.run(count=True)
+        assert got == [b.result(i) for i in range(len(sizes))]
+        assert sum(int(b.counts(i).sum()) for i in range(len(sizes))) > 0
+    finally:
+        b.close()
