@@ -179,13 +179,20 @@ constexpr int march_lanes(long long rays, long long resident, bool skipping)
 }
 
 // Dispatch order of the blocks kept in rows: consecutive blocks of a class
-// (ordered_block) go to its 32 compute units in turn, so with a multiple of 16
-// blocks per row one column of the image, which is dense or empty as a whole
-// more often than not, would stay on one or two units.  Row r of a class is
-// rotated by r times this, which puts a column 13 units further from row to
-// row (512^2, 2 lanes: 232 -> 187 us, 184 -> 149; 256^2, 4 lanes: 106 -> 98).
-// Other widths spread by themselves, and rotating them gained nothing.
-constexpr int row_rotation(int ntx) { return ntx % 16 == 0 ? ((ntx - 13) & 31) % ntx : 0; }
+// (ordered_block) go to its 32 compute units in turn, so the number of blocks
+// per row, modulo 32, is how far a column of the image, which is dense or empty
+// as a whole more often than not, moves from row to row.  Where that keeps it
+// on a few units (up to 3 either way, 4 backwards, or 16), row r of a class is
+// rotated by r times this, which moves a column by 13 units a row (512^2, 2
+// lanes: 232 -> 187 us, 184 -> 149; 496^2 306 -> 248, 171 -> 147; 480^2 270 ->
+// 251; 528^2 183 -> 165; 256^2, 4 lanes: 106 -> 98).  Other widths spread by
+// themselves: rotating them gained nothing (640^2, 672^2 +1..7 %), and above
+// the resident rays the blocks that start late even things out either way.
+constexpr int row_rotation(int ntx)
+{
+    const int n = ntx & 31;
+    return ntx >= 16 && (n <= 3 || n == 16 || n >= 28) ? ((ntx - 13) & 31) % ntx : 0;
+}
 
 // Whether HVR_ORDER_AUTO orders a frame by cost: with more blocks than the
 // march keeps resident (8 of 256 threads per unit) blocks start late, and up
