@@ -406,6 +406,14 @@ static bool volume_buf(const hvr_volume *v)
     return v->bytes <= 0xffffffffull && (uint64_t)v->nbx * v->nby * v->nbz < (1ull << 24);
 }
 
+// The largest iteration bound that the frame's rays can have.
+static double ray_steps(const FrameConst &fc)
+{
+    const double diagonal = std::sqrt((double)fc.ext[0] * fc.ext[0] + (double)fc.ext[1] * fc.ext[1] +
+                                      (double)fc.ext[2] * fc.ext[2]);
+    return std::min((double)fc.max_steps, diagonal / (double)fc.step);
+}
+
 // How a frame is marched: the fast instances of the scalar volume's format
 // (nm >= 0: normals from the same texels, as (rho, 0, 0) of the same volume,
 // or unbound; brick edge 8 or 16), with transparent-brick skipping when the
@@ -416,7 +424,7 @@ struct MarchPlan {
     bool buf;
     int lanes;
 };
-static MarchPlan march_plan(hvr_ctx *c, bool count)
+static MarchPlan march_plan(hvr_ctx *c, const FrameConst &fc, bool count)
 {
     MarchPlan m = {-1, nullptr, false, 1};
     const hvr_volume *S = c->scalar_vol, *N = c->normal_vol;
@@ -427,7 +435,9 @@ static MarchPlan march_plan(hvr_ctx *c, bool count)
     if (m.nm < 0) return m;
     m.skip = brick_flags(c, S);
     m.buf = volume_buf(S) && !c->force_global;
-    if (m.buf && !count) m.lanes = march_lanes((long long)c->W * c->H, resident_rays(c), m.skip != nullptr);
+    if (m.buf && !count)
+        m.lanes = march_lanes((long long)c->W * c->H, resident_rays(c), m.skip != nullptr, ray_steps(fc),
+                              texel_bytes(S->fmt), S->bytes);
     return m;
 }
 
@@ -492,20 +502,18 @@ static int enqueue_frame(hvr_ctx *c, bool count, uchar4 *dst, bool count_shaded 
         e1 = (*c->tev)[k + 1];
         e2 = (*c->tev)[k + 2];
     }
-    const MarchPlan plan = march_plan(c, count);
+    const MarchPlan plan = march_plan(c, fc, count);
     const MarchTile bt = march_tile(plan.lanes);
     const int ntx = (c->W + (1 << bt.lbw) - 1) >> bt.lbw, nty = (c->H + (1 << bt.lbh) - 1) >> bt.lbh;
     // cost-ordered dispatch (hvr_set_dispatch_order): the blocks of the
     // first multiple-of-8 block rows are filed by k_order_blocks and marched
     // in decreasing order of their rays' iteration bounds
     const int head_rows = nty >> 3 << 3, cap = (head_rows >> 3) * ntx;
-    const double diagonal = std::sqrt((double)fc.ext[0] * fc.ext[0] + (double)fc.ext[1] * fc.ext[1] +
-                                      (double)fc.ext[2] * fc.ext[2]);
     const bool ordered =
         head_rows > 0 && (c->order_mode == HVR_ORDER_ON ||
                           (c->order_mode == HVR_ORDER_AUTO &&
                            order_auto((long long)ntx * nty, (long long)c->W * c->H, resident_rays(c), plan.lanes,
-                                      std::min((double)fc.max_steps, diagonal / (double)fc.step))));
+                                      ray_steps(fc))));
     if (ordered) {
         const size_t words = (size_t)head_rows * ntx * (1 + kOrderBuckets);
         if (words > c->order_words) {
@@ -1783,7 +1791,7 @@ int hvr_batch_run_async(hvr_batch *b, int count)
         // few rays: several lanes each, as in a single frame of as many
         long long rays = 0;
         for (int i : k.members) rays += (long long)b->reqs[i].W * b->reqs[i].H;
-        const int lanes = march_lanes(rays, 2048ll * b->ncu, true);
+        const int lanes = march_lanes(rays, 2048ll * b->ncu, true, 0.0, texel_bytes(k.fmt), 0);
         if (lanes > 1 && !count && k.buf && k.variant == BV_DEFAULT && b->tile_shape == HVR_TILE_8X8) {
             const MarchTile bt = march_tile(lanes);
             k.variant = lanes == 4 ? BV_LANES4 : BV_LANES2;
@@ -2061,7 +2069,10 @@ int hvr_render_async_to_noalloc(hvr_ctx *c, void *dst)
     else if (N == S && c->normal_role == HVR_ROLE_NORMAL && fmt_has_normal(S->fmt)) nm = NM_SAME;
     else return fail(HVR_ESTATE, "hvr_render_async_to_noalloc: normals must come from the scalar volume, or none");
     const bool buf = volume_buf(S) && !c->force_global;
-    const int lanes = buf ? march_lanes((long long)c->W * c->H, resident_rays(c), true) : 1;
+    const FrameConst fc = frame_const(c);
+    const int lanes = buf ? march_lanes((long long)c->W * c->H, resident_rays(c), true, ray_steps(fc),
+                                        texel_bytes(S->fmt), S->bytes)
+                          : 1;
     const BatchLaunchFn fn = batch_fn(S->fmt, nm, S->lb, false, HVR_TILE_8X8, buf,
                                       lanes == 4 ? BV_LANES4 : lanes == 2 ? BV_LANES2 : BV_DEFAULT);
     if (!fn) return fail(HVR_EINVAL, "hvr_render_async_to_noalloc: brick edge must be 8 or 16 (log2 3 or 4)");
@@ -2085,8 +2096,8 @@ int hvr_render_async_to_noalloc(hvr_ctx *c, void *dst)
     const int bx = 1 << bt.lbw, by = 1 << bt.lbh;
     ReqDesc d;
     memset(&d, 0, sizeof(d));
-    d.fc = frame_const(c);
-    d.ts = tex_desc(S, HVR_ROLE_SCALAR, d.fc);
+    d.fc = fc;
+    d.ts = tex_desc(S, HVR_ROLE_SCALAR, fc);
     d.lut = c->d_lut;
     d.nz = c->d_nz ? (const int *)c->d_nz : (const int *)(blk + off.unbound_nz);
     d.range = S->d_range;

@@ -171,27 +171,40 @@ constexpr int ordered_block(int b, int head, const U *cnt, const U *slots, int c
 // 480 and 366 / 331 / 409, 1280^2 601 / 635 / 720, 2048^2 1237 / 1491 / 1780.
 // Where no brick is stepped over, rays are about equally long and the device
 // stays busy to the end: 724^2 246 / 238 and 257 / 293, 1024^2 394 / 407 and
-// 446 / 487.
-constexpr int march_lanes(long long rays, long long resident, bool skipping)
+// 446 / 487.  Both lines lie further out the longer the rays are (`steps`, the
+// largest iteration bound they can have), and that of 2 lanes does where a
+// sample waits for its texels: 16-byte ones, which take the L1 several passes,
+// and volumes well above the L2s (`bytes` in all).  692 steps, FP32+FP32x3 256^3
+// / FP16+FP16x3 320^3 / UNORM8+SNORM8x3 224^3, nothing stepped over, 1 / 2 / 4
+// lanes: 480^2 675 450 351 / 514 347 257 / 361 291 268, 640^2 721 538 495 / 548
+// 389 362 / 399 376 406, 880^2 1047 787 850 / 716 551 612 / 595 626 701;
+// skipping, 2 / 4 lanes: 640^2 299 254 / 221 206 / 252 234, 720^2 326 303 /
+// 250 240 / 285 276.  346 steps: 800^2 FP32+FP32x3 256^3 409 347 / FP16+FP16x3
+// 256^3 306 276 / UNORM8+SNORM8x3 160^3 275 299 (1 / 2 lanes), 480^2 210 191 /
+// 147 134 / 152 141 (2 / 4); 100 steps: 800^2 FP32+FP32x3 211 215.  Small volumes
+// of 8-byte texels lose 6-12 % by 2 lanes above 3/4 of the resident rays.
+constexpr int march_lanes(long long rays, long long resident, bool skipping, double steps, int texel,
+                          unsigned long long bytes)
 {
-    if (8 * rays <= 3 * resident) return 4;
-    return 4 * rays <= (skipping ? 9 : 3) * resident ? 2 : 1;
+    if (8 * rays <= (steps < 512.0 ? 3 : skipping ? 7 : 4) * resident) return 4;
+    const bool waits = steps >= 256.0 && (texel >= 16 || bytes >= 128ull << 20);
+    return 4 * rays <= (skipping ? 9 : waits ? 6 : 3) * resident ? 2 : 1;
 }
 
 // Dispatch order of the blocks kept in rows: consecutive blocks of a class
 // (ordered_block) go to its 32 compute units in turn, so the number of blocks
 // per row, modulo 32, is how far a column of the image, which is dense or empty
 // as a whole more often than not, moves from row to row.  Where that keeps it
-// on a few units (up to 3 either way, 4 backwards, or 16), row r of a class is
-// rotated by r times this, which moves a column by 13 units a row (512^2, 2
-// lanes: 232 -> 187 us, 184 -> 149; 496^2 306 -> 248, 171 -> 147; 480^2 270 ->
-// 251; 528^2 183 -> 165; 256^2, 4 lanes: 106 -> 98).  Other widths spread by
-// themselves: rotating them gained nothing (640^2, 672^2 +1..7 %), and above
-// the resident rays the blocks that start late even things out either way.
+// on a few units (0 or 1, up to 4 backwards, or 16), row r of a class is rotated
+// by r times this, which moves a column by 13 units a row (512^2, 2 lanes: 232
+// -> 187 us, 184 -> 149; 496^2 306 -> 248, 171 -> 147; 480^2 270 -> 251; 528^2
+// 183 -> 165; 256^2, 4 lanes: 106 -> 98).  Other widths spread by themselves:
+// rotating them gained nothing (640^2, 672^2 +1..7 %), and above the resident
+// rays the blocks that start late even things out either way.
 constexpr int row_rotation(int ntx)
 {
     const int n = ntx & 31;
-    return ntx >= 16 && (n <= 3 || n == 16 || n >= 28) ? ((ntx - 13) & 31) % ntx : 0;
+    return ntx >= 16 && (n <= 1 || n == 16 || n >= 28) ? ((ntx - 13) & 31) % ntx : 0;
 }
 
 // Whether HVR_ORDER_AUTO orders a frame by cost: with more blocks than the
