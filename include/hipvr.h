@@ -283,7 +283,7 @@ int hvr_timing_end(hvr_ctx *ctx, double *march_ms, double *setup_ms, int *frames
  * alpha 0 (and a finite colour) contribute nothing; the march can count
  * them and step over them without loading texels.  The image and the sample
  * counts are identical in every mode.  HVR_SKIP_AUTO (the default) steps
- * over bricks when at least a quarter of the bound volume's bricks are
+ * over bricks when at least 18 % of the bound volume's bricks are
  * transparent for the current LUT.  The first frame after a LUT or volume
  * change computes the brick flags and waits for their count. */
 #define HVR_SKIP_OFF 0
