@@ -565,14 +565,24 @@ template <int F>
 static void launch_build(const hvr_volume *v, const BuildArgs &a, unsigned blocks)
 {
     const hipStream_t st = v->ctx->stream;
+    const uint64_t voxels = (uint64_t)v->s0 * v->s1 * v->s2;
+    // from a field, and more than the last cache holds of both
+    const bool once = a.field && 4 * voxels + v->bytes >= 288ull << 20;
     // voxel offsets of 32 bits where the field's floats fit 4 GiB
     const auto go = [&](auto index) {
         using I = decltype(index);
-        if (v->lb == 2) hipLaunchKernelGGL((k_build<F, 2, I>), dim3(blocks), dim3(256), 0, st, a);
-        else if (v->lb == 3) hipLaunchKernelGGL((k_build<F, 3, I>), dim3(blocks), dim3(256), 0, st, a);
-        else hipLaunchKernelGGL((k_build<F, 4, I>), dim3(blocks), dim3(256), 0, st, a);
+        const auto launch = [&](auto o) {
+            constexpr bool ONCE = decltype(o)::value;
+            if (v->lb == 2) hipLaunchKernelGGL((k_build<F, 2, I, ONCE>), dim3(blocks), dim3(256), 0, st, a);
+            else if (v->lb == 3) hipLaunchKernelGGL((k_build<F, 3, I, ONCE>), dim3(blocks), dim3(256), 0, st, a);
+            else hipLaunchKernelGGL((k_build<F, 4, I, ONCE>), dim3(blocks), dim3(256), 0, st, a);
+        };
+        if constexpr (fmt_has_normal(F)) {
+            if (once) return launch(std::true_type{});
+        }
+        launch(std::false_type{});
     };
-    if ((uint64_t)v->s0 * v->s1 * v->s2 < (1ull << 30)) go(uint32_t(0));
+    if (voxels < (1ull << 30)) go(uint32_t(0));
     else go(uint64_t(0));
 }
 static int build_layers(const hvr_volume *v, BuildArgs a, uint32_t bz0, uint32_t bz1)

@@ -1407,12 +1407,46 @@ __device__ __forceinline__ void put_normal(uint32_t *w, float nx, float ny, floa
 // spacing), the norm sqrt((gx^2 + gy^2) + gz^2) summed left to right as
 // numpy does, plus float32(1e-8), and each component divided by it -- all
 // correctly rounded float32 operations.  Every axis has at least 2 voxels.
+// Voxel l of a field; with 32-bit indices (below 2^30) its byte offset has 32
+// bits as well, beside a base the wave shares.
+template <typename I>
+__device__ __forceinline__ float field_at(const float *__restrict__ f, I l)
+{
+    return *(const float *)((const char *)f + (I)(l * 4));
+}
 template <typename I>
 __device__ __forceinline__ float np_gradient(const float *__restrict__ f, I l, int i, int n, I st)
 {
     // the voxel itself stands in for the neighbour past a face
-    const float hi = f[i == n - 1 ? l : l + st], lo = f[i == 0 ? l : l - st], d = __fsub_rn(hi, lo);
+    const float hi = field_at(f, i == n - 1 ? l : l + st), lo = field_at(f, i == 0 ? l : l - st), d = __fsub_rn(hi, lo);
     return i == 0 || i == n - 1 ? d : __fmul_rn(d, 0.5f);  // /2, exact
+}
+template <int F>
+__device__ __forceinline__ void put_gradient(uint32_t *w, float gx, float gy, float gz)
+{
+    const float nn = __fadd_rn(
+        __fsqrt_rn(__fadd_rn(__fadd_rn(__fmul_rn(gx, gx), __fmul_rn(gy, gy)), __fmul_rn(gz, gz))), 1e-8f);
+    // The three quotients by one reciprocal (Markstein, IBM J. Res. Dev. 34,
+    // 1990): refined once it is within an ulp, the first product's exact
+    // residual makes the quotient faithful and the second one's rounds it
+    // correctly, where no residual is lost below the normal numbers; zeros keep
+    // their sign by the fixup.  Other operands are divided one by one.
+    // (g << 1) - 1 orders |g|, zero last.
+    const auto key = [](float g) { return (__float_as_uint(g) << 1) - 1u; };
+    const uint32_t least = min(min(key(gx), key(gy)), key(gz));
+    if (least >= (__float_as_uint(0x1p-60f) << 1) - 1u && nn <= 0x1p60f) {
+        float y = __builtin_amdgcn_rcpf(nn);
+        y = fmaf(fmaf(-nn, y, 1.f), y, y);
+        const auto quotient = [&](float g) {
+            float q = __fmul_rn(g, y);
+            q = fmaf(fmaf(-nn, q, g), y, q);
+            q = fmaf(fmaf(-nn, q, g), y, q);
+            return __builtin_amdgcn_div_fixupf(q, nn, g);
+        };
+        put_normal<F>(w, quotient(gx), quotient(gy), quotient(gz));
+    } else {
+        put_normal<F>(w, __fdiv_rn(gx, nn), __fdiv_rn(gy, nn), __fdiv_rn(gz, nn));
+    }
 }
 
 // l / d for l below 2^32: the quotient by double multiplication is off by one at most.
@@ -1437,32 +1471,40 @@ struct BuildArgs {
     int keep;                  // the texels hold the other part, which stays
     float2 *range;             // per-brick density range, where the scalar is written
 };
-constexpr int build_bricks(int lb) { return lb == 4 ? 4 : 8; }   // bricks along x per block
+constexpr int build_bricks(int lb) { return lb == 4 ? 1 : 4; }   // bricks along x per block: V waves each
 
 // One wave per brick (all 4 of a block for 16^3 bricks, which are as many
-// times fewer), build_bricks bricks along x per block.  Every slot of a brick
-// is written once, in order, from its voxel: texel X = c + 1 of an axis holds
-// voxel c, X = 0 and X = s + 1 the edge voxels, and slots past those are 0.
+// times fewer), build_bricks bricks along x per block: one per wave, since
+// blocks of more leave most of the device idle in their last round (2,646
+// blocks of four 16^3 bricks are 1.3 rounds of 8 per unit).  Every slot of a
+// brick is written once, in order, from its voxel: texel X = c + 1 of an axis
+// holds voxel c, X = 0 and X = s + 1 the edge voxels, and slots past those are
+// 0.  In a brick clear of the volume's faces, where the numpy axes are the GL
+// ones (s0 == s2), a slot is one offset beside seven wave-wide bases.
 // Per-brick density range (for the transparent-brick flags): over all slots as
 // stored, the apron included, so that it covers every footprint the brick
 // serves; a NaN widens it to everything.  UNORM8 ranges are in decoded units
 // (raw / 255).
-// Writing the bricks bounds a scalar or normal part (FP32+FP32x3 192^3: 70 us
-// for the scalar and 126 for the normals, which read the texels too; 2.6 and
-// 3.5 TB/s), the
-// instructions of the gradient, its norm and its divisions a field.  Writing
-// whole texels in order, the range formed on the way, replaces a thread per
-// voxel that scattered it to its up to eight slots, a clearing pass and a pass
-// for the ranges: FP16+FP16x3 255x193x160 from a field 174 -> 91 us, 320^3 in
-// 16^3 bricks 709 -> 270; FP32+FP32x3 192^3 in its two parts 236 -> 196.
-template <int F, int LB, typename I>
+// Memory bounds it (FP16+FP16x3 320^3 in 16^3 bricks: 391 MB out and, each of
+// the 8 L2s fetching its bricks' surroundings, 329 MB in, at 4.5 TB/s).  ONCE
+// writes the texels past the caches, which leaves the field there; it is for
+// field and texels together above the 256 MB of the last cache (that volume 217
+// -> 160 us, FP32+FP32x3 256^3 154 -> 114, UNORM8+SNORM8x3 384^3 316 -> 224).
+// Below, it gains nothing (FP16+FP16x3 192^3 54 / 54) and a march after it takes
+// 5-8 us longer.  Writing whole texels in order, the range formed on the way,
+// replaces a thread per voxel that scattered it to its up to eight slots, a
+// clearing pass and a pass for the ranges: FP16+FP16x3 255x193x160 from a field
+// 174 -> 81 us, 320^3 in 16^3 bricks 709 -> 160; FP32+FP32x3 192^3 in its two
+// parts 236 -> 152.  A slab of the volume per XCD fetches the field once (78 MB)
+// but was no faster on the whole (320^3 144, 384^3 298 -> 327).
+template <int F, int LB, typename I, bool ONCE>
 __global__ void __launch_bounds__(256)
 k_build(const BuildArgs a)
 {
     constexpr uint32_t B = 1u << LB, E = B + 1u, N = E * E * E, T = (uint32_t)texel_bytes(F), W = (T + 3) / 4;
     constexpr uint32_t G = (uint32_t)build_bricks(LB), V = LB == 4 ? 4 : 1;   // V: waves per brick
     __shared__ float s_range[3][4];
-    const uint32_t ngx = (a.nbx + G - 1) / G, wave = threadIdx.x >> 6;
+    const uint32_t ngx = (a.nbx + G - 1) / G, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const I plane = (I)a.s0 * (I)a.s1, n12 = (I)a.s1 * (I)a.s2, first = (I)a.first;
     for (uint64_t run = blockIdx.x; run < a.runs; run += gridDim.x)
@@ -1474,7 +1516,47 @@ k_build(const BuildArgs a)
         char *out = a.dst + brick * ((uint64_t)N * T);
         float lo = INFINITY, hi = -INFINITY;
         bool nan = false;
-        for (uint32_t k = wave % V * 64 + lane; k < N; k += 64 * V) {
+        const bool inside = fmt_has_normal(F) && a.field && a.s0 == a.s2 && bx && by && bz &&
+                            (bx + 1) * B < (uint32_t)a.s0 && (by + 1) * B < (uint32_t)a.s1 &&
+                            (bz + 1) * B < (uint32_t)a.s2;
+        const auto put = [&](uint32_t k, const uint32_t *w) {
+            char *p = out + k * T;
+            if constexpr (T == 1) *(uint8_t *)p = (uint8_t)w[0];
+            else if constexpr (T == 2) *(uint16_t *)p = (uint16_t)w[0];
+            else if constexpr (ONCE) {
+#pragma unroll
+                for (uint32_t q = 0; q < W; ++q) __builtin_nontemporal_store(w[q], (uint32_t *)p + q);
+            } else {
+#pragma unroll
+                for (uint32_t q = 0; q < W; ++q) ((uint32_t *)p)[q] = w[q];
+            }
+            if constexpr (fmt_has_scalar(F)) {
+                float v;
+                if constexpr (F == TF_S_F16) v = h16f(w[0]);
+                else if constexpr (F == TF_S_U8) v = (float)w[0];
+                else if constexpr (F == TF_S_F32) v = __uint_as_float(w[0]);
+                else v = decode_scalar<F>(w);
+                if constexpr (fmt_u8_scalar(F)) v *= 1.0f / 255.0f;
+                nan |= v != v;
+                lo = fminf(lo, v);
+                hi = fmaxf(hi, v);
+            }
+        };
+        const uint32_t k0 = wave % V * 64 + lane;
+        if (fmt_has_normal(F) && inside) {
+            // the voxel of slot 0, and from it those of the others
+            const float *f0 = a.field + ((I)(bz * B - 1) * plane + (I)(by * B - 1) * (I)a.s0 + (I)(bx * B - 1));
+            for (uint32_t k = k0; k < N; k += 64 * V) {
+                const I r = (I)(k / (E * E)) * plane + (I)(k / E % E * (uint32_t)a.s0) + (I)(k % E);
+                const auto slope = [&](I st) {
+                    return __fmul_rn(__fsub_rn(field_at(f0 + st, r), field_at(f0 - st, r)), 0.5f);
+                };
+                uint32_t w[W] = {};
+                put_scalar<F>(w, field_at(f0, r));
+                put_gradient<F>(w, slope(n12), slope((I)a.s2), slope((I)1));
+                put(k, w);
+            }
+        } else for (uint32_t k = k0; k < N; k += 64 * V) {
             const uint32_t X = bx * B + k % E, Y = by * B + k / E % E, Z = bz * B + k / (E * E);
             uint32_t w[W] = {};
             if (X <= (uint32_t)a.s0 + 1u && Y <= (uint32_t)a.s1 + 1u && Z <= (uint32_t)a.s2 + 1u) {
@@ -1490,7 +1572,7 @@ k_build(const BuildArgs a)
                 } else if (a.scalar) {
                     put_scalar<F>(w, a.scalar[l - first]);
                 } else {
-                    put_scalar<F>(w, a.field[l]);
+                    put_scalar<F>(w, field_at(a.field, l));
                     if constexpr (fmt_has_normal(F)) {
                         // numpy coordinates of flat index l
                         int i0 = z, i1 = y, i2 = x;
@@ -1510,31 +1592,11 @@ k_build(const BuildArgs a)
                         const float gx = np_gradient(a.field, l, i0, a.s0, n12);
                         const float gy = np_gradient(a.field, l, i1, a.s1, (I)a.s2);
                         const float gz = np_gradient(a.field, l, i2, a.s2, (I)1);
-                        const float nn = __fadd_rn(
-                            __fsqrt_rn(__fadd_rn(__fadd_rn(__fmul_rn(gx, gx), __fmul_rn(gy, gy)), __fmul_rn(gz, gz))),
-                            1e-8f);
-                        put_normal<F>(w, __fdiv_rn(gx, nn), __fdiv_rn(gy, nn), __fdiv_rn(gz, nn));
+                        put_gradient<F>(w, gx, gy, gz);
                     }
                 }
             }
-            char *p = out + k * T;
-            if constexpr (T == 1) *(uint8_t *)p = (uint8_t)w[0];
-            else if constexpr (T == 2) *(uint16_t *)p = (uint16_t)w[0];
-            else {
-#pragma unroll
-                for (uint32_t q = 0; q < W; ++q) ((uint32_t *)p)[q] = w[q];
-            }
-            if constexpr (fmt_has_scalar(F)) {
-                float v;
-                if constexpr (F == TF_S_F16) v = h16f(w[0]);
-                else if constexpr (F == TF_S_U8) v = (float)w[0];
-                else if constexpr (F == TF_S_F32) v = __uint_as_float(w[0]);
-                else v = decode_scalar<F>(w);
-                if constexpr (fmt_u8_scalar(F)) v *= 1.0f / 255.0f;
-                nan |= v != v;
-                lo = fminf(lo, v);
-                hi = fmaxf(hi, v);
-            }
+            put(k, w);
         }
         if (fmt_has_scalar(F) && a.range) {
             for (int off = 32; off > 0; off >>= 1) {
