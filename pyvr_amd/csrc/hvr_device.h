@@ -1,6 +1,7 @@
 // hvr_device.h -- device code of libhipvr: texel formats, GL-style sampling,
-// the ray-setup kernel, the march-and-composite kernel and the upload kernel
-// (gfx950, wave64).
+// ray setup and cost ordering, the march-and-composite kernels, the kernels that
+// build volumes and their transparency flags, and the batch kernels (gfx950,
+// wave64).
 //
 // Semantics follow the reference fragment shader pyvr/shaders/volume.frag.glsl
 // and the GL state of pyvr/moderngl_renderer/manager.py (paths relative to the
@@ -1401,12 +1402,12 @@ __device__ __forceinline__ void put_normal(uint32_t *w, float nx, float ny, floa
 }
 
 // Normals of a device float32 field (numpy C order, shape (s0, s1, s2)),
-// exactly as compute_normal_volume (pyvr/datasets/synthetic.py:109-122)
-// computes them from a float32 array: np.gradient along each numpy axis
+// as compute_normal_volume (pyvr/datasets/synthetic.py:109-122) computes them from a float32 array: np.gradient along each numpy axis
 // (central differences halved inside, one-sided at the two faces, unit
 // spacing), the norm sqrt((gx^2 + gy^2) + gz^2) summed left to right as
-// numpy does, plus float32(1e-8), and each component divided by it -- all
-// correctly rounded float32 operations.  Every axis has at least 2 voxels.
+// numpy does, plus float32(1e-8), and each component divided by it, in float32:
+// sums, products and quotients correctly rounded, the square root within an
+// ulp.  Every axis has at least 2 voxels.
 // Voxel l of a field; with 32-bit indices (below 2^30) its byte offset has 32
 // bits as well, beside a base the wave shares.
 template <typename I>

@@ -119,12 +119,12 @@ constexpr void lut_prefix_counts(const float *src, int cnt, int *nz)
     }
 }
 
-// Cost-ordered dispatch of a frame's 16x16 ray blocks.  A frame ends when
+// Cost-ordered dispatch of a frame's ray blocks.  A frame ends when
 // its longest waves do; dispatched in row order, long blocks that start
 // late (after the first round of resident blocks) set the frame's end.
-// Ray setup gives each block a cost key, the largest iteration bound of its
-// rays, and files the block under a key bucket; the march then takes the
-// blocks of the largest keys first.  Buckets split [0, max_steps] evenly,
+// k_order_blocks gives each block a cost key, the largest iteration bound of
+// three of its rays, and files the block under a key bucket; the march then
+// takes the blocks of the largest keys first.  Buckets split [0, max_steps] evenly,
 // bucket 0 holding the largest keys.
 constexpr int kOrderBuckets = 16;
 constexpr int order_bucket(int key, int max_steps)

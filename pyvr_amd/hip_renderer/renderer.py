@@ -76,9 +76,9 @@ class HipVolumeRenderer:
         Raises ``TypeError`` if ``volume`` is not a ``Volume``.  Without
         normals the normal sampler keeps its previous unit (by default unit
         0), as in the reference.  ``device_normals=True`` on a volume without
-        normals computes them on the GPU instead -- the same bytes as
-        ``volume.compute_normals()`` followed by ``load_volume``, without the
-        host gradient."""
+        normals computes them on the GPU instead -- the normals of
+        ``volume.compute_normals()`` (within an ulp, before they are stored)
+        followed by ``load_volume``, without the host gradient."""
         if not isinstance(volume, Volume):
             raise TypeError(
                 f"Expected Volume instance, got {type(volume)}. "
