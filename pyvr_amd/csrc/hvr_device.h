@@ -853,12 +853,15 @@ __device__ __forceinline__ bool group_any(int v)
 template <int P, int K>
 __device__ __forceinline__ void add_color(float tl, float q0, float q1, float q2, float &C0, float &C1, float &C2)
 {
-    // s_nop: a lane's q may have been written by the instruction before
+    // s_nop: a lane's q may have been written by the instruction before.  & : the
+    // first colours are written while q1, q2 and tl are still to be read, so none
+    // of those may share an accumulator's register, also where both hold the same
+    // value.
 #define HVR_FMAC3(QP)                                                           \
     asm volatile("s_nop 1\n\tv_fmac_f32_dpp %0, %3, %6 " QP " row_mask:0xf bank_mask:0xf\n\t" \
         "v_fmac_f32_dpp %1, %4, %6 " QP " row_mask:0xf bank_mask:0xf\n\t"               \
         "v_fmac_f32_dpp %2, %5, %6 " QP " row_mask:0xf bank_mask:0xf"                   \
-        : "+v"(C0), "+v"(C1), "+v"(C2)                                              \
+        : "+&v"(C0), "+&v"(C1), "+&v"(C2)                                           \
         : "v"(q0), "v"(q1), "v"(q2), "v"(tl))
     if constexpr (P == 2 && K == 0) HVR_FMAC3("quad_perm:[0,0,2,2]");
     else if constexpr (P == 2) HVR_FMAC3("quad_perm:[1,1,3,3]");
