@@ -1430,22 +1430,16 @@ __device__ __forceinline__ void put_gradient(uint32_t *w, float gx, float gy, fl
 {
     const float nn = __fadd_rn(
         __fsqrt_rn(__fadd_rn(__fadd_rn(__fmul_rn(gx, gx), __fmul_rn(gy, gy)), __fmul_rn(gz, gz))), 1e-8f);
-    // The three quotients by one reciprocal (Markstein, IBM J. Res. Dev. 34,
-    // 1990): refined once it is within an ulp, the first product's exact
-    // residual makes the quotient faithful and the second one's rounds it
-    // correctly, where no residual is lost below the normal numbers; zeros keep
-    // their sign by the fixup.  Other operands are divided one by one.
+    // The three quotients by one reciprocal (reciprocal_quotient), between
+    // bounds that keep the residuals normal; v_rcp_f32 is within an ulp, and zeros
+    // keep their sign by the fixup.  Other operands are divided one by one.
     // (g << 1) - 1 orders |g|, zero last.
     const auto key = [](float g) { return (__float_as_uint(g) << 1) - 1u; };
     const uint32_t least = min(min(key(gx), key(gy)), key(gz));
-    if (least >= (__float_as_uint(0x1p-60f) << 1) - 1u && nn <= 0x1p60f) {
-        float y = __builtin_amdgcn_rcpf(nn);
-        y = fmaf(fmaf(-nn, y, 1.f), y, y);
+    if (least >= (__float_as_uint(0x1p-60f) << 1) - 1u && nn <= 0x1p60f && reciprocal_divides(__float_as_uint(nn))) {
+        const float y = refine_reciprocal(nn, __builtin_amdgcn_rcpf(nn));
         const auto quotient = [&](float g) {
-            float q = __fmul_rn(g, y);
-            q = fmaf(fmaf(-nn, q, g), y, q);
-            q = fmaf(fmaf(-nn, q, g), y, q);
-            return __builtin_amdgcn_div_fixupf(q, nn, g);
+            return __builtin_amdgcn_div_fixupf(reciprocal_quotient(g, nn, y), nn, g);
         };
         put_normal<F>(w, quotient(gx), quotient(gy), quotient(gz));
     } else {

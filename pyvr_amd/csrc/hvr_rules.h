@@ -219,6 +219,26 @@ constexpr bool order_auto(long long blocks, long long rays, long long resident, 
     return blocks * 256 > resident && 4 * rays <= 9 * resident && steps >= 256.0 * lanes;
 }
 
+// Correctly rounded quotients g / d of several g by one reciprocal (Markstein,
+// IBM J. Res. Dev. 34, 1990): an approximation within an ulp of 1 / d, refined
+// once, is 1 / d correctly rounded unless the mantissa of d is all ones (its
+// reciprocal lies next to the middle of two floats); with it the first
+// product's exact residual makes the quotient faithful and the second one's
+// rounds it, as long as no residual is lost below the normal numbers.
+constexpr bool reciprocal_divides(uint32_t d_bits) { return (d_bits & 0x7fffffu) != 0x7fffffu; }
+template <typename F>   // F: float (clang takes no constexpr function of __builtin_fmaf that is no template)
+constexpr F refine_reciprocal(F d, F y)
+{
+    return __builtin_fmaf(__builtin_fmaf(-d, y, 1.f), y, y);
+}
+template <typename F>
+constexpr F reciprocal_quotient(F g, F d, F y)
+{
+    F q = g * y;
+    q = __builtin_fmaf(__builtin_fmaf(-d, q, g), y, q);
+    return __builtin_fmaf(__builtin_fmaf(-d, q, g), y, q);
+}
+
 // Inverse of a 4x4 matrix (row-major, m[4*r + c]) by Gauss-Jordan
 // elimination with partial pivoting.  Returns false when singular.
 constexpr bool inverse4(const double *m, double *inv)
