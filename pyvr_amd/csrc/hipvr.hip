@@ -4,6 +4,7 @@
 // preparation and kernel dispatch.
 #include "hvr_copy.h"
 #include "hvr_launch.h"
+#include "hvr_share.h"
 #include "../../include/hipvr.h"
 
 #include <math.h>
@@ -1507,20 +1508,8 @@ struct BatchReq {
     hvr_params params;
     int W, H;
     std::vector<float> lut;  // n x RGBA
-    uint64_t lut_hash;       // of its bytes
+    uint64_t lut_hash;       // float_hash
 };
-
-// FNV-1a over the LUT's 32-bit words: requests with other hashes hold other LUTs.
-static uint64_t lut_hash(const std::vector<float> &lut)
-{
-    uint64_t h = 0xcbf29ce484222325ull;
-    for (float f : lut) {
-        uint32_t w;
-        memcpy(&w, &f, 4);
-        h = (h ^ w) * 0x100000001b3ull;
-    }
-    return h;
-}
 
 struct hvr_batch {
     hvr_ctx *ctx;
@@ -1724,7 +1713,7 @@ int hvr_batch_add(hvr_batch *b, hvr_volume *s, int srole, hvr_volume *n, int nro
     r.H = height;
     if (lut_n > 0) r.lut.assign(lut_rgba, lut_rgba + 4 * (size_t)lut_n);
     else r.lut = {0.f, 0.f, 0.f, 1.f};  // unbound LUT texture
-    r.lut_hash = lut_hash(r.lut);
+    r.lut_hash = float_hash(r.lut.data(), r.lut.size());
     b->reqs.push_back(std::move(r));
     b->ran = b->counted = false;
     if (index) *index = (int)b->reqs.size() - 1;
@@ -1859,7 +1848,9 @@ int hvr_batch_run_async(hvr_batch *b, int count)
     size_t lut_at = lut_off, nz_at = nz_off, flag_at = 0;
     int slot = 0;
     uint32_t flag_tiles = 0;
-    std::vector<std::pair<int, int>> firsts;   // (request, descriptor) of each volume and LUT met first
+    // views of one volume through one LUT share its staged copy and flags
+    ShareTable firsts((size_t)nreq);
+    std::vector<int> request((size_t)nreq);   // of each descriptor
     for (size_t k = 0; k < cls.size(); ++k) {
         hdr->cls[k].desc_offset = (uint32_t)(desc_off + (size_t)slot * sizeof(ReqDesc));
         hdr->cls[k].nreq = (int)cls[k].members.size();
@@ -1871,23 +1862,21 @@ int hvr_batch_run_async(hvr_batch *b, int count)
             d.fc = frame_const_of(r.params, true, r.W, r.H);
             d.ts = tex_desc(r.vol, HVR_ROLE_SCALAR, d.fc);
             const int n = (int)(r.lut.size() / 4);
-            // views of one volume through one LUT share its staged copy and flags
-            const ReqDesc *same = nullptr;
-            for (const auto &f : firsts) {
-                const BatchReq &o = b->reqs[f.first];
-                if (o.vol == r.vol && o.lut_hash == r.lut_hash && o.lut.size() == r.lut.size() &&
-                    memcmp(o.lut.data(), r.lut.data(), r.lut.size() * sizeof(float)) == 0)
-                    same = descs + f.second;
-            }
+            request[slot - 1] = i;
+            const int first = firsts.find_or_add(
+                r.lut_hash ^ (uint64_t)(uintptr_t)r.vol * 0x9e3779b97f4a7c15ull, slot - 1, [&](int other) {
+                    const BatchReq &o = b->reqs[request[other]];
+                    return o.vol == r.vol && o.lut.size() == r.lut.size() &&
+                           memcmp(o.lut.data(), r.lut.data(), r.lut.size() * sizeof(float)) == 0;
+                });
             d.lut_n = n;
             d.range = r.vol->d_range;
             d.nbz = r.vol->nbz;
-            if (same) {
-                d.lut = same->lut;
-                d.nz = same->nz;
-                d.flags = same->flags;
+            if (first >= 0) {
+                d.lut = descs[first].lut;
+                d.nz = descs[first].nz;
+                d.flags = descs[first].flags;
             } else {
-                firsts.push_back({i, slot - 1});
                 memcpy(b->h_stage + lut_at, r.lut.data(), r.lut.size() * sizeof(float));
                 lut_prefix_counts(r.lut.data(), n, (int *)(b->h_stage + nz_at));
                 d.lut = (const float4 *)(b->d_stage + lut_at);
