@@ -101,7 +101,8 @@ int hvr_abi_version(void);
  * hvr_volume_upload_scalar_normals, hvr_volume_generate_blobs, hvr_set_lut,
  * hvr_set_params, hvr_bind, hvr_render_async, hvr_render_async_to,
  * hvr_read, hvr_sample_counts, hvr_batch_create, hvr_batch_add,
- * hvr_batch_run_async, hvr_batch_wait, hvr_batch_query. */
+ * hvr_batch_run_async, hvr_batch_wait, hvr_batch_query.  Inside the uploads,
+ * "hvr_upload_ring" fails a copy that takes the library's own pinned memory. */
 int hvr_debug_inject_fault(const char *function, int code, int after);
 
 /* Message of the last failed call on this thread ("" if none). */

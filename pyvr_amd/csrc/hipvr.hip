@@ -638,16 +638,31 @@ static int need_stage(hvr_ctx *c, size_t need)
 }
 static constexpr size_t kMaxStage = (size_t)256 << 20;   // what stays allocated, but for larger single planes
 
+// Whether `src` is plain host memory, which the device cannot read by itself:
+// not pinned, registered, managed or its own.
+static bool pageable(const void *src)
+{
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, src) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return at.type == hipMemoryTypeUnregistered;
+}
+
 // Host data to the device, in stream order.  From pageable memory one thread of
 // the runtime copies into pinned memory, at 30 GB/s; here four threads do
 // (CopyPool), piece by piece through a ring of three pinned parts, while the
-// pieces before cross the link at its 57 GB/s.  The caller's data is read when
-// this returns.  Less than a piece, and where the ring cannot be had, goes
-// the runtime's way.
+// pieces before cross the link (44 GB/s).  The caller's pageable data is read
+// when this returns.  What the device can read by itself it copies by itself
+// (pinned data at the link's 53 GB/s; 85 MB 1.62 ms, through the ring 1.94);
+// less than a piece, and where the ring cannot be had, goes the runtime's way.
 static constexpr size_t kUploadPiece = (size_t)4 << 20;
 static int upload_host(hvr_ctx *c, void *dst, const void *src, size_t bytes)
 {
-    if (bytes >= kUploadPiece && !c->h_up) {
+    const bool ring = bytes >= kUploadPiece && pageable(src);
+    if (ring) HVR_FAULT_POINT("hvr_upload_ring");
+    if (ring && !c->h_up) {
         bool ok = hipHostMalloc((void **)&c->h_up, 3 * kUploadPiece, hipHostMallocDefault) == hipSuccess;
         for (hipEvent_t &e : c->up_ev)
             if (ok && !e) ok = hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
@@ -657,7 +672,7 @@ static int upload_host(hvr_ctx *c, void *dst, const void *src, size_t bytes)
             c->h_up = nullptr;
         }
     }
-    if (bytes < kUploadPiece || !c->h_up) {
+    if (!ring || !c->h_up) {
         HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
         return HVR_OK;
     }
