@@ -120,7 +120,9 @@ int hvr_device_memory(int device, unsigned long long *free_bytes, unsigned long 
  * The march reads volumes below 4 GiB through buffer loads (32-bit
  * offsets); with the environment variable HVR_GATHER=global set when the
  * context is created it uses 64-bit global loads, as for larger volumes
- * (same results; for testing that path). */
+ * (same results; for testing that path).  HVR_STAGE=<bytes>, likewise, bounds
+ * the device memory a field uploaded from the host passes through, below its
+ * 256 MiB (fields larger than that arrive in groups of bricks). */
 int hvr_create(int device, int width, int height, hvr_ctx **out);
 int hvr_destroy(hvr_ctx *ctx);
 /* Change the framebuffer size (no counterpart in the reference, whose

@@ -101,7 +101,7 @@ struct hvr_ctx {
     int readback_mode;    // HVR_READBACK_COPY / _DIRECT
     bool last_host;       // the last frame was written to h_pinned
     float *d_stage;  // upload staging
-    size_t stage_bytes;
+    size_t stage_bytes, max_stage;   // what it holds, and may hold while an upload of parts fits it
     char *h_up;           // pinned ring the uploads go through (upload_host), or nullptr
     hipEvent_t up_ev[3];  // after the last copy out of each of its parts
     hipEvent_t ev[4];
@@ -561,7 +561,8 @@ static void noalloc_setup(int device);
 
 // ---------------------------------------------------------------------------
 // C ABI
-// Build brick layers [bz0, bz1) of volume v (k_build) from the source in `a`.
+// Build brick rows [by0, by1) of brick layers [bz0, bz1) of volume v (k_build)
+// from the source in `a`, whose planes lie `a.plane` voxels apart.
 template <int F>
 static void launch_build(const hvr_volume *v, const BuildArgs &a, unsigned blocks)
 {
@@ -586,7 +587,7 @@ static void launch_build(const hvr_volume *v, const BuildArgs &a, unsigned block
     if (voxels < (1ull << 30)) go(uint32_t(0));
     else go(uint64_t(0));
 }
-static int build_layers(const hvr_volume *v, BuildArgs a, uint32_t bz0, uint32_t bz1)
+static int build_group(const hvr_volume *v, BuildArgs a, uint32_t by0, uint32_t by1, uint32_t bz0, uint32_t bz1)
 {
     a.dst = (char *)v->d_texels;
     a.s0 = v->s0;
@@ -596,8 +597,10 @@ static int build_layers(const hvr_volume *v, BuildArgs a, uint32_t bz0, uint32_t
     a.nby = v->nby;
     a.inv_n12 = 1.0 / ((double)v->s1 * v->s2);
     a.inv_s2 = 1.0 / v->s2;
+    a.by0 = by0;
+    a.rows = by1 - by0;
     a.bz0 = bz0;
-    a.runs = (uint64_t)((v->nbx + build_bricks(v->lb) - 1) / build_bricks(v->lb)) * v->nby * (bz1 - bz0);
+    a.runs = (uint64_t)((v->nbx + build_bricks(v->lb) - 1) / build_bricks(v->lb)) * a.rows * (bz1 - bz0);
     const unsigned blocks = (unsigned)std::min<uint64_t>(a.runs, (1u << 24) - 1);   // below 2^32 threads
     switch (v->fmt) {
 #define HVR_BUILD(F) \
@@ -636,7 +639,7 @@ static int need_stage(hvr_ctx *c, size_t need)
     c->stage_bytes = need;
     return HVR_OK;
 }
-static constexpr size_t kMaxStage = (size_t)256 << 20;   // what stays allocated, but for larger single planes
+static constexpr size_t kMaxStage = (size_t)256 << 20;   // what stays allocated
 
 // Whether `src` is plain host memory, which the device cannot read by itself:
 // not pinned, registered, managed or its own.
@@ -776,6 +779,9 @@ int hvr_create(int device, int width, int height, hvr_ctx **out)
     c->readback_mode = HVR_READBACK_DIRECT;
     const char *gather = getenv("HVR_GATHER");
     c->force_global = gather && strcmp(gather, "global") == 0;
+    c->max_stage = kMaxStage;
+    if (const char *stage = getenv("HVR_STAGE"))
+        if (const unsigned long long n = strtoull(stage, nullptr, 10)) c->max_stage = (size_t)std::min<uint64_t>(n, kMaxStage);
     const size_t npix = (size_t)width * height;
     noalloc_setup(device);
     hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
@@ -999,35 +1005,40 @@ int hvr_volume_create(hvr_ctx *c, int s0, int s1, int s2, int sf, int nf, hvr_vo
 }
 
 // The scalar (part 1) or normal (part 2) field of volume v from host data, in
-// groups of brick layers whose source planes (with the one plane of the
-// neighbours on both sides) fit the staging buffer of up to 256 MiB.
+// groups of bricks whose source fits the staging buffer (upload_group).
 static int upload_part(hvr_volume *v, const float *data, int part)
 {
     hvr_ctx *c = v->ctx;
     HIPCHK(hipSetDevice(c->device));
-    const int comps = part == 1 ? 1 : 3;
-    const int B = 1 << v->lb;
-    const uint64_t plane = (uint64_t)v->s0 * v->s1;
-    const size_t row = (size_t)(plane * comps * sizeof(float));
-    const uint64_t fit = kMaxStage / row;   // planes
-    const uint32_t group = fit > (uint64_t)B + 2 ? (uint32_t)((fit - 2) / B) : 1;   // layers
-    if (const int rc = need_stage(c, (size_t)std::min<uint64_t>((uint64_t)group * B + 2, (uint64_t)v->s2) * row)) return rc;
+    const uint64_t comps = part == 1 ? 1 : 3, plane = (uint64_t)v->s0 * v->s1;
+    const size_t row = (size_t)(v->s0 * comps * sizeof(float));
+    const UploadGroup g = upload_group(row, v->s1, v->s2, v->lb, c->max_stage);
+    FieldBuffer f(c);
+    if (const int rc = f.get((size_t)g.bytes)) return rc;
     BuildArgs a;
     memset(&a, 0, sizeof(a));
-    (part == 1 ? a.scalar : a.normal) = c->d_stage;
+    (part == 1 ? a.scalar : a.normal) = (const float *)f.p;
     a.keep = part == 1 ? v->normals_loaded : v->scalar_loaded;
     a.range = part == 1 ? v->d_range : nullptr;
-    for (uint32_t bz = 0; bz < v->nbz; bz += group) {
-        // voxel planes of layers [bz, end): texel Z holds voxel Z - 1
-        const uint32_t end = std::min(v->nbz, bz + group);
-        const int64_t z0 = std::min<int64_t>(std::max<int64_t>((int64_t)bz * B - 1, 0), v->s2 - 1),
-                      z1 = std::min<int64_t>((int64_t)end * B, v->s2);   // one past the last
-        a.first = (uint64_t)z0 * plane;
-        if (const int rc = upload_host(c, c->d_stage, data + a.first * comps, (size_t)(z1 - z0) * row)) return rc;
-        if (const int rc = build_layers(v, a, bz, end)) return rc;
-        // the staging buffer is reused by the next group
-        HIPCHK(hipStreamSynchronize(c->stream));
-    }
+    for (uint32_t bz = 0; bz < v->nbz; bz += g.layers)
+        for (uint32_t by = 0; by < v->nby; by += g.rows) {
+            const int z0 = source_begin(bz, v->lb, v->s2), z1 = source_end(bz, g.layers, v->lb, v->s2),
+                      y0 = source_begin(by, v->lb, v->s1), y1 = source_end(by, g.rows, v->lb, v->s1);
+            const uint64_t lines = (uint64_t)(y1 - y0);
+            a.plane = lines * v->s0;
+            a.first = (uint64_t)z0 * a.plane + (uint64_t)y0 * v->s0;
+            const auto at = [&](int z) { return data + ((uint64_t)z * plane + (uint64_t)y0 * v->s0) * comps; };
+            if (lines == (uint64_t)v->s1) {
+                if (const int rc = upload_host(c, f.p, at(z0), (size_t)(z1 - z0) * lines * row)) return rc;
+            } else {
+                for (int z = z0; z < z1; ++z)
+                    if (const int rc = upload_host(c, f.p + (size_t)(z - z0) * lines * row, at(z), lines * row)) return rc;
+            }
+            if (const int rc = build_group(v, a, by, std::min(v->nby, by + g.rows), bz, std::min(v->nbz, bz + g.layers)))
+                return rc;
+            // the staging buffer is reused by the next group
+            HIPCHK(hipStreamSynchronize(c->stream));
+        }
     return HVR_OK;
 }
 
@@ -1043,7 +1054,8 @@ static int volume_from_field(hvr_volume *v, const float *d_field, bool normals)
     (normals ? a.field : a.scalar) = d_field;
     a.keep = !normals && v->normals_loaded;
     a.range = v->d_range;
-    if (const int rc = build_layers(v, a, 0, v->nbz)) return rc;
+    a.plane = (uint64_t)v->s0 * v->s1;
+    if (const int rc = build_group(v, a, 0, v->nby, 0, v->nbz)) return rc;
     HIPCHK(hipStreamSynchronize(c->stream));
     v->scalar_loaded = true;
     if (normals) v->normals_loaded = true;

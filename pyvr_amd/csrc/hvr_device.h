@@ -1459,12 +1459,14 @@ __device__ __forceinline__ uint32_t div_u32(uint32_t l, uint32_t d, double inv)
 struct BuildArgs {
     char *dst;
     int s0, s1, s2;            // GL size
-    uint32_t nbx, nby, bz0;    // bricks; the launch's first brick layer
+    uint32_t nbx, nby;         // bricks
+    uint32_t by0, rows, bz0;   // the launch's first brick row, its rows, its first brick layer
     uint64_t runs;             // groups of build_bricks bricks along x in the launch
     const float *scalar;       // the source, of one kind
     const float *normal;
     const float *field;
-    uint64_t first;            // flat index of the source's first voxel
+    uint64_t plane;            // voxels between the source's planes
+    uint64_t first;            // index of the source's first voxel, counted in such planes
     double inv_n12, inv_s2;    // 1 / (s1 s2), 1 / s2
     int keep;                  // the texels hold the other part, which stays
     float2 *range;             // per-brick density range, where the scalar is written
@@ -1504,11 +1506,11 @@ k_build(const BuildArgs a)
     __shared__ float s_range[3][4];
     const uint32_t ngx = (a.nbx + G - 1) / G, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    const I plane = (I)a.s0 * (I)a.s1, n12 = (I)a.s1 * (I)a.s2, first = (I)a.first;
+    const I plane = (I)a.plane, n12 = (I)a.s1 * (I)a.s2, first = (I)a.first;
     for (uint64_t run = blockIdx.x; run < a.runs; run += gridDim.x)
     for (uint32_t j = wave / V; j < G; j += 4 / V) {
-        const uint32_t bx = (uint32_t)(run % ngx) * G + j, by = (uint32_t)(run / ngx % a.nby),
-                       bz = a.bz0 + (uint32_t)(run / ngx / a.nby);
+        const uint32_t bx = (uint32_t)(run % ngx) * G + j, by = a.by0 + (uint32_t)(run / ngx % a.rows),
+                       bz = a.bz0 + (uint32_t)(run / ngx / a.rows);
         if (bx >= a.nbx) break;
         const uint64_t brick = ((uint64_t)bz * a.nby + by) * a.nbx + bx;
         char *out = a.dst + brick * ((uint64_t)N * T);

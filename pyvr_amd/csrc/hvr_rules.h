@@ -53,6 +53,51 @@ constexpr int slot_voxel(uint32_t X, int s)
     return c < 0 ? 0 : c < s ? c : s - 1;
 }
 
+// The bricks that one group of an upload builds: `layers` brick layers of
+// `rows` brick rows each, whose source -- the planes and rows that the bricks'
+// slots hold, one more of either than their own -- takes `bytes` of staging.
+// Whole planes while one layer's fit `max`, else rows of one layer; a single
+// row of bricks may take more than `max`.
+struct UploadGroup {
+    uint32_t layers, rows;
+    uint64_t bytes;
+};
+constexpr uint64_t slot_extent(uint64_t bricks, int lb, int s)
+{
+    const uint64_t n = (bricks << lb) + 1u;
+    return n < (uint64_t)s ? n : (uint64_t)s;
+}
+constexpr UploadGroup upload_group(uint64_t row_bytes, int s1, int s2, int lb, uint64_t max)
+{
+    UploadGroup g = {1, 1, 0};
+    const uint32_t nby = bricks_along(s1, lb), nbz = bricks_along(s2, lb);
+    const uint64_t plane = row_bytes * (uint64_t)s1, planes = max / plane, depth = slot_extent(1, lb, s2);
+    if (planes >= depth) {
+        g.rows = nby;
+        if (planes >= (uint64_t)s2) g.layers = nbz;
+        else g.layers = (uint32_t)((planes - 1) >> lb);   // at least 1: planes >= 2^lb + 1
+        g.bytes = slot_extent(g.layers, lb, s2) * plane;
+    } else {
+        const uint64_t lines = max / (row_bytes * depth);
+        if (lines >= (uint64_t)s1) g.rows = nby;
+        else if (lines > (1u << lb)) g.rows = (uint32_t)((lines - 1) >> lb);
+        g.bytes = depth * slot_extent(g.rows, lb, s1) * row_bytes;
+    }
+    return g;
+}
+// The source indices along an axis of size s for bricks [b, b + n): texel X
+// holds voxel X - 1, the edge texels the edge voxels.
+constexpr int source_begin(uint32_t b, int lb, int s)
+{
+    const int64_t at = ((int64_t)b << lb) - 1;
+    return at < 0 ? 0 : at < s ? (int)at : s - 1;
+}
+constexpr int source_end(uint32_t b, uint32_t n, int lb, int s)
+{
+    const int64_t at = ((int64_t)b + n) << lb;
+    return at < s ? (int)at : s;
+}
+
 // Whether a brick whose density range is [lo, hi] can only ever sample LUT
 // entries that are exactly transparent.  A sample of density rho reads
 // u = clamp(rho*N - 1/2, 0, N-1) and weights entry floor(u) by 1 - frac(u)
