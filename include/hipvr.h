@@ -112,7 +112,8 @@ const char *hvr_last_error(void);
 int hvr_device_count(int *count);
 
 /* Free and total device memory in bytes (no counterpart in the reference;
- * for memory-budgeted serving). */
+ * for memory-budgeted serving).  A destroyed volume's block that the library
+ * keeps for the next volume counts as free. */
 int hvr_device_memory(int device, unsigned long long *free_bytes, unsigned long long *total_bytes);
 
 /* ---- context: replaces ModernGLManager.__init__ (manager.py:14-41:
@@ -167,6 +168,17 @@ int hvr_volume_upload_normals(hvr_volume *vol, const float *data);
 int hvr_volume_upload_scalar_normals(hvr_volume *vol, const float *data);
 int hvr_volume_generate_blobs(hvr_volume *vol, int n_blobs, const double *centers, const double *sigmas,
                               const double *amps, double noise, unsigned long long seed);
+
+/* Memory kept between volumes (no counterpart in the reference).  The last
+ * block of at most 512 MiB that destroyed volumes left on a device stays
+ * allocated for the next volume on it, and a context keeps what fields passed
+ * through on their way into volumes, at most 256 MiB of device memory and 12 MiB
+ * of pinned host memory.  hvr_kept_memory: the device bytes of both.  hvr_trim
+ * gives all of it back, to other users of the device as well (it waits for the
+ * device); so do the context's end and that of the device's last context, and
+ * an allocation of this library that would fail takes the block. */
+int hvr_kept_memory(hvr_ctx *ctx, unsigned long long *bytes);
+int hvr_trim(hvr_ctx *ctx);
 
 /* Device bytes held by the volume's texels. */
 int hvr_volume_bytes(const hvr_volume *vol, uint64_t *bytes);

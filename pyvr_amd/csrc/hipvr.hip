@@ -172,10 +172,11 @@ static long long resident_rays(const hvr_ctx *c) { return 2048ll * c->ncu; }
 // go at that rate have stalled hipMalloc for 11 ms at a time.  The last block
 // freed on a device is therefore kept for the next volume on it, from any
 // context: at most one, of at most kSpareMax bytes.  It is given back when
-// the next volume cannot use it (too small, or more than a quarter too large),
-// when an allocation fails for want of memory, and with the device's last
-// context.  A block is put aside only once the device is idle, as hipFree
-// would wait for, so no stream still reads it.
+// the next volume cannot use it (too small, or more than a sixteenth too large),
+// when an allocation of this library fails for want of memory, by hvr_trim, and
+// with the device's last context; hvr_device_memory counts it as free.  A block
+// is put aside only once the device is idle, as hipFree would wait for, so no
+// stream still reads it.
 static constexpr size_t kSpareMax = (size_t)512 << 20;
 static constexpr int kMaxDevices = 64;
 struct SpareBlock {
@@ -196,6 +197,12 @@ static void *spare_take(int device, size_t *bytes)
     g_spare[device].p = nullptr;
     return p;
 }
+static size_t spare_bytes(int device)
+{
+    if (device < 0 || device >= kMaxDevices) return 0;
+    std::lock_guard<std::mutex> lock(g_spare_mu);
+    return g_spare[device].p ? g_spare[device].bytes : 0;
+}
 // hipMalloc that gives the spare block back before it fails; the device is current.
 static hipError_t dev_malloc(int device, void **p, size_t n)
 {
@@ -214,7 +221,7 @@ static hipError_t block_alloc(int device, void **p, size_t n, size_t *got)
 {
     size_t b = 0;
     if (void *spare = spare_take(device, &b)) {
-        if (b >= n && b - n <= n / 4) {
+        if (b >= n && b - n <= n / 16) {
             *p = spare;
             *got = b;
             return hipSuccess;
@@ -754,8 +761,32 @@ int hvr_device_memory(int device, unsigned long long *free_bytes, unsigned long 
     HIPCHK(hipSetDevice(device));
     size_t f = 0, t = 0;
     HIPCHK(hipMemGetInfo(&f, &t));
-    if (free_bytes) *free_bytes = f;
+    if (free_bytes) *free_bytes = f + spare_bytes(device);
     if (total_bytes) *total_bytes = t;
+    return HVR_OK;
+}
+
+int hvr_kept_memory(hvr_ctx *c, unsigned long long *bytes)
+{
+    if (!c || !bytes) return fail(HVR_EINVAL, "null argument");
+    *bytes = spare_bytes(c->device) + c->stage_bytes;
+    return HVR_OK;
+}
+
+int hvr_trim(hvr_ctx *c)
+{
+    if (!c) return fail(HVR_EINVAL, "ctx is null");
+    HIPCHK(hipSetDevice(c->device));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    size_t b;
+    if (void *spare = spare_take(c->device, &b)) HIPCHK(hipFree(spare));
+    float *const stage = c->d_stage;
+    c->d_stage = nullptr;
+    c->stage_bytes = 0;
+    if (stage) HIPCHK(hipFree(stage));
+    char *const ring = c->h_up;
+    c->h_up = nullptr;
+    if (ring) HIPCHK(hipHostFree(ring));
     return HVR_OK;
 }
 

@@ -45,6 +45,7 @@ EXPORTS = (
     "hvr_resize", "hvr_debug_inject_fault", "hvr_render_async_to_noalloc",
     "hvr_batch_set_kernel", "hvr_set_dispatch_order", "hvr_dispatch_order_info", "hvr_set_readback",
     "hvr_shaded_sample_counts", "hvr_touched_bricks", "hvr_batch_reserve", "hvr_batch_set_readback",
+    "hvr_kept_memory", "hvr_trim",
 )
 
 # batch ray-tile shapes (hvr_batch_set_tile_shape)
@@ -95,6 +96,8 @@ def _declare(L):
         "hvr_create": ([i, i, i, ctypes.POINTER(vp)], i),
         "hvr_destroy": ([vp], i),
         "hvr_resize": ([vp, i, i], i),
+        "hvr_kept_memory": ([vp, ctypes.POINTER(ctypes.c_ulonglong)], i),
+        "hvr_trim": ([vp], i),
         "hvr_debug_inject_fault": ([ctypes.c_char_p, i, i], i),
         "hvr_volume_create": ([vp, i, i, i, i, i, ctypes.POINTER(vp)], i),
         "hvr_volume_upload_scalar": ([vp, fp], i),
@@ -183,6 +186,19 @@ def device_memory(device: int = 0):
     f, t = ctypes.c_ulonglong(), ctypes.c_ulonglong()
     check(lib().hvr_device_memory(int(device), ctypes.byref(f), ctypes.byref(t)), "hvr_device_memory")
     return int(f.value), int(t.value)
+
+
+def kept_memory(ctx) -> int:
+    """Device bytes the library keeps for later volumes (``hvr_kept_memory``):
+    the device's and the context ``ctx``'s own."""
+    b = ctypes.c_ulonglong()
+    check(lib().hvr_kept_memory(ctx, ctypes.byref(b)), "hvr_kept_memory")
+    return int(b.value)
+
+
+def trim(ctx) -> None:
+    """Give that memory back (``hvr_trim``), to other users of the device too."""
+    check(lib().hvr_trim(ctx), "hvr_trim")
 
 
 def check(rc: int, what: str = "") -> None:

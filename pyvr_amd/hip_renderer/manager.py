@@ -453,6 +453,10 @@ class HipManager:
         check(self.L.hvr_last_kernel_ms(self.ctx, ctypes.byref(a), ctypes.byref(b)), "hvr_last_kernel_ms")
         return a.value, b.value
 
+    def trim(self):
+        """Give back the device memory kept for later volumes (hvr_trim)."""
+        check(self.L.hvr_trim(self.ctx), "hvr_trim")
+
     def cleanup(self):
         """Release every device resource (safe to call more than once)."""
         if self._released:

@@ -65,6 +65,15 @@ class PlainRenderer:
     def resident_bytes(self) -> int:
         return sum(rv.nbytes() for rv in self._resident.values())
 
+    def kept_bytes(self) -> int:
+        """Device bytes kept for later volumes: the last released one's block
+        and what fields passed through on their way in."""
+        return _lib.kept_memory(self.ctx)
+
+    def trim(self):
+        """Give the kept bytes back to the device (waits for it)."""
+        _lib.trim(self.ctx)
+
     def prepare(self, volume, camera, color_transfer_function, opacity_transfer_function, width: int = 512,
                 height: int = 512, config: Optional[RenderConfig] = None, light: Optional[Light] = None,
                 opacity_threshold: float = REFERENCE_TERMINATION_ALPHA, lut_size: Optional[int] = None):

@@ -184,6 +184,12 @@ class HipVolumeRenderer:
         """(march_ms, setup_ms) of the last rendered frame."""
         return self.gl_manager.last_kernel_ms()
 
+    def trim(self) -> None:
+        """Give back the device memory kept for the next volume (an earlier
+        volume's block and what its fields passed through on their way in), for
+        other users of the device."""
+        self.gl_manager.trim()
+
     def close(self) -> None:
         """Release the device resources now (also done on garbage collection)."""
         self.gl_manager.cleanup()

@@ -16,7 +16,9 @@ turns a stream of requests into batches for ``BatchRenderer``:
   launch or in-flight batch uses are evicted, least recently used first;
   the budget also reserves what the batches in flight hold (output
   pools, per-request brick flags for the largest registered volume,
-  staging), as those pools grow;
+  staging), as those pools grow, and memory kept for later volumes (an
+  evicted volume's block, upload staging) is given back where it does not
+  fit beside them;
 * with ``max_batch_samples`` a batch also stops at that many estimated
   samples (``estimated_samples``), so that a burst of large requests is
   split into batches of bounded duration;
@@ -289,10 +291,19 @@ class RenderServer:
                     room += v.bytes
                     self.evictions += 1
             if nbytes > room:
+                self._give_back()
                 return False
         self.backend.upload(volume, device_normals=device_normals)
         self._resident[key] = _Resident(volume, nbytes)
+        self._give_back()
         return True
+
+    def _give_back(self):
+        """Free what the backend keeps for later volumes where the budget has no
+        room for it beside the resident ones."""
+        kept = getattr(self.backend, "kept_bytes", None)
+        if kept is not None and self.resident_bytes() + self.reserved + kept() > self.memory_budget:
+            self.backend.trim()
 
     # -- requests ------------------------------------------------------------
     def submit(self, req: ServeRequest) -> ServeRequest:
