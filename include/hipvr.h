@@ -268,8 +268,10 @@ int hvr_shaded_sample_counts(hvr_ctx *ctx, uint32_t *counts);
 int hvr_touched_bricks(hvr_ctx *ctx, unsigned long long *touched, unsigned long long *bricks,
                        unsigned long long *brick_bytes);
 
-/* Milliseconds of the last frame's march kernel and ray-setup kernel,
- * measured with HIP events on the context's stream. */
+/* Milliseconds of the last frame's march (after a LUT or volume change with the
+ * transparent-brick flags, which it then recomputes) and of the ordering pass
+ * before it (hvr_set_dispatch_order; 0 in row order), measured with HIP events
+ * on the context's stream. */
 int hvr_last_kernel_ms(hvr_ctx *ctx, float *march_ms, float *setup_ms);
 
 /* Render into a caller-provided device buffer of width*height*4 bytes
@@ -287,7 +289,7 @@ int hvr_copy_to_host(hvr_ctx *ctx, void *host, const void *device_ptr, uint64_t 
 int hvr_device_copy(hvr_ctx *ctx, void *dst, const void *src, uint64_t bytes);
 
 /* Per-launch kernel timing over a region: after hvr_timing_begin every
- * frame records HIP events around its ray-setup and march kernels on the
+ * frame records HIP events around its ordering pass and its march on the
  * context's stream (up to `max_frames` frames); hvr_timing_end waits and
  * returns the summed kernel milliseconds and the number of frames timed. */
 int hvr_timing_begin(hvr_ctx *ctx, int max_frames);

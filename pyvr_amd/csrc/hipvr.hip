@@ -360,13 +360,13 @@ static bool flags_count(hvr_ctx *c, bool wait)
     return c->flags_count_known;
 }
 
-// Transparent-brick flags of volume v for the current LUT, recomputed when
-// either changed; their count comes back to the host without a wait.
-// Returns the flags when the march should step over transparent bricks:
-// always in HVR_SKIP_ON; in HVR_SKIP_AUTO when enough bricks are
-// transparent, or while the count is not back yet (skipping gives the same
-// image, so the choice only affects speed); nullptr otherwise.
-static const uint8_t *brick_flags(hvr_ctx *c, const hvr_volume *v)
+// Transparent-brick flags of volume v for the current LUT.  Returns the flags
+// when the march should step over transparent bricks: always in HVR_SKIP_ON; in
+// HVR_SKIP_AUTO when enough bricks are transparent, or while the count is not
+// back yet (skipping gives the same image, so the choice only affects speed);
+// nullptr otherwise.  Where the LUT or the volume changed, `stale` says that
+// launch_flags has to recompute them before the march.
+static const uint8_t *brick_flags(hvr_ctx *c, const hvr_volume *v, bool *stale)
 {
     if (c->skip_mode == HVR_SKIP_OFF || !v || !v->scalar_loaded || !c->d_nz) return nullptr;
     const uint64_t nb = (uint64_t)v->nbx * v->nby * v->nbz;
@@ -390,26 +390,36 @@ static const uint8_t *brick_flags(hvr_ctx *c, const hvr_volume *v)
             if (dev_malloc(c->device, (void **)&c->d_flags, nb) != hipSuccess) return none();
             c->flags_cap = nb;
         }
-        // the count comes back asynchronously (no wait in the frame's path)
-        uint32_t *count = c->d_nclear + c->nclear_slot;
-        hipLaunchKernelGGL(k_brick_flags, dim3(clearance_tiles(v->nbx, v->nby, v->nbz)), dim3(kClearThreads), 0,
-                           c->stream, (const float2 *)v->d_range, (int)v->nbx, (int)v->nby, (int)v->nbz,
-                           (const int *)c->d_nz, c->lut_n, c->d_flags, count, c->d_nclear + (c->nclear_slot ^ 1));
-        if (hipGetLastError() != hipSuccess) return none();
-        c->nclear_slot ^= 1;
-        if (hipMemcpyAsync(c->h_nclear, count, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream) !=
-                hipSuccess ||
-            hipEventRecord(c->flags_ev, c->stream) != hipSuccess)
-            return none();
-        c->flags_vol = v;
-        c->flags_vol_gen = v->gen;
-        c->flags_lut_gen = c->lut_gen;
-        c->flags_count_known = false;
-        c->flags_total = nb;
+        *stale = true;
+        return c->d_flags;
     }
     if (c->skip_mode == HVR_SKIP_ON) return c->d_flags;
     if (!flags_count(c, false)) return c->d_flags;   // not back yet: skipping is exact either way
     return (double)c->flags_clear >= kSkipAutoFraction * (double)c->flags_total ? c->d_flags : nullptr;
+}
+
+// The flags of volume v recomputed (memory is there, brick_flags); their count
+// comes back to the host without a wait.  Whether the march can use them.
+static bool launch_flags(hvr_ctx *c, const hvr_volume *v)
+{
+    uint32_t *count = c->d_nclear + c->nclear_slot;
+    hipLaunchKernelGGL(k_brick_flags, dim3(clearance_tiles(v->nbx, v->nby, v->nbz)), dim3(kClearThreads), 0,
+                       c->stream, (const float2 *)v->d_range, (int)v->nbx, (int)v->nby, (int)v->nbz,
+                       (const int *)c->d_nz, c->lut_n, c->d_flags, count, c->d_nclear + (c->nclear_slot ^ 1));
+    bool ok = hipGetLastError() == hipSuccess;
+    if (ok) c->nclear_slot ^= 1;
+    ok = ok && hipMemcpyAsync(c->h_nclear, count, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream) == hipSuccess &&
+         hipEventRecord(c->flags_ev, c->stream) == hipSuccess;
+    if (!ok) {
+        (void)hipGetLastError();
+        return false;
+    }
+    c->flags_vol = v;
+    c->flags_vol_gen = v->gen;
+    c->flags_lut_gen = c->lut_gen;
+    c->flags_count_known = false;
+    c->flags_total = (uint64_t)v->nbx * v->nby * v->nbz;
+    return true;
 }
 
 // Whether a volume is read through buffer loads (32-bit offsets, 24-bit brick
@@ -434,19 +444,20 @@ static double ray_steps(const FrameConst &fc)
 struct MarchPlan {
     int nm;
     const uint8_t *skip;
+    bool stale;   // skip is to be recomputed first (launch_flags)
     bool buf;
     int lanes;
 };
 static MarchPlan march_plan(hvr_ctx *c, const FrameConst &fc, bool count)
 {
-    MarchPlan m = {-1, nullptr, false, 1};
+    MarchPlan m = {-1, nullptr, false, false, 1};
     const hvr_volume *S = c->scalar_vol, *N = c->normal_vol;
     if (c->lut_n > kLutLdsMax || !S || c->scalar_role != HVR_ROLE_SCALAR || !(S->lb == 3 || S->lb == 4)) return m;
     if (!N) m.nm = NM_ZERO;
     else if (N == S && c->normal_role == HVR_ROLE_SCALAR) m.nm = NM_ALIAS;
     else if (N == S && c->normal_role == HVR_ROLE_NORMAL && fmt_has_normal(S->fmt)) m.nm = NM_SAME;
     if (m.nm < 0) return m;
-    m.skip = brick_flags(c, S);
+    m.skip = brick_flags(c, S, &m.stale);
     m.buf = volume_buf(S) && !c->force_global;
     if (m.buf && !count)
         m.lanes = march_lanes((long long)c->W * c->H, resident_rays(c), m.skip != nullptr, ray_steps(fc),
@@ -506,7 +517,8 @@ static int enqueue_frame(hvr_ctx *c, bool count, uchar4 *dst, bool count_shaded 
     // events of this frame: the context's own, or the next slots of an
     // open timing region; hvr_last_kernel_ms reads the frame's events
     // (each event is a packet of its own on the stream, for up to 5 us of the
-    // frame: a frame with nothing before its march has no first event)
+    // frame: a frame in row order has no first event, and flags that are to be
+    // recomputed count as the march's)
     hipEvent_t e0 = c->ev[0], e1 = c->ev[1], e2 = c->ev[2];
     const int timed = c->tev && c->timing_n < c->timing_max ? c->timing_n++ : -1;
     if (timed >= 0) {
@@ -515,7 +527,7 @@ static int enqueue_frame(hvr_ctx *c, bool count, uchar4 *dst, bool count_shaded 
         e1 = (*c->tev)[k + 1];
         e2 = (*c->tev)[k + 2];
     }
-    const MarchPlan plan = march_plan(c, fc, count);
+    MarchPlan plan = march_plan(c, fc, count);
     const MarchTile bt = march_tile(plan.lanes);
     const int ntx = (c->W + (1 << bt.lbw) - 1) >> bt.lbw, nty = (c->H + (1 << bt.lbh) - 1) >> bt.lbh;
     // cost-ordered dispatch (hvr_set_dispatch_order): the blocks of the
@@ -549,6 +561,7 @@ static int enqueue_frame(hvr_ctx *c, bool count, uchar4 *dst, bool count_shaded 
     if (timed >= 0) (*c->tev_ordered)[(size_t)timed] = ordered;
     // the march sets up its rays itself
     HIPCHK(hipEventRecord(e1, c->stream));
+    if (plan.stale && !launch_flags(c, c->scalar_vol)) plan.skip = nullptr;
     const bool host = !dst && c->readback_mode == HVR_READBACK_DIRECT;
     launch_march(c, fc, dst ? dst : host ? (uchar4 *)c->h_pinned_dev : c->d_out, count, plan,
                  ordered ? c->d_order : nullptr);
