@@ -302,7 +302,8 @@ int hvr_timing_end(hvr_ctx *ctx, double *march_ms, double *setup_ms, int *frames
  * counts are identical in every mode.  HVR_SKIP_AUTO (the default) steps
  * over bricks when at least 18 % of the bound volume's bricks are
  * transparent for the current LUT.  The first frame after a LUT or volume
- * change computes the brick flags and waits for their count. */
+ * change computes the brick flags; their count comes back without a wait, and
+ * until it has, AUTO steps over. */
 #define HVR_SKIP_OFF 0
 #define HVR_SKIP_ON 1
 #define HVR_SKIP_AUTO 2
