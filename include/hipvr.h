@@ -102,7 +102,9 @@ int hvr_abi_version(void);
  * hvr_set_params, hvr_bind, hvr_render_async, hvr_render_async_to,
  * hvr_read, hvr_sample_counts, hvr_batch_create, hvr_batch_add,
  * hvr_batch_run_async, hvr_batch_wait, hvr_batch_query.  Inside the uploads,
- * "hvr_upload_ring" fails a copy that takes the library's own pinned memory. */
+ * "hvr_upload_ring" fails a copy that takes the library's own pinned memory;
+ * inside hvr_batch_run_async, "hvr_batch_capture" fails a launch of a shape
+ * that has no captured graph. */
 int hvr_debug_inject_fault(const char *function, int code, int after);
 
 /* Message of the last failed call on this thread ("" if none). */

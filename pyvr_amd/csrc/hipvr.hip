@@ -1582,6 +1582,18 @@ struct BatchReq {
     uint64_t lut_hash;       // float_hash
 };
 
+// A captured launch and the shape it was captured for.  The shape holds each
+// class's kernel, which its number of rays chooses (march_lanes), so batches of
+// changing sizes come back to a few shapes: each keeps its graph, up to
+// kBatchGraphs of them (capturing and instantiating one takes 9 us of a 31 us
+// launch, and milliseconds the first time a kernel is used).
+struct BatchGraph {
+    std::string key;
+    hipGraph_t graph;
+    hipGraphExec_t exec;
+};
+constexpr size_t kBatchGraphs = 8;
+
 struct hvr_batch {
     hvr_ctx *ctx;
     hipStream_t stream;
@@ -1602,9 +1614,7 @@ struct hvr_batch {
     size_t flags_cap;
     uint32_t *d_counters;                 // tile counter per class
     std::vector<size_t> out_off;          // per request (add order): pixel offset in the pools
-    hipGraph_t graph;
-    hipGraphExec_t exec;
-    std::string key;                      // shape the graph was captured for
+    std::vector<BatchGraph> graphs;       // captured launches, most recently used first
     hipEvent_t ev0, ev1, ev2;             // graph start / end, copies back done
     bool ran, counted;
     size_t out_pixels;
@@ -1651,13 +1661,14 @@ static int grow(int device, void **d, void **h, size_t *cap, size_t need, bool *
     return HVR_OK;
 }
 
-static void batch_drop_graph(hvr_batch *b)
+// Drop the graphs from the n-th most recently used on (no launch in flight).
+static void batch_drop_graphs(hvr_batch *b, size_t n = 0)
 {
-    if (b->exec) (void)hipGraphExecDestroy(b->exec);
-    if (b->graph) (void)hipGraphDestroy(b->graph);
-    b->exec = nullptr;
-    b->graph = nullptr;
-    b->key.clear();
+    for (size_t k = n; k < b->graphs.size(); ++k) {
+        (void)hipGraphExecDestroy(b->graphs[k].exec);
+        (void)hipGraphDestroy(b->graphs[k].graph);
+    }
+    if (n < b->graphs.size()) b->graphs.resize(n);
 }
 
 extern "C" {
@@ -1673,8 +1684,6 @@ int hvr_batch_create(hvr_ctx *c, hvr_batch **out)
     b->tile_shape = HVR_TILE_8X8;
     b->variant = BV_DEFAULT;
     b->readback = HVR_READBACK_DIRECT;
-    b->exec = nullptr;
-    b->graph = nullptr;
     hipError_t e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreate(&b->ev0);
     if (e == hipSuccess) e = hipEventCreate(&b->ev1);
@@ -1694,7 +1703,7 @@ int hvr_batch_destroy(hvr_batch *b)
     if (!b) return HVR_OK;
     (void)hipSetDevice(b->ctx->device);
     if (b->stream) (void)hipStreamSynchronize(b->stream);
-    batch_drop_graph(b);
+    batch_drop_graphs(b);
     (void)hipFree(b->d_stage);
     (void)hipFree(b->d_out);
     (void)hipFree(b->d_counts);
@@ -1811,7 +1820,7 @@ int hvr_batch_reserve(hvr_batch *b, int max_requests, unsigned long long max_pix
     if (const int rc = grow(b->ctx->device, (void **)&b->d_out, (void **)&b->h_out, &b->out_cap, pixels * 4, &moved_out)) return rc;
     if (const int rc = grow(b->ctx->device, (void **)&b->d_flags, nullptr, &b->flags_cap, flags, &moved_out)) return rc;
     if (moved_out) b->h_out_dev_of = nullptr;   // a new pinned pool may reuse the old address
-    if (moved) batch_drop_graph(b);
+    if (moved) batch_drop_graphs(b);
     return HVR_OK;
 }
 
@@ -1899,7 +1908,7 @@ int hvr_batch_run_async(hvr_batch *b, int count)
         b->counts_cap = cb / 4;
     }
     if (moved_out) b->h_out_dev_of = nullptr;   // a new pinned pool may reuse the old address
-    if (moved) batch_drop_graph(b);
+    if (moved) batch_drop_graphs(b);
     // direct: the march stores each pixel straight into the pinned pool
     // through its device address (posted writes over the host link while
     // the batch runs, no copy after it)
@@ -1972,8 +1981,12 @@ int hvr_batch_run_async(hvr_batch *b, int count)
     for (const Cls &k : cls)
         key += "/" + std::to_string(k.fmt) + "." + std::to_string(k.nm) + "." + std::to_string(k.lb) + "." +
                std::to_string(k.buf) + "." + std::to_string(k.variant);
-    if (key != b->key || !b->exec) {
-        batch_drop_graph(b);
+    const auto known = std::find_if(b->graphs.begin(), b->graphs.end(), [&](const BatchGraph &g) { return g.key == key; });
+    if (known != b->graphs.end()) {
+        std::rotate(b->graphs.begin(), known, known + 1);
+    } else {
+        HVR_FAULT_POINT("hvr_batch_capture");
+        batch_drop_graphs(b, kBatchGraphs - 1);
         HIPCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
         int rc = HVR_OK;
         if (hipMemcpyAsync(b->d_stage, b->h_stage, b->stage_cap, hipMemcpyHostToDevice, b->stream) != hipSuccess)
@@ -1989,18 +2002,20 @@ int hvr_batch_run_async(hvr_batch *b, int count)
                 batch_fn(cls[k].fmt, cls[k].nm, cls[k].lb, count != 0, b->tile_shape, cls[k].buf, cls[k].variant);
             rc = fn ? fn(b->d_stage, (int)k, b->d_counters + k, lut_cap, b->ncu, b->stream) : HVR_EINVAL;
         }
-        hipGraph_t g = nullptr;
-        const hipError_t e = hipStreamEndCapture(b->stream, &g);
+        BatchGraph g = {key, nullptr, nullptr};
+        const hipError_t e = hipStreamEndCapture(b->stream, &g.graph);
         if (rc != HVR_OK || e != hipSuccess) {
-            if (g) (void)hipGraphDestroy(g);
+            if (g.graph) (void)hipGraphDestroy(g.graph);
             return fail(HVR_EDEVICE, "capturing the batch graph failed");
         }
-        b->graph = g;
-        HIPCHK(hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
-        b->key = key;
+        if (const hipError_t ei = hipGraphInstantiate(&g.exec, g.graph, nullptr, nullptr, 0)) {
+            (void)hipGraphDestroy(g.graph);
+            return fail_hip(ei, "instantiating the batch graph");
+        }
+        b->graphs.insert(b->graphs.begin(), std::move(g));
     }
     HIPCHK(hipEventRecord(b->ev0, b->stream));
-    HIPCHK(hipGraphLaunch(b->exec, b->stream));
+    HIPCHK(hipGraphLaunch(b->graphs.front().exec, b->stream));
     HIPCHK(hipEventRecord(b->ev1, b->stream));
     if (!direct) HIPCHK(hipMemcpyAsync(b->h_out, b->d_out, pixels * 4, hipMemcpyDeviceToHost, b->stream));
     if (count) HIPCHK(hipMemcpyAsync(b->h_counts, b->d_counts, pixels * 4, hipMemcpyDeviceToHost, b->stream));
