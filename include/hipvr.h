@@ -125,7 +125,9 @@ int hvr_device_memory(int device, unsigned long long *free_bytes, unsigned long 
  * context is created it uses 64-bit global loads, as for larger volumes
  * (same results; for testing that path).  HVR_STAGE=<bytes>, likewise, bounds
  * the device memory a field uploaded from the host passes through, below its
- * 256 MiB (fields larger than that arrive in groups of bricks). */
+ * 256 MiB (fields larger than that arrive in groups of bricks), and
+ * HVR_BUILD=wide builds volumes with 64-bit voxel offsets, as from 2^30 voxels
+ * on. */
 int hvr_create(int device, int width, int height, hvr_ctx **out);
 int hvr_destroy(hvr_ctx *ctx);
 /* Change the framebuffer size (no counterpart in the reference, whose

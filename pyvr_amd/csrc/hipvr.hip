@@ -134,6 +134,7 @@ struct hvr_ctx {
     int skip_mode;         // HVR_SKIP_OFF / _ON / _AUTO
     int skip_used;         // whether the last frame's march stepped over bricks
     bool force_global;     // HVR_GATHER=global at creation: 64-bit loads for every volume
+    bool force_wide;       // HVR_BUILD=wide at creation: 64-bit voxel offsets for every volume
     int ncu;               // compute units of the device
     size_t pix_cap;        // pixels d_out and h_pinned hold
     size_t counts_cap;     // pixels d_counts holds
@@ -604,7 +605,7 @@ static void launch_build(const hvr_volume *v, const BuildArgs &a, unsigned block
         }
         launch(std::false_type{});
     };
-    if (voxels < (1ull << 30)) go(uint32_t(0));
+    if (voxels < (1ull << 30) && !v->ctx->force_wide) go(uint32_t(0));
     else go(uint64_t(0));
 }
 static int build_group(const hvr_volume *v, BuildArgs a, uint32_t by0, uint32_t by1, uint32_t bz0, uint32_t bz1)
@@ -823,6 +824,8 @@ int hvr_create(int device, int width, int height, hvr_ctx **out)
     c->readback_mode = HVR_READBACK_DIRECT;
     const char *gather = getenv("HVR_GATHER");
     c->force_global = gather && strcmp(gather, "global") == 0;
+    const char *build = getenv("HVR_BUILD");
+    c->force_wide = build && strcmp(build, "wide") == 0;
     c->max_stage = kMaxStage;
     if (const char *stage = getenv("HVR_STAGE"))
         if (const unsigned long long n = strtoull(stage, nullptr, 10)) c->max_stage = (size_t)std::min<uint64_t>(n, kMaxStage);
