@@ -325,9 +325,9 @@ int hvr_skip_info(hvr_ctx *ctx, unsigned long long *clear_bricks, unsigned long 
  * bound of its rays and the march starts the longest first.  The image and
  * the sample counts are identical in every mode.  HVR_ORDER_AUTO (the
  * default) orders frames of more blocks than the device keeps resident at
- * once (8 per compute unit) and at least 8 block rows, unless the frame is
- * larger than 2.25 times what is resident or its rays take few steps, where
- * row order is faster. */
+ * once (8 per compute unit) and at least 8 block rows whose rays take many
+ * steps, unless transparent bricks are stepped over and the frame is larger
+ * than 2.25 times what is resident, where row order is faster. */
 #define HVR_ORDER_OFF 0
 #define HVR_ORDER_ON 1
 #define HVR_ORDER_AUTO 2

@@ -430,13 +430,14 @@ static bool volume_buf(const hvr_volume *v)
     return v->bytes <= 0xffffffffull && (uint64_t)v->nbx * v->nby * v->nbz < (1ull << 24);
 }
 
-// The largest iteration bound that the frame's rays can have.
-static double ray_steps(const FrameConst &fc)
+// The largest iteration bound that a frame's rays can have.
+static double ray_steps(const float *bmin, const float *bmax, double step, int max_steps)
 {
-    const double diagonal = std::sqrt((double)fc.ext[0] * fc.ext[0] + (double)fc.ext[1] * fc.ext[1] +
-                                      (double)fc.ext[2] * fc.ext[2]);
-    return std::min((double)fc.max_steps, diagonal / (double)fc.step);
+    double d2 = 0.0;
+    for (int k = 0; k < 3; ++k) d2 += ((double)bmax[k] - bmin[k]) * ((double)bmax[k] - bmin[k]);
+    return std::min((double)max_steps, std::sqrt(d2) / step);
 }
+static double ray_steps(const FrameConst &fc) { return ray_steps(fc.bmin, fc.bmax, fc.step, fc.max_steps); }
 
 // How a frame is marched: the fast instances of the scalar volume's format
 // (nm >= 0: normals from the same texels, as (rho, 0, 0) of the same volume,
@@ -538,8 +539,8 @@ static int enqueue_frame(hvr_ctx *c, bool count, uchar4 *dst, bool count_shaded 
     const bool ordered =
         head_rows > 0 && (c->order_mode == HVR_ORDER_ON ||
                           (c->order_mode == HVR_ORDER_AUTO &&
-                           order_auto((long long)ntx * nty, (long long)c->W * c->H, resident_rays(c), plan.lanes,
-                                      ray_steps(fc))));
+                           order_auto((long long)ntx * nty, (long long)c->W * c->H, resident_rays(c),
+                                      plan.skip != nullptr, plan.lanes, ray_steps(fc))));
     if (ordered) {
         const size_t words = (size_t)head_rows * ntx * (1 + kOrderBuckets);
         if (words > c->order_words) {
@@ -1586,7 +1587,7 @@ struct BatchReq {
 };
 
 // A captured launch and the shape it was captured for.  The shape holds each
-// class's kernel, which its number of rays chooses (march_lanes), so batches of
+// class's kernel, which its number of rays chooses (batch_lanes), so batches of
 // changing sizes come back to a few shapes: each keeps its graph, up to
 // kBatchGraphs of them (capturing and instantiating one takes 9 us of a 31 us
 // launch, and milliseconds the first time a kernel is used).
@@ -1875,10 +1876,15 @@ int hvr_batch_run_async(hvr_batch *b, int count)
         k.variant = count ? (int)BV_DEFAULT : b->variant;
         k.bx = b->tile_shape == HVR_TILE_16X4 ? 32 : 16;
         k.by = (b->tile_shape == HVR_TILE_16X4 ? 4 : 8) * (batch_variant_waves(k.variant) / 2);
-        // few rays: several lanes each, as in a single frame of as many
-        long long rays = 0;
-        for (int i : k.members) rays += (long long)b->reqs[i].W * b->reqs[i].H;
-        const int lanes = march_lanes(rays, 2048ll * b->ncu, true, 0.0, texel_bytes(k.fmt), 0);
+        // few rays: several lanes each
+        double rays = 0.0, samples = 0.0;
+        for (int i : k.members) {
+            const BatchReq &r = b->reqs[i];
+            const double n = (double)r.W * r.H;
+            rays += n;
+            samples += n * ray_steps(r.params.bmin, r.params.bmax, r.params.step, r.params.max_steps);
+        }
+        const int lanes = batch_lanes((long long)rays, 2048ll * b->ncu, samples / rays);
         if (lanes > 1 && !count && k.buf && k.variant == BV_DEFAULT && b->tile_shape == HVR_TILE_8X8) {
             const MarchTile bt = march_tile(lanes);
             k.variant = lanes == 4 ? BV_LANES4 : BV_LANES2;
@@ -2163,9 +2169,7 @@ int hvr_render_async_to_noalloc(hvr_ctx *c, void *dst)
     else return fail(HVR_ESTATE, "hvr_render_async_to_noalloc: normals must come from the scalar volume, or none");
     const bool buf = volume_buf(S) && !c->force_global;
     const FrameConst fc = frame_const(c);
-    const int lanes = buf ? march_lanes((long long)c->W * c->H, resident_rays(c), true, ray_steps(fc),
-                                        texel_bytes(S->fmt), S->bytes)
-                          : 1;
+    const int lanes = buf ? batch_lanes((long long)c->W * c->H, resident_rays(c), ray_steps(fc)) : 1;
     const BatchLaunchFn fn = batch_fn(S->fmt, nm, S->lb, false, HVR_TILE_8X8, buf,
                                       lanes == 4 ? BV_LANES4 : lanes == 2 ? BV_LANES2 : BV_DEFAULT);
     if (!fn) return fail(HVR_EINVAL, "hvr_render_async_to_noalloc: brick edge must be 8 or 16 (log2 3 or 4)");

@@ -762,7 +762,7 @@ __device__ __forceinline__ void composite(const FrameConst &fc, const float4 &q,
 }
 
 // K2 -- march and composite (volume.frag.glsl:84-121), P adjacent lanes per
-// ray (march_lanes; one, in most large frames).  A block of 4 waves covers
+// ray (march_lanes; one in most large frames).  A block of 4 waves covers
 // 16x16, 16x8 or 8x8 pixels; each wave64 an 8x8, 8x4 or 4x4 tile.  Blocks
 // are dispatched round-robin over the 8 XCDs (block b on XCD (b + c) mod 8,
 // c varying from launch to launch), and each XCD runs its blocks in order.
@@ -1776,7 +1776,7 @@ struct TileShape<1> {
 // compiler then keeps a few per-ray values in scratch outside the march
 // loop rather than run 7 waves.  16-byte texels would spill inside the
 // loop, so their kernels keep the registers they need.
-// P lanes per ray (march_lanes, by a class's rays; no gating): a wave covers
+// P lanes per ray (batch_lanes, by a class's rays; no gating): a wave covers
 // 8x4 or 4x4 pixels then.
 template <int SF, int NM, int LB, bool COUNT, int TS, bool BUF, int W = kBatchWaves, bool SKIP = true,
           bool GATE = true, int P = 1>

@@ -210,30 +210,67 @@ constexpr int ordered_block(int b, int head, const U *cnt, const U *slots, int c
 // composite them in order, a ray ends in as many fewer iterations, for more
 // instructions a sample (14-18 % with 2 lanes, about 35 % with 4).  `resident`:
 // the rays the device marches at once with one lane each (524,288 on 256
-// compute units).  Measured (us, 1 / 2 / 4 lanes; cameras averaged): 64^2 of a
-// 256^3 volume 338 / 177 / 100, 362^2 of it 268 / 166 / 116, 512^2 dense
-// 192 / 146 / 154, transparent-skipping 512^2 79 / 63 / 66, 1024^2 504 / 452 /
-// 480 and 366 / 331 / 409, 1280^2 601 / 635 / 720, 2048^2 1237 / 1491 / 1780.
-// Where no brick is stepped over, rays are about equally long and the device
-// stays busy to the end: 724^2 246 / 238 and 257 / 293, 1024^2 394 / 407 and
-// 446 / 487.  Both lines lie further out the longer the rays are (`steps`, the
-// largest iteration bound they can have), and that of 2 lanes does where a
-// sample waits for its texels: 16-byte ones, which take the L1 several passes,
-// and volumes well above the L2s (`bytes` in all).  692 steps, FP32+FP32x3 256^3
-// / FP16+FP16x3 320^3 / UNORM8+SNORM8x3 224^3, nothing stepped over, 1 / 2 / 4
-// lanes: 480^2 675 450 351 / 514 347 257 / 361 291 268, 640^2 721 538 495 / 548
-// 389 362 / 399 376 406, 880^2 1047 787 850 / 716 551 612 / 595 626 701;
-// skipping, 2 / 4 lanes: 640^2 299 254 / 221 206 / 252 234, 720^2 326 303 /
-// 250 240 / 285 276.  346 steps: 800^2 FP32+FP32x3 256^3 409 347 / FP16+FP16x3
-// 256^3 306 276 / UNORM8+SNORM8x3 160^3 275 299 (1 / 2 lanes), 480^2 210 191 /
-// 147 134 / 152 141 (2 / 4); 100 steps: 800^2 FP32+FP32x3 211 215.  Small volumes
-// of 8-byte texels lose 6-12 % by 2 lanes above 3/4 of the resident rays.
+// compute units).
+//
+// Where transparent bricks are stepped over, rays differ in length and the
+// lines lie far out.  Measured (us, 1 / 2 / 4 lanes; cameras averaged): 64^2 of
+// a 256^3 volume 338 / 177 / 100, 362^2 of it 268 / 166 / 116, 512^2 79 / 63 /
+// 66, 1024^2 504 / 452 / 480 and 366 / 331 / 409, 1280^2 601 / 635 / 720, 2048^2
+// 1237 / 1491 / 1780; 692 steps (`steps`: the largest iteration bound the rays
+// can have), 2 / 4 lanes: 640^2 299 254 / 221 206 / 252 234, 720^2 326 303 / 250
+// 240 / 285 276 (FP32+FP32x3 256^3 / FP16+FP16x3 320^3 / UNORM8+SNORM8x3 224^3).
+//
+// Where none are, rays of a filled volume are about equally long and the device
+// stays busy to the end, while those that end in dense matter or cross thin noise
+// still differ.  Long rays gain from lanes as long as a sample waits for its
+// texels: 16-byte ones, which take the L1 several passes, and volumes well above
+// the L2s (`bytes` in all); few steps leave little to share out; texels below 4
+// bytes, whose loads cost more than what is done with them, gain throughout.  A
+// volume filled with thin fog, us by 1 / 2 / 4 lanes in row order at 0.15, 0.3, 0.5,
+// 0.75 and 1.5 of the resident rays:
+//   FP32+FP32x3 256^3, 692 steps     411 266 219  447 425 350  679 544 504  728 695 715  1258 1162 1330
+//   FP16+FP16x3 256^3, 692 steps     275 189 149  285 263 244  368 363 361  450 476 499  796 815 916
+//   UNORM8+SNORM8x3 224^3, 692       292 212 166  333 308 285  437 424 403  524 563 576  922 972 1069
+//   FP16+SNORM8x3 96^3, 2000         854 753 625  1078 1115 1079  1484 1617 1618  1870 2191 2313  3451 3809 4320
+//   FP16+FP16x3 448^3, 346           280 232 211  267 319 280  331 331 325  342 375 382  479 511 570
+//   FP32+FP32x3 256^3, 100           107 110 94  111 134 142  176 169 191  189 216 269  321 341 504
+//   UNORM8+SNORM8x3 224^3, 100       73 58 49  85 81 79  108 111 108  136 146 150  232 248 276
+//   FP32 256^3, 692                  253 158 115  253 199 190  295 269 278  368 348 380  601 588 695
+//   UNORM8 224^3, 346                123 111 79  155 175 129  259 231 182  295 296 249  491 490 448
+// 448 random frames without skipping (the workloads' ranges of volumes, presets
+// and sizes) take 0.64 times as long by these lines as by one lane in plain row or
+// cost order, two of them more than 4.5 % longer and the worst 12 %; 1992 of
+// volumes filled with fog 0.84 times, 77 of them more than 4.5 % longer and the
+// worst 20 %.  With 4 lanes out to 3/8 and 2 out to 3/4 of the resident rays for
+// few steps and small texels, too, the fog's worst took 37 % longer.
 constexpr int march_lanes(long long rays, long long resident, bool skipping, double steps, int texel,
                           unsigned long long bytes)
 {
-    if (8 * rays <= (steps < 512.0 ? 3 : skipping ? 7 : 4) * resident) return 4;
-    const bool waits = steps >= 256.0 && (texel >= 16 || bytes >= 128ull << 20);
-    return 4 * rays <= (skipping ? 9 : waits ? 6 : 3) * resident ? 2 : 1;
+    if (skipping) return 8 * rays <= (steps < 512.0 ? 3 : 7) * resident ? 4 : 4 * rays <= 9 * resident ? 2 : 1;
+    if (texel < 4) return 4 * rays <= 3 * resident ? 4 : 1;
+    if (steps < 256.0) return 16 * rays <= 5 * resident ? 4 : 16 * rays <= 9 * resident ? 2 : 1;
+    if (8 * rays <= (steps < 512.0 ? 3 : 4) * resident) return 4;
+    return 4 * rays <= (texel >= 16 || bytes >= 128ull << 20 ? 6 : 3) * resident ? 2 : 1;
+}
+
+// Lanes per ray of a class of a batch, whose kernel takes transparent bricks
+// into account whether there are any or not (how many there are is not known
+// when it is launched) and fetches its tiles itself, the costliest first.
+// `steps`: of a mean ray.  500 random batches of one to four requests take 0.76
+// times as long by these lines as by one lane; over twelve volumes, mostly
+// empty, partly empty and filled, by steps: 50 1.01, 100 0.95, 346 0.84, 692 0.76,
+// 2000 0.63.  From the resident rays on, mostly empty volumes still gain by 2
+// lanes and filled ones lose (1.25 times, 692 steps, the time of one lane before
+// over that by 1 and by 2: 1.16, 1.24 and 1.00, 1.00; 2 times, 346 steps: 1.15, 1.11
+// and 0.99, 0.91).  One rule for all steps, 4 lanes out to 3/8 and 2 out to 9/4 of
+// the resident rays, took 7 % longer at 50 steps than one lane and cost 872 of
+// those 6432 batches more than 10 %; these lines cost 141.
+constexpr int batch_lanes(long long rays, long long resident, double steps)
+{
+    if (steps < 64.0) return 10 * rays <= resident ? 4 : 4 * rays <= resident ? 2 : 1;
+    if (steps < 256.0) return 4 * rays <= resident ? 4 : 4 * rays <= 3 * resident ? 2 : 1;
+    if (8 * rays <= 3 * resident) return 4;
+    return 4 * rays <= (steps < 512.0 ? 5 : steps < 1024.0 ? 7 : 9) * resident ? 2 : 1;
 }
 
 // Dispatch order of the blocks kept in rows: consecutive blocks of a class
@@ -253,15 +290,17 @@ constexpr int row_rotation(int ntx)
 }
 
 // Whether HVR_ORDER_AUTO orders a frame by cost: with more blocks than the
-// march keeps resident (8 of 256 threads per unit) blocks start late, and up
-// to 2.25 times the resident rays that sets the frame's end; beyond, and where
-// the rays' `steps` are few, the frame loses more to marching all dense blocks
-// at once than it gains (us in row order / ordered: 1024^2, 1 lane, 346 steps
-// 394 / 364, 446 / 422; 2 lanes, 692 steps 529 / 495; 2 lanes, 100 steps
-// 159 / 178; 1536^2 767 / 771; 2048^2, 100 steps 452 / 516).
-constexpr bool order_auto(long long blocks, long long rays, long long resident, int lanes, double steps)
+// march keeps resident (8 of 256 threads per unit) blocks start late, and
+// that sets the frame's end, unless the rays' `steps` are few.  Where bricks are
+// stepped over, a frame of more than 2.25 times the resident rays loses more to
+// marching all dense blocks at once than it gains (us in row order / ordered:
+// 1024^2, 1 lane, 346 steps 394 / 364, 446 / 422; 2 lanes, 692 steps 529 / 495; 2
+// lanes, 100 steps 159 / 178; 1536^2 767 / 771; 2048^2, 100 steps 452 / 516).
+// Where none are, it does not (three times the resident rays of a filled volume,
+// 692 steps: 4 % longer in row order, 2000 steps 5 to 9 %).
+constexpr bool order_auto(long long blocks, long long rays, long long resident, bool skipping, int lanes, double steps)
 {
-    return blocks * 256 > resident && 4 * rays <= 9 * resident && steps >= 256.0 * lanes;
+    return blocks * 256 > resident && steps >= 256.0 * lanes && (!skipping || 4 * rays <= 9 * resident);
 }
 
 // Correctly rounded quotients g / d of several g by one reciprocal (Markstein,

@@ -28,16 +28,19 @@ def test_rules_on_both_sides_of_their_lines(tmp_path):
     assert res.returncode == 0 and "split ok" in res.stdout, res.stdout + res.stderr
 
 
-# 1024^2 on 256 compute units, 8-byte texels of a small volume: one lane without
-# skipping and two with it; steps: the box's diagonal 2 sqrt(3) over the step
+# 2 and 2.32 times the rays of 256 compute units, 8-byte texels of a small volume:
+# one lane without skipping, two with it up to 2.25 times; steps: the box's
+# diagonal 2 sqrt(3) over the step
 @pytest.mark.gpu
-@pytest.mark.parametrize("skip,step,expect", [(False, 0.01, 1), (False, 0.02, 0), (True, 0.005, 1), (True, 0.01, 0)])
-def test_auto_orders_by_the_rendered_frames_lanes(hip, skip, step, expect):
+@pytest.mark.parametrize("size,skip,step,expect,counting", [(1024, False, 0.01, 1, 1), (1104, False, 0.01, 1, 1),
+                                                            (1104, False, 0.02, 0, 0), (1024, True, 0.005, 1, 1),
+                                                            (1024, True, 0.01, 0, 1), (1104, True, 0.005, 0, 0)])
+def test_auto_orders_by_the_rendered_frames_lanes(hip, size, skip, step, expect, counting):
     from pyvr_amd.config import RenderConfig
     from pyvr_amd.hip_renderer import VolumeRenderer, _lib
 
     sc = scenes.c0(size=48, image=64)
-    r = VolumeRenderer(1024, 1024, config=RenderConfig.custom(step_size=step, max_steps=1000), light=sc.light,
+    r = VolumeRenderer(size, size, config=RenderConfig.custom(step_size=step, max_steps=1000), light=sc.light,
                        scalar_format="f16", normal_format="f16x3")
     L, ctx = hip, r.gl_manager.ctx
 
@@ -54,7 +57,7 @@ def test_auto_orders_by_the_rendered_frames_lanes(hip, skip, step, expect):
         img = r.render()
         assert ordered() == expect
         r.sample_counts()
-        assert ordered() == (1 if step <= 0.01 else 0)      # the counting frame's: one lane
+        assert ordered() == counting      # the counting frame's: one lane
         _lib.check(L.hvr_set_dispatch_order(ctx, _lib.ORDER_OFF), "order")
         assert r.render() == img and ordered() == 0
         assert np.frombuffer(img, np.uint8).any()

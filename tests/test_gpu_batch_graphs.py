@@ -19,7 +19,7 @@ def disarm():
 
 
 # 4, 2 and 1 lanes per ray on 256 compute units
-SIZES = [(300, 300), (800, 800), (1200, 1200)]
+SIZES = [(300, 300), (700, 700), (1200, 1200)]
 
 
 @pytest.fixture(scope="module")
@@ -47,7 +47,7 @@ def test_sizes_across_the_lines_keep_their_graphs(hip, scene):
         b.reserve(4, 1 << 21, 4096)
         for size in SIZES:
             _run(b, scene, size)
-        sizes = SIZES + SIZES[::-1] + [(301, 280), (805, 790), (1100, 1201)]
+        sizes = SIZES + SIZES[::-1] + [(301, 280), (705, 690), (1100, 1201)]
         want = [_run_alone(scene, size, k) for k, size in enumerate(sizes)]
         _lib.inject_fault("hvr_batch_capture", code=-2)
         assert [_run(b, scene, size, k) for k, size in enumerate(sizes)] == want
