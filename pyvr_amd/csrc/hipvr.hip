@@ -718,7 +718,7 @@ static int upload_host(hvr_ctx *c, void *dst, const void *src, size_t bytes)
 struct FieldBuffer {
     hvr_ctx *c;
     char *p = nullptr;
-    bool own = false;
+    bool own = false, idle = false;   // idle: the stream has been waited for since the last use
     explicit FieldBuffer(hvr_ctx *ctx) : c(ctx) {}
     FieldBuffer(const FieldBuffer &) = delete;
     int get(size_t bytes)
@@ -736,7 +736,7 @@ struct FieldBuffer {
     {
         // also after a failure: nothing queued may still read the buffer
         // (or, in the caller's frame, the host memory copied from)
-        (void)hipStreamSynchronize(c->stream);
+        if (!idle) (void)hipStreamSynchronize(c->stream);
         if (own) (void)hipFree(p);
     }
 };
@@ -1087,6 +1087,7 @@ static int upload_part(hvr_volume *v, const float *data, int part)
             // the staging buffer is reused by the next group
             HIPCHK(hipStreamSynchronize(c->stream));
         }
+    f.idle = true;
     return HVR_OK;
 }
 
