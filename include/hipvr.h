@@ -157,9 +157,10 @@ int hvr_volume_upload_normals(hvr_volume *vol, const float *data);
  * 109-122, and are uploaded by create_normal_texture, manager.py:110-135).
  *
  * hvr_volume_upload_scalar_normals: upload the float32 scalar field (numpy
- * C order) once and compute the normals on the device, bit for bit as
+ * C order) once and compute the normals on the device, as
  * compute_normal_volume computes them from that float32 array (np.gradient,
- * norm summed left to right, + 1e-8, division); every axis needs >= 2
+ * norm summed left to right, + 1e-8, division; in float32, correctly rounded but
+ * for the square root, which is within an ulp); every axis needs >= 2
  * voxels.  The volume must hold both fields.
  *
  * hvr_volume_generate_blobs: fill the scalar field (and the normals, when

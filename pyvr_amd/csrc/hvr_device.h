@@ -1485,10 +1485,14 @@ constexpr int build_bricks(int lb) { return lb == 4 ? 1 : 4; }   // bricks along
 // stored, the apron included, so that it covers every footprint the brick
 // serves; a NaN widens it to everything.  UNORM8 ranges are in decoded units
 // (raw / 255).
-// Memory bounds it (FP16+FP16x3 320^3 in 16^3 bricks: 391 MB out and, each of
-// the 8 L2s fetching its bricks' surroundings, 329 MB in, at 4.5 TB/s).  ONCE
+// What bounds it, FP16+FP16x3 from a field: for 320^3 in 16^3 bricks (163 us)
+// VALU issue, 72 % busy, and memory (392 MB out; 658 MB in, since each of the 8
+// L2s fetches its bricks' surroundings, from the last cache for the most part).
+// 512^3 in 8^3 bricks takes 1020 us, 1.5 times as long per voxel: 1.73 GB out
+// and 1.85 GB in at 3.5 TB/s where 1.60 and 0.54 GB are what it cannot do
+// without, VALU issue 51 % busy, a wave 17 us for the 12 rounds of its brick.  ONCE
 // writes the texels past the caches, which leaves the field there; it is for
-// field and texels together above the 256 MB of the last cache (that volume 217
+// field and texels together above the 256 MB of the last cache (the 320^3 217
 // -> 160 us, FP32+FP32x3 256^3 154 -> 114, UNORM8+SNORM8x3 384^3 316 -> 224).
 // Below, it gains nothing (FP16+FP16x3 192^3 54 / 54) and a march after it takes
 // 5-8 us longer.  Writing whole texels in order, the range formed on the way,
@@ -1670,7 +1674,9 @@ k_blob_factors(double *__restrict__ fac, int s0, int s1, int s2, const BlobSpec 
 // A wave takes 64 voxels along the last axis and kBlobRows rows of the middle
 // one: the last axis' factor is a load per blob, the others' are scalar.
 // With every factor computed at every voxel (three exponentials in double per
-// blob) the kernel took 1058 us for 8 blobs at 320^3; these two take 106.
+// blob) the kernel took 1058 us for 8 blobs at 320^3; these two take 110-120.
+// VALU issue bounds it (88 % busy for 8 blobs at 512^3, 390 us: the noise's hash,
+// an FP64 product and sum per blob); the field is written at 1.4 TB/s.
 static constexpr int kBlobRows = 8;
 static __global__ void __launch_bounds__(256)
 k_blob_field(float *__restrict__ out, int s0, int s1, int s2, const BlobSpec *__restrict__ spec,

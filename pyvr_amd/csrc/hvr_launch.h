@@ -33,7 +33,9 @@ enum BatchVariant : int {
     BV_WAVES8 = 2,    // 8 waves per block
     BV_NOGATE = 3,    // normals for every shaded sample
     BV_NOSKIP = 4,    // no transparent-brick skipping
-    BV_LANES2 = 5,    // 2 or 4 lanes per ray, in BV_DEFAULT's place (batch_lanes)
+    // 2 or 4 lanes per ray, in BV_DEFAULT's place for classes of few rays with
+    // 8x8 tiles (batch_lanes; the other variants and 16x4 tiles have one lane)
+    BV_LANES2 = 5,
     BV_LANES4 = 6,
     BV_COUNT = 7
 };
@@ -56,15 +58,14 @@ typedef int (*BatchLaunchFn)(const char *blk, int cls, uint32_t *ctr, int lut_ca
     X(TF_C_F16_F16)
 
 // Per format F:
-//   launch_march_F: k_march for normal mode nm (NM_ZERO / NM_ALIAS /
-//     NM_SAME), brick log2 lb (3 or 4), counting, skipping, buffer loads;
-//     returns false when this format has no such instance (NM_SAME without
-//     normals);
+//   launch_march_F: k_march for normal mode nm (NM_ZERO / NM_ALIAS, and
+//     NM_SAME where the format holds normals), brick log2 lb (3 or 4),
+//     counting, skipping, buffer loads;
 //   batch_fn_F: the batched launcher for those choices, tile shape ts and
 //     kernel variant (BV_*), or nullptr when there is none (counting runs
 //     use BV_DEFAULT only).
 #define HVR_DECLARE_FORMAT(F)                                                                   \
-    bool launch_march_##F(const MarchArgs &a, int nm, int lb, bool count, bool skip, bool buf); \
+    void launch_march_##F(const MarchArgs &a, int nm, int lb, bool count, bool skip, bool buf); \
     BatchLaunchFn batch_fn_##F(int nm, int lb, bool count, int ts, bool buf, int variant);
 HVR_FAST_FORMATS(HVR_DECLARE_FORMAT)
 #undef HVR_DECLARE_FORMAT

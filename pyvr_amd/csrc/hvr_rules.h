@@ -14,6 +14,8 @@ namespace hvr {
 // extended texture holds s + 2 texels (the edge copies), X in [0, s + 1].
 constexpr uint32_t bricks_along(int s, int lb) { return ((uint32_t)s >> lb) + 1u; }
 
+// The layout seen from the voxels, for checking slot_voxel (which the build
+// kernel fills every slot by) against it.
 // Slots along one axis that hold texel coordinate c of a texture of size s
 // stored in nb bricks: (brick, local) pairs; returns how many (1..4).  In
 // extended coordinates the texel sits at X = c + 1, and also at X = 0 when

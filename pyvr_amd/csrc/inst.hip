@@ -105,23 +105,13 @@ BatchLaunchFn batch_nm(int lb, bool count, int ts, bool buf, int v)
 
 }  // namespace
 
-bool HVR_CAT(launch_march_, HVR_INST_FMT)(const MarchArgs &a, int nm, int lb, bool count, bool skip, bool buf)
+void HVR_CAT(launch_march_, HVR_INST_FMT)(const MarchArgs &a, int nm, int lb, bool count, bool skip, bool buf)
 {
-    if (nm == NM_ZERO) {
-        march_nm<NM_ZERO>(a, lb, count, skip, buf);
-        return true;
-    }
-    if (nm == NM_ALIAS) {
-        march_nm<NM_ALIAS>(a, lb, count, skip, buf);
-        return true;
-    }
     if constexpr (fmt_has_normal(F)) {
-        if (nm == NM_SAME) {
-            march_nm<NM_SAME>(a, lb, count, skip, buf);
-            return true;
-        }
+        if (nm == NM_SAME) return march_nm<NM_SAME>(a, lb, count, skip, buf);
     }
-    return false;
+    if (nm == NM_ZERO) march_nm<NM_ZERO>(a, lb, count, skip, buf);
+    else march_nm<NM_ALIAS>(a, lb, count, skip, buf);
 }
 
 // Batched launchers: scalar-only formats read normals as (rho, 0, 0) or none,

@@ -8,6 +8,8 @@ the same images; only the time differs.
 Each candidate renders the requests (all, or an evenly spaced sample of
 ``max_requests``) in one batch; the figure of merit is the median device time
 of ``runs`` launches after a warm-up launch (which also captures the graph).
+The default variant with 8x8 tiles marches batches of few rays by several lanes
+per ray, the others by one: a sample of few or small requests favours it.
 Results can be kept in a JSON cache keyed by the workload's signature
 (formats, volume shapes, image sizes, request count), so a server tunes once.
 """

@@ -107,7 +107,8 @@ class DeviceBlobVolume:
 class ResidentVolume:
     """A ``Volume`` (or ``DeviceBlobVolume``) on the device, shared by
     requests.  ``device_normals``: compute the normals of a volume without
-    normals on the device (the bytes compute_normal_volume would give)."""
+    normals on the device (compute_normal_volume's, within an ulp before they
+    are stored)."""
 
     def __init__(self, L, ctx, volume, scalar_format: str, normal_format: str, device_normals: bool = False):
         generated = isinstance(volume, DeviceBlobVolume)
@@ -147,7 +148,9 @@ class ResidentVolume:
 
 
 # Kernel variants of the batched march (hvr_batch_set_kernel): waves per
-# block, transparent-brick skipping, normals gated on non-zero alpha.
+# block, transparent-brick skipping, normals gated on non-zero alpha.  With 8x8
+# tiles, "default" marches classes of few rays by 2 or 4 lanes per ray; the others
+# have one.
 KERNEL_VARIANTS = {"default": (4, True, True), "waves2": (2, True, True), "waves8": (8, True, True),
                    "nogate": (4, True, False), "noskip": (4, False, True)}
 

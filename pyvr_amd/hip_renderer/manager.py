@@ -111,8 +111,9 @@ class _DeviceVolume:
         self.normals_loaded = True
 
     def upload_scalar_normals(self, data: np.ndarray):
-        """Scalar field, and its normals computed on the device exactly as
-        compute_normal_volume computes them from the float32 array."""
+        """Scalar field, and its normals computed on the device as
+        compute_normal_volume computes them from the float32 array (the square
+        root within an ulp)."""
         a = np.ascontiguousarray(data, dtype=np.float32)
         check(self.L.hvr_volume_upload_scalar_normals(self.handle,
                                                       a.ctypes.data_as(ctypes.POINTER(ctypes.c_float))),
