@@ -368,7 +368,9 @@ int hvr_batch_set_tile_shape(hvr_batch *batch, int shape);
  * default): waves per block and whether transparent bricks are stepped over
  * (skip) and normals interpolated only for samples of non-zero alpha (gate).
  * Supported: (4, 1, 1) -- the default --, (2, 1, 1), (8, 1, 1), (4, 1, 0),
- * (4, 0, 1).  Every variant gives the same image; the autotuner times them. */
+ * (4, 0, 1).  With 8 x 8 tiles the default marches requests of few rays by 2 or
+ * 4 lanes per ray; the others have one.  Every variant gives the same image; the
+ * autotuner times them. */
 int hvr_batch_set_kernel(hvr_batch *batch, int waves_per_block, int skip, int gate);
 /* Where the batch's march writes its images (no counterpart in the
  * reference): HVR_READBACK_DIRECT (the default) straight into the pinned
