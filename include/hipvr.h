@@ -104,7 +104,8 @@ int hvr_abi_version(void);
  * hvr_batch_run_async, hvr_batch_wait, hvr_batch_query.  Inside the uploads,
  * "hvr_upload_ring" fails a copy that takes the library's own pinned memory;
  * inside hvr_batch_run_async, "hvr_batch_capture" fails a launch of a shape
- * that has no captured graph. */
+ * that has no captured graph and "hvr_batch_grow" the growth of a pool, whose
+ * old memory is gone by then. */
 int hvr_debug_inject_fault(const char *function, int code, int after);
 
 /* Message of the last failed call on this thread ("" if none). */

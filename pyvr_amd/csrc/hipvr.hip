@@ -1647,9 +1647,9 @@ static BatchLaunchFn batch_fn(int fmt, int nm, int lb, bool count, int ts, bool 
     }
 }
 
-// Grow a device (and optionally pinned host) buffer to at least `need`
-// bytes.  Returns true when it was reallocated.
-static int grow(int device, void **d, void **h, size_t *cap, size_t need, bool *moved)
+// Grow a device (and optionally pinned host) buffer to at least `need` bytes.
+// After a failure its capacity is 0.
+static int grow(int device, void **d, void **h, size_t *cap, size_t need)
 {
     if (need <= *cap) return HVR_OK;
     size_t n = *cap ? *cap : 4096;
@@ -1661,10 +1661,10 @@ static int grow(int device, void **d, void **h, size_t *cap, size_t need, bool *
         *h = nullptr;
     }
     *cap = 0;
+    HVR_FAULT_POINT("hvr_batch_grow");
     HIPCHK(dev_malloc(device, d, n));
     if (h) HIPCHK(hipHostMalloc(h, n, hipHostMallocDefault));
     *cap = n;
-    *moved = true;
     return HVR_OK;
 }
 
@@ -1676,6 +1676,18 @@ static void batch_drop_graphs(hvr_batch *b, size_t n = 0)
         (void)hipGraphDestroy(b->graphs[k].graph);
     }
     if (n < b->graphs.size()) b->graphs.resize(n);
+}
+
+// The batch's pools of at least these bytes (no launch in flight).  What holds
+// their addresses goes before any of them moves, since a later one may fail.
+static int batch_grow(hvr_batch *b, size_t stage, size_t out, size_t flags)
+{
+    const int device = b->ctx->device;
+    if (stage > b->stage_cap) batch_drop_graphs(b);
+    if (out > b->out_cap) b->h_out_dev_of = nullptr;   // a new pinned pool may reuse the old address
+    if (const int rc = grow(device, (void **)&b->d_stage, (void **)&b->h_stage, &b->stage_cap, stage)) return rc;
+    if (const int rc = grow(device, (void **)&b->d_out, (void **)&b->h_out, &b->out_cap, out)) return rc;
+    return grow(device, (void **)&b->d_flags, nullptr, &b->flags_cap, flags);
 }
 
 extern "C" {
@@ -1822,13 +1834,7 @@ int hvr_batch_reserve(hvr_batch *b, int max_requests, unsigned long long max_pix
     const size_t stage = align_up(nz_off + nreq * (kLutLdsMax + 1) * sizeof(int), 256);
     const size_t pixels = (size_t)max_pixels + 64 * nreq;   // each request padded to 64 pixels
     const size_t flags = nreq * align_up((size_t)max_bricks, 256);
-    bool moved = false, moved_out = false;
-    if (const int rc = grow(b->ctx->device, (void **)&b->d_stage, (void **)&b->h_stage, &b->stage_cap, stage, &moved)) return rc;
-    if (const int rc = grow(b->ctx->device, (void **)&b->d_out, (void **)&b->h_out, &b->out_cap, pixels * 4, &moved_out)) return rc;
-    if (const int rc = grow(b->ctx->device, (void **)&b->d_flags, nullptr, &b->flags_cap, flags, &moved_out)) return rc;
-    if (moved_out) b->h_out_dev_of = nullptr;   // a new pinned pool may reuse the old address
-    if (moved) batch_drop_graphs(b);
-    return HVR_OK;
+    return batch_grow(b, stage, pixels * 4, flags);
 }
 
 int hvr_batch_run_async(hvr_batch *b, int count)
@@ -1909,18 +1915,13 @@ int hvr_batch_run_async(hvr_batch *b, int count)
     }
     const size_t nz_off = align_up(lut_off + lut_bytes, 256);
     const size_t stage_need = align_up(nz_off + nz_bytes, 256);
-    bool moved = false;
-    if (const int rc = grow(b->ctx->device, (void **)&b->d_stage, (void **)&b->h_stage, &b->stage_cap, stage_need, &moved)) return rc;
-    bool moved_out = false;
-    if (const int rc = grow(b->ctx->device, (void **)&b->d_out, (void **)&b->h_out, &b->out_cap, pixels * 4, &moved_out)) return rc;
-    if (const int rc = grow(b->ctx->device, (void **)&b->d_flags, nullptr, &b->flags_cap, flag_bytes, &moved_out)) return rc;
+    if (const int rc = batch_grow(b, stage_need, pixels * 4, flag_bytes)) return rc;
     if (count) {
         size_t cb = b->counts_cap * 4;
-        if (const int rc = grow(b->ctx->device, (void **)&b->d_counts, (void **)&b->h_counts, &cb, pixels * 4, &moved_out)) return rc;
+        const int rc = grow(b->ctx->device, (void **)&b->d_counts, (void **)&b->h_counts, &cb, pixels * 4);
         b->counts_cap = cb / 4;
+        if (rc) return rc;
     }
-    if (moved_out) b->h_out_dev_of = nullptr;   // a new pinned pool may reuse the old address
-    if (moved) batch_drop_graphs(b);
     // direct: the march stores each pixel straight into the pinned pool
     // through its device address (posted writes over the host link while
     // the batch runs, no copy after it)
